@@ -10,8 +10,9 @@
 // fp16 path (d = 64 or 128): a workgroup owns 128 queries, 32 per wave (two 16-query
 // column blocks, so every K and V^T fragment read from LDS feeds two MFMAs).  Key blocks
 // of 64 are staged in LDS (K as [key][dim], V^T as [dim][key]) through a two-stage ring
-// whose next block is loaded into registers while the current one is used (for d = 64
-// and S % 8 == 0, flash_f16_dma64 streams the blocks by DMA instead, see there).  Each wave
+// whose next block is loaded into registers while the current one is used (flash_f16_dma,
+// which the fused op takes unless a weight or bias is misaligned, streams the blocks by
+// DMA instead, see there).  Each wave
 // computes S^T = K·Q^T with v_mfma_f32_16x16x32_f16, so a lane holds 16 scores of ONE
 // query per column block: the row max and row sum are lane-local plus a 4-lane exchange.
 // The probabilities are converted to fp16 in registers and fed back as the B operand of
@@ -225,18 +226,28 @@ void flash_f16(cf_flash_args_t a) {
     }
 }
 
-// ---- d = 64, S % 8 == 0: the same computation with K and V^T blocks streamed by DMA
-// (global_load_lds_dwordx4) into a kFlashStages-deep LDS ring instead of through
-// registers, so kFlashStages - 1 key blocks are in flight while one is used and no
-// wave waits on a block's loads before storing them.  K rows (128 B) and V^T rows (64
+// ---- The same computation with K and V blocks streamed by DMA (global_load_lds_dwordx4)
+// into an LDS ring of NS stages instead of through registers, so NS - 1 key blocks are in
+// flight while one is used and no wave waits on a block's loads before storing them.
+// Inputs are the row-concatenated projection (RC, any S, d = 64 or 128) or head-major
+// q / k / v^T (d = 64, S % 8 == 0).
+// d = 128: a stage is 32 KB, so two stages (64 KB) keep two workgroups per CU, as the
+// register-staged kernel had; three stages would leave one.  The block in flight has a
+// whole block's arithmetic (about 0.8 us with two workgroups per CU) to land.  What bounds
+// it is LDS reads and MFMAs about equally (a 16-query wave reads 32 KB per key block, ~240
+// clk of the CU's LDS against 128 clk of its MFMAs; 32-query waves halve the former).  One
+// sequence of 2048, 32 / 8 heads, causal: 101 us register-staged, 52 us here (660 TFLOP/s
+// of the causal work; not causal 77 us, 890).  3 sequences of 197, 12 heads of 64, causal:
+// 16.5 us register-staged (its V^T rows are misaligned at odd S), 5.5 us here.
+// At d = 64: K rows (128 B) and V^T rows (64
 // keys, 128 B) are XOR-swizzled in 16-byte chunks so the K fragment reads (16 rows, one
 // chunk: chunk ^ (row / 2) % 8) and the V^T fragment reads (16 rows, 8 bytes: chunk ^
 // (row / 2 ^ row / 16) % 8) are bank-conflict free.  The V^T term in row / 16 makes the
 // reads of row blocks u and u+1 differ by more than a constant, so the compiler keeps
 // them as separate ds_read_b64 instead of pairing them into ds_read2st64_b64, which
 // measured four times the LDS cycles (SQ_LDS_BANK_CONFLICT) on gfx950.  Rows and chunks
-// past the sequence end are clamped to the last valid ones (S % 8 == 0 keeps every 8-key
-// chunk whole) and get p = 0.  The row max is reduced with the gfx950 row swaps, and the
+// past the sequence end are clamped to the last valid ones (head-major: S % 8 == 0 keeps
+// every 8-key chunk whole) and get p = 0.  The row max is reduced with the gfx950 row swaps, and the
 // running max only moves when a block exceeds it by more than kLazy (log2 units), so the
 // accumulators are rarely rescaled.
 // The kernel is bound by its VALU work per score (the exponential and its neighbours),
@@ -245,31 +256,36 @@ void flash_f16(cf_flash_args_t a) {
 // offsets fixed for the whole loop, and the row sum of p comes out of the matrix core:
 // one more MFMA per 32 keys with an all-ones A operand gives every lane the full sum
 // over the block's keys for its query, from the same fp16 p that weights V.
-constexpr int kFlashStages = 3;
 constexpr float kLazy = 8.0f;
 
-__device__ __forceinline__ int fswz(int row) { return (row >> 1) & 7; }
+// K (and Q) rows, read as 16 rows x one chunk per fragment.  d = 64: two 128-byte rows
+// per 256-byte bank window; d = 128: each row is a window of its own.
+template <int D>
+__device__ __forceinline__ int fswz(int row) { return D == 64 ? (row >> 1) & 7 : row & 15; }
 __device__ __forceinline__ int vswz(int row) { return ((row >> 1) ^ (row >> 4)) & 7; }
 
 // V rows [key][dim] (the row-concatenated input), read transposed by ds_read_b64_tr_b16:
 // rows of one 32-lane half of a read (keys kb .. kb+7) land in distinct banks.
-__device__ __forceinline__ int trswz(int row) { return 2 * ((row >> 1) & 3); }
+template <int D>
+__device__ __forceinline__ int trswz(int row) { return D == 64 ? 2 * ((row >> 1) & 3) : 2 * (row & 7); }
 
 // RC: Q, K and V come from the row-concatenated (B*S, qkv_ld) matrix (K and V rows as
 // they are; V read transposed from LDS), else from q / k / vt laid out head-major.
 // Waves per SIMD the build must allow: three 16-query workgroups per CU; the 32-query
 // build (taken with at least two workgroups per CU) at three would spill registers.
-template <int NJ, bool RC = false>
-__global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2)
-void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div_hq, FastDiv div_g) {
-    constexpr int D = 64;
+template <int D, int NJ, bool RC = false>
+__global__ __launch_bounds__(kThreads, D == 64 && NJ == 1 ? 3 : 2)
+void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot, FastDiv div_hq, FastDiv div_g) {
     constexpr int QW = 16 * NJ;                   // queries per wave
     constexpr int QB = 4 * QW;                    // queries per workgroup
     constexpr int KT = D / 32;                    // 32-dim steps of S^T
     constexpr int UT = D / 16;                    // 16-dim tiles of O^T
-    constexpr int TILE = kKB * D;                 // halves per block per tensor (8 KB)
-    constexpr int NS = kFlashStages;
-    static_assert(NS == 3, "the prologue issues two blocks");
+    constexpr int TILE = kKB * D;                 // halves per block per tensor (D = 64: 8 KB)
+    constexpr int NS = D == 64 ? 3 : 2;           // ring stages: 48 or 64 KB
+    constexpr int CPR = D / 8;                    // 16-byte chunks per K (and, RC, V) row
+    constexpr int RPI = 64 / CPR;                 // rows per 1 KB DMA instruction
+    constexpr int NI = 16 / RPI;                  // DMA instructions per tensor, wave and block
+    static_assert(D == 64 || (D == 128 && RC), "head-major V^T rows only at d = 64");
     __shared__ __attribute__((aligned(16))) _Float16 ring[NS * 2 * TILE];
 
     // Causal (pairs == 0, the default): one query block per workgroup, every head's
@@ -288,7 +304,14 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
     const int rq = fastdiv(rest, div_slot), rr = rest - rq * (a.causal && !pairs ? ngrp : nslot);
     const int qi = a.causal && !pairs ? rq : rr;
     const int grp = a.causal && !pairs ? rr : rq;
-    const int hb = grp * 8 + r8;
+    // Position i = 8 grp + r8 of the head-batch order (i % 8 is its XCD).  With kv_order
+    // (B * H_kv a multiple of 8) the G query heads of one KV head are 8 positions apart,
+    // so they share an XCD and its L2 holds each K / V once; else plain (b, h) order.
+    int hb = grp * 8 + r8;
+    if (kv_order) {
+        const int kq = fastdiv(grp, div_g);
+        hb = (kq * 8 + r8) * (a.H_q / a.H_kv) + (grp - kq * (a.H_q / a.H_kv));
+    }
     if (hb >= HB) return;                          // padding of the last group of 8
     const int b = fastdiv(hb, div_hq), h = hb - b * a.H_q;
     const int S = a.S;
@@ -314,19 +337,19 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
 #pragma unroll
     for (int j = 0; j < NJ; j++) query[j] = qw + 16 * j + lr;
 
-    // DMA: each wave fills K rows 16w .. 16w+15 and V^T rows 16w .. 16w+15 of a stage,
-    // 8 rows per instruction; lane L writes physical chunk L % 8 of row 8u + L / 8.  A
-    // full block is a uniform base (its first key) plus these per-lane byte offsets
+    // DMA: each wave fills K rows 16w .. 16w+15 and V (or V^T) rows 16w .. 16w+15 of a
+    // stage, RPI rows per instruction; lane L writes physical chunk L % CPR of row
+    // RPI u + L / CPR.  A full block is a uniform base (its first key) plus these per-lane byte offsets
     // (V^T rows are S keys apart: the launcher keeps 64 * S * 2 bytes below 2^32).
     const uint32_t ring_base = lds_offset(ring);
-    const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(ring_base + (uint32_t)(16 * wave) * 128u);
-    const int drow0 = 16 * wave + (lane >> 3), dch = lane & 7;
-    uint32_t koff[2], voff[2];
+    const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(ring_base + (uint32_t)(16 * wave) * (uint32_t)(2 * D));
+    const int drow0 = 16 * wave + lane / CPR, dch = lane % CPR;
+    uint32_t koff[NI], voff[NI];
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const int row = drow0 + 8 * u;
-        koff[u] = ((uint32_t)row * (uint32_t)ld + 8u * (uint32_t)(dch ^ fswz(row))) * 2u;
-        voff[u] = RC ? ((uint32_t)row * (uint32_t)ld + 8u * (uint32_t)(dch ^ trswz(row))) * 2u
+    for (int u = 0; u < NI; u++) {
+        const int row = drow0 + RPI * u;
+        koff[u] = ((uint32_t)row * (uint32_t)ld + 8u * (uint32_t)(dch ^ fswz<D>(row))) * 2u;
+        voff[u] = RC ? ((uint32_t)row * (uint32_t)ld + 8u * (uint32_t)(dch ^ trswz<D>(row))) * 2u
                      : ((uint32_t)row * (uint32_t)S + 8u * (uint32_t)(dch ^ vswz(row))) * 2u;
     }
     auto issue = [&](int blk, auto stage_c) {
@@ -338,22 +361,22 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
             const _Float16* kblk = kp + (size_t)k0 * ld;
             const _Float16* vblk = RC ? vp + (size_t)k0 * ld : vp + k0;
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                lds_dma16_s(koff[u], kblk, kb + (uint32_t)(8 * u) * 128u);
-                lds_dma16_s(voff[u], vblk, vb + (uint32_t)(8 * u) * 128u);
+            for (int u = 0; u < NI; u++) {
+                lds_dma16_s(koff[u], kblk, kb + (uint32_t)u * 1024u);
+                lds_dma16_s(voff[u], vblk, vb + (uint32_t)u * 1024u);
             }
         } else {
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const int row = drow0 + 8 * u;
-                const int kc = dch ^ fswz(row);
-                lds_dma16(kp + (size_t)min(k0 + row, S - 1) * ld + 8 * kc, kb + (uint32_t)(8 * u) * 128u);
+            for (int u = 0; u < NI; u++) {
+                const int row = drow0 + RPI * u;
+                const int kc = dch ^ fswz<D>(row);
+                lds_dma16(kp + (size_t)min(k0 + row, S - 1) * ld + 8 * kc, kb + (uint32_t)u * 1024u);
                 if constexpr (RC) {
-                    lds_dma16(vp + (size_t)min(k0 + row, S - 1) * ld + 8 * (dch ^ trswz(row)),
-                              vb + (uint32_t)(8 * u) * 128u);
+                    lds_dma16(vp + (size_t)min(k0 + row, S - 1) * ld + 8 * (dch ^ trswz<D>(row)),
+                              vb + (uint32_t)u * 1024u);
                 } else {
                     const int vcol = min(k0 + 8 * (dch ^ vswz(row)), S - 8);
-                    lds_dma16(vp + (size_t)row * S + vcol, vb + (uint32_t)(8 * u) * 128u);
+                    lds_dma16(vp + (size_t)row * S + vcol, vb + (uint32_t)u * 1024u);
                 }
             }
         }
@@ -365,7 +388,7 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
 #pragma unroll
         for (int kt = 0; kt < KT; kt++) {
             const int row = 16 * t + lr;
-            k_rd[t][kt] = row * D + 8 * ((4 * kt + lq) ^ fswz(row));
+            k_rd[t][kt] = row * D + 8 * ((4 * kt + lq) ^ fswz<D>(row));
         }
     int v_rd[UT][2][2];
 #pragma unroll
@@ -379,7 +402,7 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
                     // 16u + 4(lr%4) .. +3, and receives dim 16u + lr of those 4 keys.
                     const int row = 32 * s2 + 16 * hh + 4 * lq + (lr >> 2);
                     const int col = 16 * u + 4 * (lr & 3);
-                    v_rd[u][s2][hh] = TILE + row * D + 8 * ((col >> 3) ^ trswz(row)) + (col & 7);
+                    v_rd[u][s2][hh] = TILE + row * D + 8 * ((col >> 3) ^ trswz<D>(row)) + (col & 7);
                 } else {
                     const int row = 16 * u + lr;
                     const int ch = 4 * s2 + 2 * hh + (lq >> 1);      // keys 32s + 16hh + 4lq
@@ -406,24 +429,26 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
 
     const int k_end = a.causal ? min(S, q0 + QB) : S;
     const int nblk = (k_end + kKB - 1) / kKB;
-    // The workgroup's Q rows (QB x 128 B, swizzled like K) go by DMA into ring stage
-    // NS-1, which the first blocks leave free, ahead of blocks 0 and 1: the Q and K/V
-    // latencies overlap.  Wave w loads rows 8u .. 8u+7 for u = QB/32 * w + v.
-    constexpr int QI = QB / 32;                   // Q DMA instructions per wave
+    // The workgroup's Q rows (QB x 2 D bytes, swizzled like K) go by DMA into ring stage
+    // NS-1, which the first NS-1 blocks leave free, ahead of those blocks: the Q and K/V
+    // latencies overlap.  Wave w loads rows RPI u .. +RPI-1 for u = QI * w + v.
+    static_assert(QB * D <= 2 * TILE, "Q fits a ring stage");
+    constexpr int QI = QB / RPI / 4;              // Q DMA instructions per wave
     {
         const uint32_t qb_lds = ring_base + (uint32_t)((NS - 1) * 2 * TILE) * 2u;
 #pragma unroll
         for (int v = 0; v < QI; v++) {
-            const int u = QI * wave + v, row = 8 * u + (lane >> 3);
-            lds_dma16(qp + (size_t)min(q0 + row, S - 1) * ld + 8 * (dch ^ fswz(row)),
+            const int u = QI * wave + v, row = RPI * u + lane / CPR;
+            lds_dma16(qp + (size_t)min(q0 + row, S - 1) * ld + 8 * (dch ^ fswz<D>(row)),
                       __builtin_amdgcn_readfirstlane(qb_lds + (uint32_t)u * 1024u));
         }
     }
     if (0 < nblk) issue(0, std::integral_constant<int, 0>{});
-    if (1 < nblk) issue(1, std::integral_constant<int, 1>{});
-    // Q landed when at most the blocks' loads (4 per block) are outstanding.
-    if (nblk >= 2) wait_vm<8>();
-    else wait_vm<4>();
+    if constexpr (NS > 2)
+        if (1 < nblk) issue(1, std::integral_constant<int, 1>{});
+    // Q landed when at most the blocks' loads (2 NI per block) are outstanding.
+    if (NS > 2 && nblk >= 2) wait_vm<4 * NI>();
+    else wait_vm<2 * NI>();
     ring_barrier();
     // B operand Q^T: lane (lr, lq) holds Q[query][32kt + 8lq .. +7].
     h8_t qf[NJ][KT];
@@ -433,14 +458,14 @@ void flash_f16_dma64(cf_flash_args_t a, int pairs, FastDiv div_slot, FastDiv div
         for (int j = 0; j < NJ; j++) {
             const int row = QW * wave + 16 * j + lr;
 #pragma unroll
-            for (int kt = 0; kt < KT; kt++) qf[j][kt] = *(const h8_t*)(qs + row * D + 8 * ((4 * kt + lq) ^ fswz(row)));
+            for (int kt = 0; kt < KT; kt++) qf[j][kt] = *(const h8_t*)(qs + row * D + 8 * ((4 * kt + lq) ^ fswz<D>(row)));
         }
     }
     wait_lds_reads();                              // stage NS-1 is refilled after the next barrier
     auto step = [&](int bi, auto stage_c) {
         constexpr int stage = decltype(stage_c)::value;
-        // Blocks issued after this one that may still be in flight (4 loads each).
-        wait_ahead<4, NS - 2>(nblk - 1 - bi);
+        // Blocks issued after this one that may still be in flight (2 NI loads each).
+        wait_ahead<2 * NI, NS - 2>(nblk - 1 - bi);
         ring_barrier();                            // every wave's part of block bi landed;
                                                    // block bi-1's stage is free again
         if (bi + NS - 1 < nblk) issue(bi + NS - 1, std::integral_constant<int, (stage + NS - 1) % NS>{});
@@ -824,9 +849,9 @@ extern "C" void cf_flash_set_mode(int32_t mode) { g_flash_mode = mode >= 0 && mo
 extern "C" void cf_flash_set_causal_pairs(int32_t on) { g_flash_pairs = on > 0 ? 1 : 0; }
 
 extern "C" int32_t cf_flash_rowcat_ok(const cf_flash_args_t* a) {
-    return a->elem == CF_ELEM_F16 && a->d == 64 && a->S > 0 && a->S % 8 == 0 && a->S <= (1 << 24) &&
+    return a->elem == CF_ELEM_F16 && (a->d == 64 || a->d == 128) && a->S > 0 && a->S <= (1 << 24) &&
            a->H_kv > 0 && a->H_q % a->H_kv == 0 && a->scale > 0.0f &&
-           a->qkv_ld == (a->H_q + 2 * a->H_kv) * 64 && ((uintptr_t)a->q | (uintptr_t)a->o) % 16 == 0;
+           a->qkv_ld == (a->H_q + 2 * a->H_kv) * a->d && ((uintptr_t)a->q | (uintptr_t)a->o) % 16 == 0;
 }
 
 extern "C" int cf_launch_flash_attn(const cf_flash_args_t* a, void* stream) {
@@ -841,7 +866,7 @@ extern "C" int cf_launch_flash_attn(const cf_flash_args_t* a, void* stream) {
         if (groups * nqb * 8 > 0x7fffffffLL) return (int)hipErrorInvalidValue;
         dim3 grid((unsigned)(groups * nqb * 8));
         // The DMA kernel addresses V^T rows with 32-bit byte offsets: 64 * S * 2 < 2^32.
-        if (a->d == 64 && a->S % 8 == 0 && a->S <= (1 << 24) && (g_flash_mode != 0 || a->qkv_ld)) {
+        if (a->qkv_ld || (a->d == 64 && a->S % 8 == 0 && a->S <= (1 << 24) && g_flash_mode != 0)) {
             // 16 queries per wave (64 per workgroup) doubles the workgroups, and with
             // them the waves per SIMD that hide each block's latency chain; 32 per wave
             // halves the LDS traffic per query (every wave reads the whole K/V^T block),
@@ -864,11 +889,20 @@ extern "C" int cf_launch_flash_attn(const cf_flash_args_t* a, void* stream) {
             // config 5's attention as runtime divisions in every workgroup's prologue).
             const FastDiv dslot = fastdiv_make((int)(a->causal && !pairs ? groups : nslot));
             const FastDiv dhq = fastdiv_make(a->H_q), dg = fastdiv_make(a->H_q / a->H_kv);
-            if (a->qkv_ld) {
-                if (nj == 1) hipLaunchKernelGGL((flash_f16_dma64<1, true>), grid2, dim3(kThreads), 0, s, *a, pairs, dslot, dhq, dg);
-                else hipLaunchKernelGGL((flash_f16_dma64<2, true>), grid2, dim3(kThreads), 0, s, *a, pairs, dslot, dhq, dg);
-            } else if (nj == 1) hipLaunchKernelGGL(flash_f16_dma64<1>, grid2, dim3(kThreads), 0, s, *a, pairs, dslot, dhq, dg);
-            else hipLaunchKernelGGL(flash_f16_dma64<2>, grid2, dim3(kThreads), 0, s, *a, pairs, dslot, dhq, dg);
+            // GQA: the query heads of one KV head on one XCD (kv_order in the kernel), where
+            // the KV heads divide evenly over the 8 XCDs.
+            const int kv_order = a->H_q > a->H_kv && (long long)a->B * a->H_kv % 8 == 0 ? 1 : 0;
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, grid2, dim3(kThreads), 0, s, *a, pairs, kv_order, dslot, dhq, dg);
+            };
+            if (a->d == 128) {
+                if (nj == 1) go(flash_f16_dma<128, 1, true>);
+                else go(flash_f16_dma<128, 2, true>);
+            } else if (a->qkv_ld) {
+                if (nj == 1) go(flash_f16_dma<64, 1, true>);
+                else go(flash_f16_dma<64, 2, true>);
+            } else if (nj == 1) go(flash_f16_dma<64, 1>);
+            else go(flash_f16_dma<64, 2>);
         } else if (a->d == 64) hipLaunchKernelGGL(flash_f16<64>, grid, dim3(kThreads), 0, s, *a);
         else hipLaunchKernelGGL(flash_f16<128>, grid, dim3(kThreads), 0, s, *a);
         return (int)hipGetLastError();

@@ -768,7 +768,7 @@ void gemm_f32(cf_gemm_args_t a, Tiling t) {
 }
 
 // ------------------------------------------------------ fp16, wave-specialised ---
-// BM x BN tiles (BM = 256 or 128) of 8 waves: waves 4-7 only issue the direct-to-LDS
+// BM x BN tiles (BM = 256, 128 or 64) of 8 waves: waves 4-7 only issue the direct-to-LDS
 // loads, waves 0-3 only read LDS and run MFMAs, and one barrier per 64-k stage orders the
 // two.  A wave that both issues a stage's DMA instructions and multiplies stalls at the
 // issue (measured ~650 clocks of every stage) and its MFMAs never overlap the loads: a
@@ -780,6 +780,13 @@ void gemm_f32(cf_gemm_args_t a, Tiling t) {
 // columns of one k) are padded by one 16-byte chunk, which the transposing B reads
 // (ds_read_b64_tr_b16) measure at the ds_read_b64 rate.  A compute wave owns 64 rows x
 // BN / NWN columns (NWN = 256 / BM waves along N).
+//
+// Row-major and row-concatenated outputs take any M and any total width that is a multiple
+// of 8: a tile over the end loads the last row or 8-column chunk again (clamped, never past
+// the operands) and stores only what exists, so an odd batch of prompts (591 x 768 x 768
+// and x 2304: 21.1 and 22.0 us in the register-staged kernel) costs what its tiles cost
+// (6.5 and 8.2 us).  64-row tiles serve the small products, where 128-row ones leave most
+// CUs idle.
 //
 // Columns are the concatenation of the segments (Q | K | V for the projection), and a
 // tile may straddle a segment boundary: every 8-column chunk belongs to one segment (the
@@ -903,8 +910,8 @@ __device__ __forceinline__ int ws_seg(const cf_gemm_args_t& a, const int (&start
 enum { WS_EPI_ROWMAJOR = 0, WS_EPI_RESIDUAL = 1, WS_EPI_QKV = 2 };
 
 template <int BM, int BN, int EPI>
-__device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], int nseg, int m0, int n0, int tid,
-                                         const _Float16* smem, bool vt_tile);
+__device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], int nseg, int m0, int n0, int rows,
+                                         int cols, int tid, const _Float16* smem, bool vt_tile);
 
 template <int BM, int BN, int S, int EPI>
 __global__ __launch_bounds__(512, 1)
@@ -922,6 +929,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
     start[1] = a.n[0];
     start[2] = a.n[0] + (a.nseg > 1 ? a.n[1] : 0);
     start[3] = start[2] + (a.nseg > 2 ? a.n[2] : 0);
+    const int ntot = start[3];
     int tile_m, tile_n;
     tile_of_block(blockIdx.x, t, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -943,7 +951,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
 #pragma unroll
         for (int v = 0; v < A_PW; v++) {
             const int row = 8 * (A_PW * cw + v) + (lane >> 3), pc = lane & 7;
-            a_off[v] = ((uint32_t)(m0 + row) * (uint32_t)K + 8u * (uint32_t)(pc ^ ((row >> 1) & 7))) * 2u;
+            a_off[v] = ((uint32_t)min(m0 + row, a.M - 1) * (uint32_t)K + 8u * (uint32_t)(pc ^ ((row >> 1) & 7))) * 2u;
         }
         const _Float16* w_ptr[W_PW];
         uint32_t w_step[W_PW];
@@ -960,7 +968,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
         const _Float16* const wb2 = a.nseg > 2 ? (const _Float16*)a.w[2] : wb1;
         const int ns0 = a.n[0], ns1 = a.nseg > 1 ? a.n[1] : ns0, ns2 = a.nseg > 2 ? a.n[2] : ns1;
         const int st1 = a.nseg > 1 ? start[1] : INT_MAX, st2 = a.nseg > 2 ? start[2] : INT_MAX;
-        const int last = n0 + BN - 8;
+        const int last = min(n0 + BN, ntot) - 8;
         const int s_lo = n0 >= st2 ? 2 : n0 >= st1 ? 1 : 0, s_hi = last >= st2 ? 2 : last >= st1 ? 1 : 0;
         if (s_hi == s_lo) {
             // One segment (every tile of a one-segment product, most of a Q|K|V one):
@@ -974,7 +982,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 nw += u < W_INSTR ? 1 : 0;
                 const int q = min(64 * u + lane, W_CH - 1);
                 const int r = q / WCPR, c = min(q - r * WCPR, BN / 8 - 1);
-                w_ptr[v] = wb + ((size_t)r * ns + (n0 + 8 * c - st));
+                w_ptr[v] = wb + ((size_t)r * ns + (min(n0 + 8 * c, last) - st));
                 w_step[v] = (uint32_t)(WS_BK * ns);
             }
         } else if (s_hi - s_lo == 1) {
@@ -989,7 +997,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 nw += u < W_INSTR ? 1 : 0;
                 const int q = min(64 * u + lane, W_CH - 1);
                 const int r = q / WCPR, c = min(q - r * WCPR, BN / 8 - 1);
-                const int gc = n0 + 8 * c;
+                const int gc = min(n0 + 8 * c, last);
                 const bool hi = gc >= shi;
                 const int ns = hi ? nhi : nlo;
                 w_ptr[v] = (hi ? whi : wlo) + ((size_t)r * ns + (gc - (hi ? shi : slo)));
@@ -1002,7 +1010,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 nw += u < W_INSTR ? 1 : 0;
                 const int q = min(64 * u + lane, W_CH - 1);
                 const int r = q / WCPR, c = min(q - r * WCPR, BN / 8 - 1);
-                const int gc = n0 + 8 * c;
+                const int gc = min(n0 + 8 * c, last);
                 const bool in1 = gc >= st1, in2 = gc >= st2;     // start[2] >= start[1]: in2 implies in1
                 const int ns = in2 ? ns2 : in1 ? ns1 : ns0;
                 w_ptr[v] = (in2 ? wb2 : in1 ? wb1 : wb0) + ((size_t)r * ns + (gc - (in2 ? st2 : in1 ? st1 : 0)));
@@ -1069,7 +1077,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 for (int j = 0; j < NJ; j++) {
                     if constexpr (CT) {
                         int col;
-                        const int sg = ws_seg(a, start, n0 + wn + 16 * j + 4 * lq, col);
+                        const int sg = ws_seg(a, start, min(n0 + wn + 16 * j + 4 * lq, ntot - 4), col);
                         const CF_GLOBAL _Float16* bias = epi.bias(sg);
                         b4[j] = bias ? *(const CF_GLOBAL h4_t*)(bias + col) : h4_t{0, 0, 0, 0};
                     } else {
@@ -1139,7 +1147,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
         }
     }
     ring_barrier();   // every loader is past its last stage and the tile is staged
-    ws_store<BM, BN, EPI>(epi, start, a.nseg, m0, n0, tid, smem, vt_tile);
+    ws_store<BM, BN, EPI>(epi, start, a.nseg, m0, n0, min(BM, a.M - m0), min(BN, ntot - n0), tid, smem, vt_tile);
 }
 
 // Store phase of gemm_f16_ws (all 512 threads): the staged tile goes out as 16-byte chunks,
@@ -1147,8 +1155,8 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
 // row) or, for v^T columns, 8 rows of one column read down the staged column.  Each pass
 // has a fixed trip count, and all of a thread's LDS reads are issued before its stores.
 template <int BM, int BN, int EPI>
-__device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], int nseg, int m0, int n0, int tid,
-                                         const _Float16* smem, bool vt_tile) {
+__device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], int nseg, int m0, int n0, int rows,
+                                         int cols, int tid, const _Float16* smem, bool vt_tile) {
     constexpr int CPR = BN / 8, NCH = BM * CPR, IT = (NCH + 511) / 512;
     constexpr bool qkv = EPI == WS_EPI_QKV;
     const WsRows wr = ws_rows(e, m0);
@@ -1157,8 +1165,8 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
 #pragma unroll
         for (int it = 0; it < IT; it++) {
             const int id = tid + 512 * it;
-            if (id < NCH) {
-                const int r = id / CPR, c8 = id - r * CPR;
+            const int r = id / CPR, c8 = id - r * CPR;
+            if (r < rows && 8 * c8 < cols) {       // rows <= BM: also the end of the tile
                 *(CF_GLOBAL h8_t*)(e.out0 + (size_t)(m0 + r) * e.n0w + n0 + 8 * c8) = *(const h8_t*)(smem + r * (BN + 8) + 8 * c8);
             }
         }
@@ -1187,7 +1195,8 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
         size_t off[IT];
 #pragma unroll
         for (int it = 0; it < IT; it++) {
-            const int id = min(tid + 512 * it, NCH - 1), r = id / CPR, c8 = id - r * CPR;
+            const int id = min(tid + 512 * it, NCH - 1), rt = id / CPR;
+            const int r = min(rt, rows - 1), c8 = min(id - rt * CPR, cols / 8 - 1);
             const float* sp = (const float*)smem + r * (BN + 4) + 8 * c8;
             off[it] = (size_t)(m0 + r) * e.n0w + n0 + 8 * c8;
             lo[it] = *(const f4_t*)sp;
@@ -1196,7 +1205,8 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
         }
 #pragma unroll
         for (int it = 0; it < IT; it++) {
-            if (tid + 512 * it >= NCH) continue;
+            const int id = tid + 512 * it, rt = id / CPR;
+            if (rt >= rows || 8 * (id - rt * CPR) >= cols) continue;
             const float f[8] = {lo[it][0], lo[it][1], lo[it][2], lo[it][3], hi[it][0], hi[it][1], hi[it][2], hi[it][3]};
             h8_t v;
 #pragma unroll
@@ -1247,7 +1257,7 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
 // (~32 B/clk per CU with whole A lines) and its MFMA work at ~60 % of the CU's 4096
 // FLOP/clk (one compute wave per SIMD), times the rounds of tiles over the CUs.
 inline double ws_cost(long long M, long long Ntot, long long K, int bm, int bn, int cus) {
-    const long long tiles = (M / bm) * (Ntot / bn);
+    const long long tiles = ((M + bm - 1) / bm) * ((Ntot + bn - 1) / bn);
     const double dma = (double)(bm + bn) * (double)K * 2.0 / 32.0;
     const double mfma = 2.0 * bm * bn * (double)K / 2500.0;
     const long long rounds = (tiles + cus - 1) / cus;
@@ -1340,11 +1350,13 @@ const WsCandidate kWsShapes[] = {
     {128, 128, ws_lds_bytes<128, 128, 3>(), launch_ws<128, 128, 3>},
     {128, 96, ws_lds_bytes<128, 96, 3>(), launch_ws<128, 96, 3>},
     {128, 64, ws_lds_bytes<128, 64, 3>(), launch_ws<128, 64, 3>},
+    {64, 128, ws_lds_bytes<64, 128, 3>(), launch_ws<64, 128, 3>},
+    {64, 64, ws_lds_bytes<64, 64, 3>(), launch_ws<64, 64, 3>},
 };
 
 // The wave-specialised shape for this product, or nullptr where the kernel does not apply
-// (fp16 only; 16-byte aligned rows and stores; M a multiple of the tile height; K a
-// multiple of 64; every segment width a multiple of 8; 32-bit A offsets).
+// (fp16 only; 16-byte aligned rows and stores; K a multiple of 64; every segment width a
+// multiple of 8; 32-bit A offsets; whole tiles for the Q|K|V scatter).
 const WsCandidate* ws_pick(const cf_gemm_args_t* a, const Tiling& t) {
     if (g_gemm_ws == 1 || a->elem != CF_ELEM_F16 || !t.epi_vec || !t.a_vec) return nullptr;
     // Row-major outputs only by default: with the Q|K|V scatter the kernel measured no
@@ -1364,7 +1376,8 @@ const WsCandidate* ws_pick(const cf_gemm_args_t* a, const Tiling& t) {
     const WsCandidate* best = nullptr;
     double best_cost = 0.0;
     for (const WsCandidate& c : kWsShapes) {
-        if (a->M % c.bm != 0 || ntot % c.bn != 0) continue;
+        // The Q|K|V scatter takes whole tiles; row-major outputs any rows and columns.
+        if (a->out_kind == CF_GEMM_OUT_QKV && (a->M % c.bm != 0 || ntot % c.bn != 0)) continue;
         // The staged tile (fp32 with a residual, else fp16) fits in the rings.
         const unsigned staged = res32 ? (unsigned)c.bm * (c.bn + 4) * 4u : (unsigned)c.bm * (c.bn + 8) * 2u;
         const unsigned staged_vt = (unsigned)c.bn * (c.bm + 8) * 2u;     // v^T tiles, column-major
@@ -1433,10 +1446,11 @@ extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
     if (const WsCandidate* c = ws_pick(a, t)) {
         long long ntot = 0;
         for (int s = 0; s < a->nseg; s++) ntot += a->n[s];
-        t.n_tiles_m = a->M / c->bm;
-        const long long blocks = (long long)t.n_tiles_m * (ntot / c->bn);
+        const long long tiles_n = (ntot + c->bn - 1) / c->bn;
+        t.n_tiles_m = (a->M + c->bm - 1) / c->bm;
+        const long long blocks = (long long)t.n_tiles_m * tiles_n;
         if (blocks <= 0 || blocks > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-        set_order(t, (int)(ntot / c->bn));
+        set_order(t, (int)tiles_n);
         const hipError_t e = c->launch(dim3((unsigned)blocks), (hipStream_t)stream, *a, t);
         if (e != hipSuccess) return (int)e;
         return (int)hipGetLastError();

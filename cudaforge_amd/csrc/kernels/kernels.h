@@ -219,8 +219,8 @@ int32_t cf_gemm_rowcat_ok(const cf_gemm_args_t* a);
  * vt (B, H_kv, d, S) -> o (B, S, H_q, d) == (B*S, H_q*d) row-major.
  * With qkv_ld > 0 the inputs are instead one row-major (B*S, qkv_ld) matrix at q whose
  * row holds Q (H_q*d) | K (H_kv*d) | V (H_kv*d) side by side, qkv_ld = (H_q + 2 H_kv) d
- * (the CF_GEMM_OUT_ROWCAT product); k and vt are unused.  Only the fp16 d = 64 kernel
- * with S % 8 == 0 reads that layout (cf_flash_rowcat_ok).
+ * (the CF_GEMM_OUT_ROWCAT product); k and vt are unused.  The fp16 d = 64 and d = 128
+ * kernels read that layout, any S (cf_flash_rowcat_ok).
  * ------------------------------------------------------------------------------- */
 typedef struct {
     const void* q;
@@ -236,9 +236,10 @@ typedef struct {
 
 int cf_launch_flash_attn(const cf_flash_args_t* a, void* stream);
 int32_t cf_flash_rowcat_ok(const cf_flash_args_t* a);
-/* Selects the fp16 d = 64 prefill attention kernel (tuning and tests): 0 the register-
- * staged kernel, 1 / 2 the DMA-ring kernel with 32 / 16 queries per wave, 3 (default)
- * the DMA-ring kernel where it applies (S % 8 == 0) with the width chosen by size. */
+/* Selects the fp16 prefill attention kernel (tuning and tests): 0 the register-staged
+ * kernel for head-major inputs, 1 / 2 the DMA-ring kernel with 32 / 16 queries per wave,
+ * 3 (default) the DMA-ring kernel where it applies (row-concatenated inputs; head-major
+ * ones with d = 64 and S % 8 == 0) with the width chosen by size. */
 void cf_flash_set_mode(int32_t mode);
 /* Causal fp16 DMA attention: 1 runs each query block and its mirror in one workgroup;
  * 0 (default) one block per workgroup, heaviest first (tests and measurements). */

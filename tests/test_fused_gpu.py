@@ -232,6 +232,30 @@ def test_prefill_row_concatenated_qkv(gpu, native, B, S, H, H_kv, causal):
     assert max_abs(outs[0], outs[2]) <= 1e-2
 
 
+@pytest.mark.parametrize("B,S,H,H_kv,d,causal", [
+    (1, 1, 2, 1, 64, True), (3, 197, 6, 2, 64, True), (1, 63, 4, 4, 128, False), (1, 65, 4, 4, 128, True),
+    (2, 131, 8, 4, 128, True), (4, 129, 4, 2, 128, False), (1, 300, 16, 16, 128, True), (2, 9, 12, 12, 64, False)])
+def test_prefill_any_length(gpu, native, B, S, H, H_kv, d, causal):
+    """Row-concatenated prefill where tiles and key blocks end early: one row, one past and
+    one short of a 64-key block, token counts that are no multiple of any GEMM tile, GQA
+    with the KV heads a multiple of the XCDs (8 positions apart in the grid) and not, both
+    query widths, against the oracle and the head-major kernels."""
+    c = FusedCase(B, S, H, H_kv, d, seed=S + d, f16=True, causal=causal, residual=S % 2 == 1, bias_std=0.02)
+    want = c.oracle()
+    try:
+        outs = []
+        for rowcat, mode in ((1, 3), (1, 1), (1, 2), (0, 3)):
+            native.mha_fused_set_rowcat(rowcat)
+            native.cf_flash_set_mode(mode)
+            outs.append(run_fused_gpu(c))
+    finally:
+        native.mha_fused_set_rowcat(1)
+        native.cf_flash_set_mode(3)
+    for o in outs:
+        assert max_abs(want, o) <= TOL16
+        assert max_abs(outs[0], o) <= 1e-2
+
+
 WS_SHAPES = [(256, 192), (256, 144), (256, 128), (256, 96), (256, 64), (256, 48), (128, 192), (128, 128),
              (128, 96), (128, 64)]
 

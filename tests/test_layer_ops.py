@@ -155,6 +155,30 @@ def test_matmul_cuda(gpu, f16, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", [(256, 48), (128, 96), (64, 64), (64, 128)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 200, 128), (129, 72, 192), (300, 328, 64)])
+def test_matmul_f16_tile_ends(gpu, native, bm, bn, M, N, K):
+    """The wave-specialised GEMM with its last row and column tiles cut short: values at the
+    ends and nothing written past the M x N result."""
+    import cudaforge_amd as cf
+    A = O.round_f16(O.normal((M, K), M + N))
+    B = O.round_f16(O.normal((K, N), K + 1, 0.0, 1.0 / np.sqrt(K)))
+    bias = O.round_f16(O.normal((N,), 5, 0.0, 0.1))
+    want = A.astype(np.float64) @ B.astype(np.float64) + bias
+    guard = 1024
+    C = cf.DeviceBuffer.from_numpy(np.full(M * N + guard, 7.0, np.float16))
+    try:
+        native.cf_gemm_set_ws_shape(bm, bn)
+        p = cf.MatmulParams(M, N, K, False, False, 1, 0, 0, 0, 0)
+        assert cf.call_op("matmul_f16_cuda", [dev(A, True), dev(B, True), dev(bias, True)], [C], p) == 0
+        got = C.download().astype(np.float32)
+    finally:
+        native.cf_gemm_set_ws_shape(0, 0)
+    assert max_abs(want, got[:M * N].reshape(M, N)) <= TOL16
+    assert np.all(got[M * N:] == 7.0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])
 def test_matmul_cuda_transposed_batched(gpu, f16, ta, tb):
