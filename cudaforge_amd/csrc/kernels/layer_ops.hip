@@ -19,62 +19,53 @@ template <typename T> struct Vec4;
 template <> struct Vec4<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct Vec4<_Float16> { typedef _Float16 type __attribute__((ext_vector_type(4))); };
 
-// LayerNorm, WPR waves (1 or 4) per row; thread r of the row holds VPL groups of 4
-// consecutive elements (group j: elements 4*(64*WPR*j + r) .. +3, masked past the end).
-// Requires D % 4 == 0 and 8/16-byte aligned rows.  Every load is unconditional (clamped to
-// the row's last group), gain and bias included, so a row costs one round trip to memory:
-// under a branch each group's load was waited for before the next (16 rows x 4096, 16
-// groups per lane: 16.0 us in a kernel trace; 4.8 us with four waves per row).
-template <typename T, int VPL, int WPR>
+// LayerNorm, one wave per row; each lane holds VPL groups of 4 consecutive elements
+// (lane l, group j: elements 4*(64*j + l) .. +3), D == 256*VPL... or fewer groups when
+// the row is shorter (masked).  Requires D % 4 == 0 and 8/16-byte aligned rows.
+template <typename T, int VPL>
 __global__ __launch_bounds__(256) void layernorm_vec(cf_layernorm_args_t a) {
     typedef typename Vec4<T>::type V;
-    constexpr int TPR = 64 * WPR;                  // threads per row
-    __shared__ float red[2][4];
-    const int r = threadIdx.x % TPR, wave = threadIdx.x >> 6;
-    const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
-    if (row >= a.N) return;                        // WPR == 4: the whole workgroup
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= a.N) return;
     const int D = a.D, ng = D >> 2;
     const V* x = (const V*)((const T*)a.x + row * D);
-    const V* g = (const V*)a.gamma;
-    const V* b = (const V*)a.beta;
-    V q[VPL], gv[VPL], bv[VPL];
-#pragma unroll
-    for (int j = 0; j < VPL; j++) q[j] = x[min(TPR * j + r, ng - 1)];
-#pragma unroll
-    for (int j = 0; j < VPL; j++) {
-        gv[j] = g[min(TPR * j + r, ng - 1)];
-        bv[j] = b[min(TPR * j + r, ng - 1)];
-    }
-    auto row_sum = [&](float s, int k) {
-        s = wave_sum(s);
-        if constexpr (WPR == 1) return s;
-        if ((threadIdx.x & 63) == 0) red[k][wave] = s;
-        __syncthreads();
-        return (red[k][0] + red[k][1]) + (red[k][2] + red[k][3]);
-    };
+    float v[VPL][4];
     float s = 0.0f;
 #pragma unroll
-    for (int j = 0; j < VPL; j++)
+    for (int j = 0; j < VPL; j++) {
+        const int gi = 64 * j + lane;
+        if (gi < ng) {
+            const V q = x[gi];
 #pragma unroll
-        for (int e = 0; e < 4; e++) s += TPR * j + r < ng ? (float)q[j][e] : 0.0f;
-    const float mean = row_sum(s, 0) / (float)D;
+            for (int e = 0; e < 4; e++) { v[j][e] = (float)q[e]; s += v[j][e]; }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[j][e] = 0.0f;
+        }
+    }
+    const float mean = wave_sum(s) / (float)D;
     float q2 = 0.0f;
 #pragma unroll
     for (int j = 0; j < VPL; j++)
+        if (64 * j + lane < ng) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float dv = (float)q[j][e] - mean;
-            q2 += TPR * j + r < ng ? dv * dv : 0.0f;
+            for (int e = 0; e < 4; e++) { const float dv = v[j][e] - mean; q2 += dv * dv; }
         }
-    const float inv_std = 1.0f / sqrtf(row_sum(q2, 1) / (float)D + a.eps);
+    const float inv_std = 1.0f / sqrtf(wave_sum(q2) / (float)D + a.eps);
+    const V* g = (const V*)a.gamma;
+    const V* b = (const V*)a.beta;
     V* y = (V*)((T*)a.y + row * D);
 #pragma unroll
     for (int j = 0; j < VPL; j++) {
-        const int gi = TPR * j + r;
-        V o;
+        const int gi = 64 * j + lane;
+        if (gi < ng) {
+            const V gv = g[gi], bv = b[gi];
+            V o;
 #pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = (T)(((float)q[j][e] - mean) * inv_std * (float)gv[j][e] + (float)bv[j][e]);
-        if (gi < ng) y[gi] = o;
+            for (int e = 0; e < 4; e++) o[e] = (T)((v[j][e] - mean) * inv_std * (float)gv[e] + (float)bv[e]);
+            y[gi] = o;
+        }
     }
 }
 
@@ -98,66 +89,22 @@ __global__ __launch_bounds__(256) void layernorm_any(cf_layernorm_args_t a) {
     for (int i = lane; i < D; i += 64) y[i] = (T)(((float)x[i] - mean) * inv_std * (float)g[i] + (float)b[i]);
 }
 
-template <typename T, int VPL>
-void launch_layernorm_vec(const cf_layernorm_args_t& a, bool wide, hipStream_t s) {
-    if (wide) hipLaunchKernelGGL((layernorm_vec<T, VPL, 4>), dim3((unsigned)a.N), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((layernorm_vec<T, VPL, 1>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
-}
-
 template <typename T>
 hipError_t launch_layernorm(const cf_layernorm_args_t& a, hipStream_t s) {
+    const unsigned blocks = (unsigned)((a.N + 3) / 4);
     const uintptr_t al = (uintptr_t)a.x | (uintptr_t)a.y | (uintptr_t)a.gamma | (uintptr_t)a.beta;
     const bool vec = a.D % 4 == 0 && al % (4 * sizeof(T)) == 0;
-    // Four waves per row for long rows (a wave would hold more than 8 groups per lane) and
-    // while one wave per row gives the CUs less than two waves each.
-    const int g1 = (a.D / 4 + 63) / 64;
-    const bool wide = g1 > 8 || (g1 > 1 && a.N < 2LL * cdna4::cu_count());
-    const int groups = wide ? (a.D / 4 + 255) / 256 : g1;
-    if (!vec || groups > 8 || (wide && a.N > 0x7fffffffLL))
-        hipLaunchKernelGGL((layernorm_any<T>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
-    else if (groups <= 1) launch_layernorm_vec<T, 1>(a, wide, s);
-    else if (groups <= 2) launch_layernorm_vec<T, 2>(a, wide, s);
-    else if (groups <= 3) launch_layernorm_vec<T, 3>(a, wide, s);
-    else if (groups <= 4) launch_layernorm_vec<T, 4>(a, wide, s);
-    else if (groups <= 6) launch_layernorm_vec<T, 6>(a, wide, s);
-    else launch_layernorm_vec<T, 8>(a, wide, s);
+    const int groups = (a.D / 4 + 63) / 64;
+    if (vec && groups <= 1) hipLaunchKernelGGL((layernorm_vec<T, 1>), dim3(blocks), dim3(256), 0, s, a);
+    else if (vec && groups <= 2) hipLaunchKernelGGL((layernorm_vec<T, 2>), dim3(blocks), dim3(256), 0, s, a);
+    else if (vec && groups <= 4) hipLaunchKernelGGL((layernorm_vec<T, 4>), dim3(blocks), dim3(256), 0, s, a);
+    else if (vec && groups <= 8) hipLaunchKernelGGL((layernorm_vec<T, 8>), dim3(blocks), dim3(256), 0, s, a);
+    else if (vec && groups <= 16) hipLaunchKernelGGL((layernorm_vec<T, 16>), dim3(blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((layernorm_any<T>), dim3(blocks), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-// Cast: grid-stride elementwise.  Between f32 and f16, eight elements per thread with
-// 16-byte accesses where both ends are aligned (`vec`; the last n % 8 one by one).
-template <typename I, typename O>
-__device__ __forceinline__ void cast8(const I* __restrict__ in, O* __restrict__ out, int64_t i, int64_t n, bool vec) {
-    typedef I i8_t __attribute__((ext_vector_type(8)));
-    typedef O o8_t __attribute__((ext_vector_type(8)));
-    if (vec && i + 8 <= n) {
-        *(o8_t*)(out + i) = __builtin_convertvector(*(const i8_t*)(in + i), o8_t);
-    } else {
-        for (int64_t j = i; j < i + 8 && j < n; j++) out[j] = (O)in[j];
-    }
-}
-template <typename I, typename O>
-__global__ __launch_bounds__(256) void cast8_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n, bool vec) {
-    for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (int64_t)gridDim.x * 2048)
-        cast8(in, out, i, n, vec);
-}
-
-// Several f32 -> f16 arrays in one launch (the mixed-precision prefill's ten operands, whose
-// ten launches of 1.5-3.2 us took longer than its products): entry e owns workgroups
-// first[e] .. first[e+1] - 1 of 2048 elements each.
-struct CastMany {
-    cf_cast_many_args_t a;
-    unsigned first[CF_CAST_MANY + 1];
-    unsigned vec;                      // bit e: entry e's ends are aligned
-};
-__global__ __launch_bounds__(256) void cast_many_kernel(CastMany c) {
-    int e = 0;
-#pragma unroll
-    for (int k = 1; k < CF_CAST_MANY; k++) e += blockIdx.x >= c.first[k] ? 1 : 0;
-    const int64_t i = ((int64_t)(blockIdx.x - c.first[e]) * 256 + threadIdx.x) * 8;
-    if (i < c.a.n[e]) cast8((const float*)c.a.in[e], (_Float16*)c.a.out[e], i, c.a.n[e], (c.vec >> e) & 1u);
-}
-
+// Cast: grid-stride elementwise.
 template <typename I, typename O>
 __global__ __launch_bounds__(256) void cast_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
@@ -201,33 +148,14 @@ extern "C" int cf_launch_cast(const void* in, void* out, int64_t n, int32_t kind
     if (!in || !out || n < 0) return (int)hipErrorInvalidValue;
     if (n == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 g(grid_1d(n)), g8(grid_1d((n + 7) / 8)), b(256);
-    const bool vec = ((uintptr_t)in | (uintptr_t)out) % 16 == 0;
+    const dim3 g(grid_1d(n)), b(256);
     switch (kind) {
         case CF_CAST_I64_F32: hipLaunchKernelGGL((cast_kernel<int64_t, float>), g, b, 0, s, (const int64_t*)in, (float*)out, n); break;
         case CF_CAST_F32_I64: hipLaunchKernelGGL((cast_kernel<float, int64_t>), g, b, 0, s, (const float*)in, (int64_t*)out, n); break;
-        case CF_CAST_F32_F16: hipLaunchKernelGGL((cast8_kernel<float, _Float16>), g8, b, 0, s, (const float*)in, (_Float16*)out, n, vec); break;
-        case CF_CAST_F16_F32: hipLaunchKernelGGL((cast8_kernel<_Float16, float>), g8, b, 0, s, (const _Float16*)in, (float*)out, n, vec); break;
+        case CF_CAST_F32_F16: hipLaunchKernelGGL((cast_kernel<float, _Float16>), g, b, 0, s, (const float*)in, (_Float16*)out, n); break;
+        case CF_CAST_F16_F32: hipLaunchKernelGGL((cast_kernel<_Float16, float>), g, b, 0, s, (const _Float16*)in, (float*)out, n); break;
         default: return (int)hipErrorInvalidValue;
     }
-    return (int)hipGetLastError();
-}
-
-extern "C" int cf_launch_cast_many(const cf_cast_many_args_t* a, void* stream) {
-    CastMany c;
-    c.a = *a;
-    c.vec = 0;
-    unsigned long long at = 0;
-    for (int e = 0; e < CF_CAST_MANY; e++) {
-        c.first[e] = (unsigned)at;
-        if (a->n[e] < 0 || (a->n[e] > 0 && (!a->in[e] || !a->out[e]))) return (int)hipErrorInvalidValue;
-        if (((uintptr_t)a->in[e] | (uintptr_t)a->out[e]) % 16 == 0) c.vec |= 1u << e;
-        at += ((unsigned long long)a->n[e] + 2047) / 2048;
-        if (at > 0x7fffffffULL) return (int)hipErrorInvalidValue;
-    }
-    c.first[CF_CAST_MANY] = (unsigned)at;
-    if (at == 0) return 0;
-    hipLaunchKernelGGL(cast_many_kernel, dim3((unsigned)at), dim3(256), 0, (hipStream_t)stream, c);
     return (int)hipGetLastError();
 }
 
