@@ -19,53 +19,62 @@ template <typename T> struct Vec4;
 template <> struct Vec4<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct Vec4<_Float16> { typedef _Float16 type __attribute__((ext_vector_type(4))); };
 
-// LayerNorm, one wave per row; each lane holds VPL groups of 4 consecutive elements
-// (lane l, group j: elements 4*(64*j + l) .. +3), D == 256*VPL... or fewer groups when
-// the row is shorter (masked).  Requires D % 4 == 0 and 8/16-byte aligned rows.
-template <typename T, int VPL>
+// LayerNorm, WPR waves (1 or 4) per row; thread r of the row holds VPL groups of 4
+// consecutive elements (group j: elements 4*(64*WPR*j + r) .. +3, masked past the end).
+// Requires D % 4 == 0 and 8/16-byte aligned rows.  Every load is unconditional (clamped to
+// the row's last group), gain and bias included, so a row costs one round trip to memory:
+// under a branch each group's load was waited for before the next (16 rows x 4096, 16
+// groups per lane: 16.0 us in a kernel trace; 4.8 us with four waves per row).
+template <typename T, int VPL, int WPR>
 __global__ __launch_bounds__(256) void layernorm_vec(cf_layernorm_args_t a) {
     typedef typename Vec4<T>::type V;
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= a.N) return;
+    constexpr int TPR = 64 * WPR;                  // threads per row
+    __shared__ float red[2][4];
+    const int r = threadIdx.x % TPR, wave = threadIdx.x >> 6;
+    const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+    if (row >= a.N) return;                        // WPR == 4: the whole workgroup
     const int D = a.D, ng = D >> 2;
     const V* x = (const V*)((const T*)a.x + row * D);
-    float v[VPL][4];
-    float s = 0.0f;
+    const V* g = (const V*)a.gamma;
+    const V* b = (const V*)a.beta;
+    V q[VPL], gv[VPL], bv[VPL];
+#pragma unroll
+    for (int j = 0; j < VPL; j++) q[j] = x[min(TPR * j + r, ng - 1)];
 #pragma unroll
     for (int j = 0; j < VPL; j++) {
-        const int gi = 64 * j + lane;
-        if (gi < ng) {
-            const V q = x[gi];
-#pragma unroll
-            for (int e = 0; e < 4; e++) { v[j][e] = (float)q[e]; s += v[j][e]; }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[j][e] = 0.0f;
-        }
+        gv[j] = g[min(TPR * j + r, ng - 1)];
+        bv[j] = b[min(TPR * j + r, ng - 1)];
     }
-    const float mean = wave_sum(s) / (float)D;
+    auto row_sum = [&](float s, int k) {
+        s = wave_sum(s);
+        if constexpr (WPR == 1) return s;
+        if ((threadIdx.x & 63) == 0) red[k][wave] = s;
+        __syncthreads();
+        return (red[k][0] + red[k][1]) + (red[k][2] + red[k][3]);
+    };
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPL; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) s += TPR * j + r < ng ? (float)q[j][e] : 0.0f;
+    const float mean = row_sum(s, 0) / (float)D;
     float q2 = 0.0f;
 #pragma unroll
     for (int j = 0; j < VPL; j++)
-        if (64 * j + lane < ng) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) { const float dv = v[j][e] - mean; q2 += dv * dv; }
+        for (int e = 0; e < 4; e++) {
+            const float dv = (float)q[j][e] - mean;
+            q2 += TPR * j + r < ng ? dv * dv : 0.0f;
         }
-    const float inv_std = 1.0f / sqrtf(wave_sum(q2) / (float)D + a.eps);
-    const V* g = (const V*)a.gamma;
-    const V* b = (const V*)a.beta;
+    const float inv_std = 1.0f / sqrtf(row_sum(q2, 1) / (float)D + a.eps);
     V* y = (V*)((T*)a.y + row * D);
 #pragma unroll
     for (int j = 0; j < VPL; j++) {
-        const int gi = 64 * j + lane;
-        if (gi < ng) {
-            const V gv = g[gi], bv = b[gi];
-            V o;
+        const int gi = TPR * j + r;
+        V o;
 #pragma unroll
-            for (int e = 0; e < 4; e++) o[e] = (T)((v[j][e] - mean) * inv_std * (float)gv[e] + (float)bv[e]);
-            y[gi] = o;
-        }
+        for (int e = 0; e < 4; e++) o[e] = (T)(((float)q[j][e] - mean) * inv_std * (float)gv[j][e] + (float)bv[j][e]);
+        if (gi < ng) y[gi] = o;
     }
 }
 
@@ -89,18 +98,29 @@ __global__ __launch_bounds__(256) void layernorm_any(cf_layernorm_args_t a) {
     for (int i = lane; i < D; i += 64) y[i] = (T)(((float)x[i] - mean) * inv_std * (float)g[i] + (float)b[i]);
 }
 
+template <typename T, int VPL>
+void launch_layernorm_vec(const cf_layernorm_args_t& a, bool wide, hipStream_t s) {
+    if (wide) hipLaunchKernelGGL((layernorm_vec<T, VPL, 4>), dim3((unsigned)a.N), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((layernorm_vec<T, VPL, 1>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
+}
+
 template <typename T>
 hipError_t launch_layernorm(const cf_layernorm_args_t& a, hipStream_t s) {
-    const unsigned blocks = (unsigned)((a.N + 3) / 4);
     const uintptr_t al = (uintptr_t)a.x | (uintptr_t)a.y | (uintptr_t)a.gamma | (uintptr_t)a.beta;
     const bool vec = a.D % 4 == 0 && al % (4 * sizeof(T)) == 0;
-    const int groups = (a.D / 4 + 63) / 64;
-    if (vec && groups <= 1) hipLaunchKernelGGL((layernorm_vec<T, 1>), dim3(blocks), dim3(256), 0, s, a);
-    else if (vec && groups <= 2) hipLaunchKernelGGL((layernorm_vec<T, 2>), dim3(blocks), dim3(256), 0, s, a);
-    else if (vec && groups <= 4) hipLaunchKernelGGL((layernorm_vec<T, 4>), dim3(blocks), dim3(256), 0, s, a);
-    else if (vec && groups <= 8) hipLaunchKernelGGL((layernorm_vec<T, 8>), dim3(blocks), dim3(256), 0, s, a);
-    else if (vec && groups <= 16) hipLaunchKernelGGL((layernorm_vec<T, 16>), dim3(blocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((layernorm_any<T>), dim3(blocks), dim3(256), 0, s, a);
+    // Four waves per row for long rows (a wave would hold more than 8 groups per lane) and
+    // while one wave per row gives the CUs less than two waves each.
+    const int g1 = (a.D / 4 + 63) / 64;
+    const bool wide = g1 > 8 || (g1 > 1 && a.N < 2LL * cdna4::cu_count());
+    const int groups = wide ? (a.D / 4 + 255) / 256 : g1;
+    if (!vec || groups > 8 || (wide && a.N > 0x7fffffffLL))
+        hipLaunchKernelGGL((layernorm_any<T>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
+    else if (groups <= 1) launch_layernorm_vec<T, 1>(a, wide, s);
+    else if (groups <= 2) launch_layernorm_vec<T, 2>(a, wide, s);
+    else if (groups <= 3) launch_layernorm_vec<T, 3>(a, wide, s);
+    else if (groups <= 4) launch_layernorm_vec<T, 4>(a, wide, s);
+    else if (groups <= 6) launch_layernorm_vec<T, 6>(a, wide, s);
+    else launch_layernorm_vec<T, 8>(a, wide, s);
     return hipGetLastError();
 }
 

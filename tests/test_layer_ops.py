@@ -103,6 +103,20 @@ def test_layernorm_f16_cuda(gpu, N, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("N", [3, 700])
+@pytest.mark.parametrize("D", [4, 256, 260, 772, 1028, 1536, 2052, 4096, 4100, 8192, 8196])
+def test_layernorm_row_widths(gpu, f16, N, D):
+    """Each count of 4-element groups per lane, full and cut short, with one wave and four
+    waves per row (few and many rows), in place."""
+    x, g, b = _ln_inputs(N, D, N + 3 * D)
+    if f16:
+        x, g, b = (O.round_f16(a) for a in (x, g, b))
+    got = _ln_gpu(x, g, b, 1e-5, f16, in_place=True)
+    assert max_abs(O.layernorm(x, g, b, 1e-5), got) <= (TOL16 if f16 else TOL32)
+
+
+@pytest.mark.gpu
 def test_cast_f32_cuda_all_pairs(gpu):
     import cudaforge_amd as cf
 
