@@ -798,15 +798,16 @@ void gemm_f32(cf_gemm_args_t a, Tiling t) {
 // read down the staged column) for v^T.
 constexpr int WS_BK = 64;
 
-template <int BM, int BN>
+// WT: W given as (N, K), so a stage of W is BN rows of 64 k, laid out and read like A.
+template <int BM, int BN, bool WT = false>
 struct WsShape {
     static constexpr int NWN = 256 / BM;           // compute waves along N
     static constexpr int WN = BN / NWN;            // columns per compute wave
     static constexpr int NJ = WN / 16;             // 16-column MFMA blocks per compute wave
     static constexpr int A_ST = BM * WS_BK;        // halves per stage of A
-    static constexpr int WCPR = BN / 8 + 1;        // 16-byte chunks per padded W row
-    static constexpr int LDW = WCPR * 8;           // halves per W row in LDS
-    static constexpr int W_CH = WS_BK * WCPR;      // chunks per W stage
+    static constexpr int WCPR = BN / 8 + 1;        // 16-byte chunks per padded (K, N) W row
+    static constexpr int LDW = WCPR * 8;           // halves per (K, N) W row in LDS
+    static constexpr int W_CH = WT ? BN * 8 : WS_BK * WCPR;   // chunks per W stage
     static constexpr int W_INSTR = (W_CH + 63) / 64;
     static constexpr int W_ST = W_INSTR * 512;     // halves per stage of W (whole DMA instructions)
     static constexpr int ST = A_ST + W_ST;
@@ -815,8 +816,8 @@ struct WsShape {
     static_assert(WN % 16 == 0 && BN % 8 == 0, "tile width");
 };
 
-template <int BM, int BN, int S>
-constexpr unsigned ws_lds_bytes() { return (unsigned)S * WsShape<BM, BN>::ST * 2u; }
+template <int BM, int BN, int S, bool WT = false>
+constexpr unsigned ws_lds_bytes() { return (unsigned)S * WsShape<BM, BN, WT>::ST * 2u; }
 
 // What the epilogue reads of the launch arguments, loaded into registers at kernel start:
 // reading them from the argument block after the main loop cost ~1 us per group of fields
@@ -907,16 +908,20 @@ __device__ __forceinline__ int ws_seg(const cf_gemm_args_t& a, const int (&start
 // Epilogue kinds of gemm_f16_ws, a template parameter so that each launch carries only its
 // own staging and store code (a run-time switch between them measured ~1 us per switch
 // on the config-3 QKV product).
-enum { WS_EPI_ROWMAJOR = 0, WS_EPI_RESIDUAL = 1, WS_EPI_QKV = 2 };
+// WS_EPI_PARTIAL: blockIdx.y is one of a.ksplit ranges of k; its fp32 sums go to
+// a.partials [range][M][total columns] straight from the accumulators (16 bytes per lane),
+// and gemm_splitk_sum adds the ranges, the bias and the residual.
+enum { WS_EPI_ROWMAJOR = 0, WS_EPI_RESIDUAL = 1, WS_EPI_QKV = 2, WS_EPI_PARTIAL = 3 };
 
 template <int BM, int BN, int EPI>
 __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], int nseg, int m0, int n0, int rows,
                                          int cols, int tid, const _Float16* smem, bool vt_tile);
 
-template <int BM, int BN, int S, int EPI>
+template <int BM, int BN, int S, int EPI, bool WT>
 __global__ __launch_bounds__(512, 1)
 void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
-    using SH = WsShape<BM, BN>;
+    using SH = WsShape<BM, BN, WT>;
+    static_assert(!WT || EPI != WS_EPI_QKV, "W (N, K): row-major outputs");
     constexpr int NJ = SH::NJ, A_ST = SH::A_ST, LDW = SH::LDW, ST = SH::ST, A_PW = SH::A_PW, W_PW = SH::W_PW;
     constexpr int WCPR = SH::WCPR, W_CH = SH::W_CH, W_INSTR = SH::W_INSTR;
     extern __shared__ __attribute__((aligned(16))) _Float16 smem_ws[];
@@ -933,7 +938,13 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
     int tile_m, tile_n;
     tile_of_block(blockIdx.x, t, tile_m, tile_n);
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int K = a.K, nk = K / WS_BK;
+    const int K = a.K;
+    int kt0 = 0, nk = K / WS_BK;                   // this workgroup's first stage and stages
+    if constexpr (EPI == WS_EPI_PARTIAL) {
+        const int per = (nk + a.ksplit - 1) / a.ksplit;   // the launcher leaves no range empty
+        kt0 = (int)blockIdx.y * per;
+        nk = min(nk, kt0 + per) - kt0;
+    }
     // Every column of the tile goes to v^T: accumulate C and stage it column-major.
     const bool vt_tile = EPI == WS_EPI_QKV && a.nseg == 3 && n0 >= start[2];
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
@@ -946,7 +957,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
         // stage's first k) plus per-lane 32-bit offsets.  W: instruction u covers padded
         // chunks 64u .. 64u+63 of the stage; a lane keeps its chunk's 64-bit address and
         // steps it by 64 rows of its segment per stage (pad chunks re-read the row's last).
-        const _Float16* __restrict__ A = (const _Float16*)a.a;
+        const _Float16* __restrict__ A = (const _Float16*)a.a + (size_t)kt0 * WS_BK;
         uint32_t a_off[A_PW];
 #pragma unroll
         for (int v = 0; v < A_PW; v++) {
@@ -970,7 +981,18 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
         const int st1 = a.nseg > 1 ? start[1] : INT_MAX, st2 = a.nseg > 2 ? start[2] : INT_MAX;
         const int last = min(n0 + BN, ntot) - 8;
         const int s_lo = n0 >= st2 ? 2 : n0 >= st1 ? 1 : 0, s_hi = last >= st2 ? 2 : last >= st1 ? 1 : 0;
-        if (s_hi == s_lo) {
+        if constexpr (WT) {
+            // (N, K), one segment: instruction u covers W rows (columns of C) 8u .. 8u+7 of
+            // the tile, swizzled like A; rows past the last column re-read it.
+#pragma unroll
+            for (int v = 0; v < W_PW; v++) {
+                const int u = cw + 4 * v;
+                nw += u < W_INSTR ? 1 : 0;
+                const int row = min(8 * u + (lane >> 3), BN - 1), pc = lane & 7;
+                w_ptr[v] = wb0 + (size_t)min(n0 + row, ntot - 1) * K + 8 * (pc ^ ((row >> 1) & 7));
+                w_step[v] = WS_BK;
+            }
+        } else if (s_hi == s_lo) {
             // One segment (every tile of a one-segment product, most of a Q|K|V one):
             // wave-uniform base, width and start.
             const _Float16* const wb = s_lo == 2 ? wb2 : s_lo == 1 ? wb1 : wb0;
@@ -1017,6 +1039,10 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 w_step[v] = (uint32_t)(WS_BK * ns);
             }
         }
+        if constexpr (EPI == WS_EPI_PARTIAL)
+            if (kt0)
+#pragma unroll
+                for (int v = 0; v < W_PW; v++) w_ptr[v] += (size_t)kt0 * w_step[v];
         const uint32_t lds0 = lds_offset(smem);
         const uint32_t a_lds = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(A_PW * cw) * 1024u);
         const uint32_t w_lds = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)A_ST * 2u + (uint32_t)cw * 1024u);
@@ -1059,8 +1085,14 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 const int row = wm + 16 * i + lr;
                 a_rd[h][i] = row * WS_BK + 8 * ((4 * h + lq) ^ ((row >> 1) & 7));
             }
+        // W fragments: k rows (K, N) read transposed, w_rd[e] for their two halves; (N, K)
+        // rows as they are, w_rd[h] for the stage's two 32-k halves (j adds 16 rows, a
+        // multiple of the swizzle's period).
 #pragma unroll
-        for (int e = 0; e < 2; e++) w_rd[e] = A_ST + (8 * lq + 4 * e + (lr >> 2)) * LDW + wn + 4 * (lr & 3);
+        for (int e = 0; e < 2; e++) {
+            if constexpr (WT) w_rd[e] = A_ST + (wn + lr) * WS_BK + 8 * ((4 * e + lq) ^ (((wn + lr) >> 1) & 7));
+            else w_rd[e] = A_ST + (8 * lq + 4 * e + (lr >> 2)) * LDW + wn + 4 * (lr & 3);
+        }
         // CT: accumulate C^T (operands swapped), acc[i][j][e] = C[wm + 16i + lr][wn + 16j + 4lq + e],
         // for destinations contiguous along n; otherwise C, acc[i][j][e] = C[wm + 16i + 4lq + e]
         // [wn + 16j + lr], for tiles whose every column goes to v^T (contiguous along s).
@@ -1085,7 +1117,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                     }
                 }
             };
-            if constexpr (EPI != WS_EPI_QKV) load_bias();
+            if constexpr (EPI == WS_EPI_ROWMAJOR || EPI == WS_EPI_RESIDUAL) load_bias();
             f4_t acc[4][NJ];
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -1101,8 +1133,10 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
 #pragma unroll
                     for (int i = 0; i < 4; i++) af[i] = *(const h8_t*)(st + a_rd[h][i]);
 #pragma unroll
-                    for (int j = 0; j < NJ; j++)
-                        bf[j] = b_frag_tr(st + 32 * h * LDW + w_rd[0] + 16 * j, st + 32 * h * LDW + w_rd[1] + 16 * j);
+                    for (int j = 0; j < NJ; j++) {
+                        if constexpr (WT) bf[j] = *(const h8_t*)(st + w_rd[h] + 16 * j * WS_BK);
+                        else bf[j] = b_frag_tr(st + 32 * h * LDW + w_rd[0] + 16 * j, st + 32 * h * LDW + w_rd[1] + 16 * j);
+                    }
 #pragma unroll
                     for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -1113,7 +1147,18 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
                 ring_barrier();
             });
             if constexpr (EPI == WS_EPI_QKV) load_bias();
-            if constexpr (CT) {
+            if constexpr (EPI == WS_EPI_PARTIAL) {
+                float* const part = a.partials + (size_t)blockIdx.y * a.M * ntot;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int m = m0 + wm + 16 * i + lr;
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+                        const int n = n0 + wn + 16 * j + 4 * lq;
+                        if (m < a.M && n < ntot) *(f4_t*)(part + (size_t)m * ntot + n) = acc[i][j];
+                    }
+                }
+            } else if constexpr (CT) {
                 // Stage [BM][BN]: bias added in fp32; fp16 (one rounding) without a residual,
                 // fp32 with one.  A lane's four columns lie in one segment (n[s] % 8 == 0).
                 constexpr bool f32s = EPI == WS_EPI_RESIDUAL;
@@ -1146,6 +1191,7 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
             run(std::true_type{});
         }
     }
+    if constexpr (EPI == WS_EPI_PARTIAL) return;
     ring_barrier();   // every loader is past its last stage and the tile is staged
     ws_store<BM, BN, EPI>(epi, start, a.nseg, m0, n0, min(BM, a.M - m0), min(BN, ntot - n0), tid, smem, vt_tile);
 }
@@ -1160,15 +1206,28 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
     constexpr int CPR = BN / 8, NCH = BM * CPR, IT = (NCH + 511) / 512;
     constexpr bool qkv = EPI == WS_EPI_QKV;
     const WsRows wr = ws_rows(e, m0);
+    // Whole tiles skip the end-of-matrix tests (with them, BERT-base's output
+    // projection measured 9.0 us, without 8.45).
+    const bool whole = rows == BM && cols == BN;
     if constexpr (EPI == WS_EPI_ROWMAJOR) {
         // Row-major C: consecutive threads along a row.
+        if (whole) {
+#pragma unroll
+            for (int it = 0; it < IT; it++) {
+                const int id = tid + 512 * it;
+                if (id < NCH) {
+                    const int r = id / CPR, c8 = id - r * CPR;
+                    *(CF_GLOBAL h8_t*)(e.out0 + (size_t)(m0 + r) * e.n0w + n0 + 8 * c8) = *(const h8_t*)(smem + r * (BN + 8) + 8 * c8);
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int it = 0; it < IT; it++) {
             const int id = tid + 512 * it;
             const int r = id / CPR, c8 = id - r * CPR;
-            if (r < rows && 8 * c8 < cols) {       // rows <= BM: also the end of the tile
+            if (r < rows && 8 * c8 < cols)         // rows <= BM: also the end of the tile
                 *(CF_GLOBAL h8_t*)(e.out0 + (size_t)(m0 + r) * e.n0w + n0 + 8 * c8) = *(const h8_t*)(smem + r * (BN + 8) + 8 * c8);
-            }
         }
         return;
     }
@@ -1190,29 +1249,34 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
     }
     if constexpr (EPI == WS_EPI_RESIDUAL) {
         const CF_GLOBAL _Float16* __restrict__ res = e.res;
-        f4_t lo[IT], hi[IT];
-        h8_t rv[IT];
-        size_t off[IT];
+        auto add_and_store = [&](auto whole_c) {
+            constexpr bool W = decltype(whole_c)::value;
+            f4_t lo[IT], hi[IT];
+            h8_t rv[IT];
+            size_t off[IT];
 #pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int id = min(tid + 512 * it, NCH - 1), rt = id / CPR;
-            const int r = min(rt, rows - 1), c8 = min(id - rt * CPR, cols / 8 - 1);
-            const float* sp = (const float*)smem + r * (BN + 4) + 8 * c8;
-            off[it] = (size_t)(m0 + r) * e.n0w + n0 + 8 * c8;
-            lo[it] = *(const f4_t*)sp;
-            hi[it] = *(const f4_t*)(sp + 4);
-            rv[it] = *(const CF_GLOBAL h8_t*)(res + off[it]);
-        }
+            for (int it = 0; it < IT; it++) {
+                const int id = min(tid + 512 * it, NCH - 1), rt = id / CPR, ct = id - rt * CPR;
+                const int r = W ? rt : min(rt, rows - 1), c8 = W ? ct : min(ct, cols / 8 - 1);
+                const float* sp = (const float*)smem + r * (BN + 4) + 8 * c8;
+                off[it] = (size_t)(m0 + r) * e.n0w + n0 + 8 * c8;
+                lo[it] = *(const f4_t*)sp;
+                hi[it] = *(const f4_t*)(sp + 4);
+                rv[it] = *(const CF_GLOBAL h8_t*)(res + off[it]);
+            }
 #pragma unroll
-        for (int it = 0; it < IT; it++) {
-            const int id = tid + 512 * it, rt = id / CPR;
-            if (rt >= rows || 8 * (id - rt * CPR) >= cols) continue;
-            const float f[8] = {lo[it][0], lo[it][1], lo[it][2], lo[it][3], hi[it][0], hi[it][1], hi[it][2], hi[it][3]};
-            h8_t v;
+            for (int it = 0; it < IT; it++) {
+                const int id = tid + 512 * it, rt = id / CPR;
+                if (W ? id >= NCH : rt >= rows || 8 * (id - rt * CPR) >= cols) continue;
+                const float f[8] = {lo[it][0], lo[it][1], lo[it][2], lo[it][3], hi[it][0], hi[it][1], hi[it][2], hi[it][3]};
+                h8_t v;
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = (_Float16)(f[e] + (float)rv[it][e]);
-            *(CF_GLOBAL h8_t*)(e.out0 + off[it]) = v;
-        }
+                for (int k = 0; k < 8; k++) v[k] = (_Float16)(f[k] + (float)rv[it][k]);
+                *(CF_GLOBAL h8_t*)(e.out0 + off[it]) = v;
+            }
+        };
+        if (whole) add_and_store(std::true_type{});
+        else add_and_store(std::false_type{});
         return;
     }
     {
@@ -1253,15 +1317,56 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
     }
 }
 
-// Per-tile cost model of the wave-specialised kernel, in CU clocks: the larger of its DMA
-// (~32 B/clk per CU with whole A lines) and its MFMA work at ~60 % of the CU's 4096
-// FLOP/clk (one compute wave per SIMD), times the rounds of tiles over the CUs.
-inline double ws_cost(long long M, long long Ntot, long long K, int bm, int bn, int cus) {
-    const long long tiles = ((M + bm - 1) / bm) * ((Ntot + bn - 1) / bn);
-    const double dma = (double)(bm + bn) * (double)K * 2.0 / 32.0;
-    const double mfma = 2.0 * bm * bn * (double)K / 2500.0;
-    const long long rounds = (tiles + cus - 1) / cus;
-    return (double)rounds * (dma > mfma ? dma : mfma);
+// Sum of gemm_f16_ws's k ranges: KS >= a.ksplit partials of four columns of one row per
+// thread, all loaded before the first add (the range index clamped, the surplus left out),
+// plus bias and residual in fp32 and one rounding.
+template <int KS>
+__global__ __launch_bounds__(64)
+void gemm_splitk_sum(cf_gemm_args_t a, int ntot, FastDiv div_row) {
+    const int id = blockIdx.x * 64 + threadIdx.x;          // four columns: M * ntot / 4 < 2^31
+    const int m = fastdiv(id, div_row), n = 4 * (id - m * (ntot / 4));
+    if (m >= a.M) return;
+    const float* p = a.partials + (size_t)m * ntot + n;
+    const size_t plane = (size_t)a.M * ntot;
+    f4_t v[KS];
+#pragma unroll
+    for (int k = 0; k < KS; k++) v[k] = *(const f4_t*)(p + (size_t)min(k, a.ksplit - 1) * plane);
+    const int n1 = a.n[0], n2 = n1 + (a.nseg > 1 ? a.n[1] : 0);
+    const int seg = a.nseg > 2 && n >= n2 ? 2 : a.nseg > 1 && n >= n1 ? 1 : 0;
+    const _Float16* bias = (const _Float16*)(seg == 2 ? a.bias[2] : seg == 1 ? a.bias[1] : a.bias[0]);
+    const int col = n - (seg == 2 ? n2 : seg == 1 ? n1 : 0);
+    const h4_t b = bias ? *(const h4_t*)(bias + col) : h4_t{0, 0, 0, 0};
+    const h4_t r = a.residual ? *(const h4_t*)((const _Float16*)a.residual + (size_t)m * ntot + n) : h4_t{0, 0, 0, 0};
+    f4_t s = v[0];
+#pragma unroll
+    for (int k = 1; k < KS; k++)
+        if (k < a.ksplit) s += v[k];
+    h4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = (_Float16)(s[e] + (float)b[e] + (float)r[e]);
+    *(h4_t*)((_Float16*)a.out[0] + (size_t)m * ntot + n) = o;
+}
+
+// Cost model of the wave-specialised kernel, in CU clocks, fitted to a sweep of every tile
+// and range count over M of 1 to 2100 and (K, N) of 768 x 768 to 14336 x 4096, both W
+// layouts (its choice is on average 2 % off the best measured one).  A stage takes the
+// larger of its DMA (34 B/clk per CU), its MFMA work (2400 FLOP/clk) and 360 clk of issue
+// and barrier; a tile its stages, times the rounds of tiles over the CUs; a product at
+// least the time its operands take at 31 B/clk per CU that has a tile and 2500 B/clk (6
+// TB/s) in all.  k ranges add the second launch (8900 clk, 3.7 us) and the partial sums'
+// way through memory.
+constexpr int kWsMaxSplit = 16;
+inline float ws_cost(float mk_kn_bytes, float mn, int bm, int bn, int tiles, int stages, int ks, int rounds) {
+    float stage = 360.0f;
+    const float dma = (float)((bm + bn) * WS_BK * 2) * (1.0f / 34.0f), mfma = (float)(2 * bm * bn * WS_BK) * (1.0f / 2400.0f);
+    if (dma > stage) stage = dma;
+    if (mfma > stage) stage = mfma;
+    float t = (float)rounds * (float)stages * stage;
+    const float rate = 31.0f * (float)tiles;
+    const float mem = mk_kn_bytes / (rate < 2500.0f ? rate : 2500.0f);
+    t = mem > t ? mem + 0.05f * t : t + 0.05f * mem;      // the smaller one breaks ties
+    if (ks > 1) t += 8900.0f + (float)ks * mn * (8.0f / 1900.0f);
+    return t;
 }
 
 int g_gemm_stages = 0;   // tuning override of the direct-to-LDS kernel's ring depth (3, 4; 0 = automatic)
@@ -1306,126 +1411,138 @@ void launch_async_192(dim3 grid, hipStream_t s, const cf_gemm_args_t& a, const T
 int g_gemm_ws = 0;        // 0: wave-specialised kernel where it applies; 1: never
 int g_gemm_ws_bm = 0;     // tuning/test override of its tile (both 0 = cost model)
 int g_gemm_ws_bn = 0;
+int g_gemm_ws_ks = 0;     // test override of its k ranges (0 = cost model)
 
 // The wave-specialised kernel's dynamic LDS above 64 KB is enabled once per device and
 // instantiation (a bit per device id below 64, every launch above).
-template <int BM, int BN, int S, int EPI>
+template <int BM, int BN, int S, int EPI, bool WT>
 hipError_t launch_ws_epi(dim3 grid, hipStream_t st, const cf_gemm_args_t& a, const Tiling& t) {
-    constexpr unsigned lds = ws_lds_bytes<BM, BN, S>();
+    constexpr unsigned lds = ws_lds_bytes<BM, BN, S, WT>();
     static std::atomic<uint64_t> raised{0};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev >= 64 || !((raised.load(std::memory_order_acquire) >> dev) & 1u)) {
-        e = hipFuncSetAttribute((const void*)gemm_f16_ws<BM, BN, S, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds);
+        e = hipFuncSetAttribute((const void*)gemm_f16_ws<BM, BN, S, EPI, WT>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         if (dev < 64) raised.fetch_or(1ull << dev, std::memory_order_release);
     }
-    hipLaunchKernelGGL((gemm_f16_ws<BM, BN, S, EPI>), grid, dim3(512), lds, st, a, t);
+    hipLaunchKernelGGL((gemm_f16_ws<BM, BN, S, EPI, WT>), grid, dim3(512), lds, st, a, t);
     return hipSuccess;
 }
 
 template <int BM, int BN, int S>
 hipError_t launch_ws(dim3 grid, hipStream_t st, const cf_gemm_args_t& a, const Tiling& t) {
-    if (a.out_kind == CF_GEMM_OUT_QKV) return launch_ws_epi<BM, BN, S, WS_EPI_QKV>(grid, st, a, t);
-    if (a.residual) return launch_ws_epi<BM, BN, S, WS_EPI_RESIDUAL>(grid, st, a, t);
-    return launch_ws_epi<BM, BN, S, WS_EPI_ROWMAJOR>(grid, st, a, t);
+    if (a.ksplit > 1) {
+        // k ranges pay off on small outputs only (ws_cost), where the small tiles are taken.
+        if constexpr (BM <= 128)
+            return a.w_nk ? launch_ws_epi<BM, BN, S, WS_EPI_PARTIAL, true>(grid, st, a, t)
+                          : launch_ws_epi<BM, BN, S, WS_EPI_PARTIAL, false>(grid, st, a, t);
+        return hipErrorInvalidValue;
+    }
+    if (a.w_nk)
+        return a.residual ? launch_ws_epi<BM, BN, S, WS_EPI_RESIDUAL, true>(grid, st, a, t)
+                          : launch_ws_epi<BM, BN, S, WS_EPI_ROWMAJOR, true>(grid, st, a, t);
+    if (a.out_kind == CF_GEMM_OUT_QKV) return launch_ws_epi<BM, BN, S, WS_EPI_QKV, false>(grid, st, a, t);
+    if (a.residual) return launch_ws_epi<BM, BN, S, WS_EPI_RESIDUAL, false>(grid, st, a, t);
+    return launch_ws_epi<BM, BN, S, WS_EPI_ROWMAJOR, false>(grid, st, a, t);
 }
 
+// 64-row tiles come with a ring of 6 stages, for grids of at most one tile per CU (more of
+// the k loop's latency covered: 232 x 4096 x 4096, W (N, K): 17.6 -> 14.9 us), and of 3, of
+// which a CU holds two or three (591 x 2304 x 768 at 64 x 64, 360 tiles: 7.8 us, 6 stages
+// 9.4).
+enum { WS_ANY = 0, WS_DEEP = 1, WS_SHALLOW = 2 };
 struct WsCandidate {
-    int bm, bn;
-    unsigned lds;
+    int bm, bn, depth;
+    unsigned lds, lds_nk;    // dynamic LDS with W (K, N) and (N, K)
     hipError_t (*launch)(dim3, hipStream_t, const cf_gemm_args_t&, const Tiling&);
 };
 // 256-row tiles hold 192 columns on 2 stages (LDS), narrower ones on 3; 128-row tiles on 3.
 const WsCandidate kWsShapes[] = {
-    {256, 192, ws_lds_bytes<256, 192, 2>(), launch_ws<256, 192, 2>},
-    {256, 144, ws_lds_bytes<256, 144, 3>(), launch_ws<256, 144, 3>},
-    {256, 128, ws_lds_bytes<256, 128, 3>(), launch_ws<256, 128, 3>},
-    {256, 96, ws_lds_bytes<256, 96, 3>(), launch_ws<256, 96, 3>},
-    {256, 64, ws_lds_bytes<256, 64, 3>(), launch_ws<256, 64, 3>},
-    {256, 48, ws_lds_bytes<256, 48, 3>(), launch_ws<256, 48, 3>},
-    {128, 192, ws_lds_bytes<128, 192, 3>(), launch_ws<128, 192, 3>},
-    {128, 128, ws_lds_bytes<128, 128, 3>(), launch_ws<128, 128, 3>},
-    {128, 96, ws_lds_bytes<128, 96, 3>(), launch_ws<128, 96, 3>},
-    {128, 64, ws_lds_bytes<128, 64, 3>(), launch_ws<128, 64, 3>},
-    {64, 128, ws_lds_bytes<64, 128, 3>(), launch_ws<64, 128, 3>},
-    {64, 64, ws_lds_bytes<64, 64, 3>(), launch_ws<64, 64, 3>},
+    {256, 192, WS_ANY, ws_lds_bytes<256, 192, 2>(), ws_lds_bytes<256, 192, 2, true>(), launch_ws<256, 192, 2>},
+    {256, 144, WS_ANY, ws_lds_bytes<256, 144, 3>(), ws_lds_bytes<256, 144, 3, true>(), launch_ws<256, 144, 3>},
+    {256, 128, WS_ANY, ws_lds_bytes<256, 128, 3>(), ws_lds_bytes<256, 128, 3, true>(), launch_ws<256, 128, 3>},
+    {256, 96, WS_ANY, ws_lds_bytes<256, 96, 3>(), ws_lds_bytes<256, 96, 3, true>(), launch_ws<256, 96, 3>},
+    {256, 64, WS_ANY, ws_lds_bytes<256, 64, 3>(), ws_lds_bytes<256, 64, 3, true>(), launch_ws<256, 64, 3>},
+    {256, 48, WS_ANY, ws_lds_bytes<256, 48, 3>(), ws_lds_bytes<256, 48, 3, true>(), launch_ws<256, 48, 3>},
+    {128, 192, WS_ANY, ws_lds_bytes<128, 192, 3>(), ws_lds_bytes<128, 192, 3, true>(), launch_ws<128, 192, 3>},
+    {128, 128, WS_ANY, ws_lds_bytes<128, 128, 3>(), ws_lds_bytes<128, 128, 3, true>(), launch_ws<128, 128, 3>},
+    {128, 96, WS_ANY, ws_lds_bytes<128, 96, 3>(), ws_lds_bytes<128, 96, 3, true>(), launch_ws<128, 96, 3>},
+    {128, 64, WS_ANY, ws_lds_bytes<128, 64, 3>(), ws_lds_bytes<128, 64, 3, true>(), launch_ws<128, 64, 3>},
+    {64, 128, WS_DEEP, ws_lds_bytes<64, 128, 6>(), ws_lds_bytes<64, 128, 6, true>(), launch_ws<64, 128, 6>},
+    {64, 64, WS_DEEP, ws_lds_bytes<64, 64, 6>(), ws_lds_bytes<64, 64, 6, true>(), launch_ws<64, 64, 6>},
+    {64, 128, WS_SHALLOW, ws_lds_bytes<64, 128, 3>(), ws_lds_bytes<64, 128, 3, true>(), launch_ws<64, 128, 3>},
+    {64, 64, WS_SHALLOW, ws_lds_bytes<64, 64, 3>(), ws_lds_bytes<64, 64, 3, true>(), launch_ws<64, 64, 3>},
 };
+constexpr int kWsCount = (int)(sizeof(kWsShapes) / sizeof(kWsShapes[0]));
 
 // The wave-specialised shape for this product, or nullptr where the kernel does not apply
 // (fp16 only; 16-byte aligned rows and stores; K a multiple of 64; every segment width a
 // multiple of 8; 32-bit A offsets; whole tiles for the Q|K|V scatter).
-const WsCandidate* ws_pick(const cf_gemm_args_t* a, const Tiling& t) {
-    if (g_gemm_ws == 1 || a->elem != CF_ELEM_F16 || !t.epi_vec || !t.a_vec) return nullptr;
+struct WsChoice {
+    int i;      // index into kWsShapes, -1 where the kernel does not apply
+    int ks;     // k ranges
+};
+WsChoice ws_pick(const cf_gemm_args_t* a, const Tiling& t) {
+    const WsChoice none{-1, 1};
+    if (g_gemm_ws == 1 || a->elem != CF_ELEM_F16 || !t.epi_vec || !t.a_vec) return none;
+    if (a->w_nk && (a->nseg != 1 || a->out_kind != CF_GEMM_OUT_ROWMAJOR)) return none;
     // Row-major outputs only by default: with the Q|K|V scatter the kernel measured no
     // faster than the pipelined one (BERT-base 4096 x 2304 x 768: 23.8 vs 23.2 us with
     // biases; the same product stored row-major takes 19.2 us), while the output
     // projections gain (4096 x 768 x 768: 8.4 vs 9.9 us; 4096 x 1024 x 1024: 12.1 vs
     // 13.3 us).  A tile override (cf_gemm_set_ws_shape) still routes the scatter here.
-    if (a->out_kind == CF_GEMM_OUT_QKV && g_gemm_ws_bm == 0) return nullptr;
-    if (a->out_kind == CF_GEMM_OUT_ROWCAT && a->residual) return nullptr;
-    if (a->K % WS_BK != 0 || (long long)a->M * a->K * 2 >= (1LL << 32)) return nullptr;
+    if (a->out_kind == CF_GEMM_OUT_QKV && g_gemm_ws_bm == 0) return none;
+    if (a->out_kind == CF_GEMM_OUT_ROWCAT && a->residual) return none;
+    if (a->K % WS_BK != 0 || (long long)a->M * a->K * 2 >= (1LL << 32)) return none;
     long long ntot = 0;
     for (int s = 0; s < a->nseg; s++) {
-        if (!t.w_vec[s] || a->n[s] % 8 != 0 || (uintptr_t)a->bias[s] % 16 != 0) return nullptr;
+        if (!t.w_vec[s] || a->n[s] % 8 != 0 || (uintptr_t)a->bias[s] % 16 != 0) return none;
         ntot += a->n[s];
     }
     const bool res32 = a->residual != nullptr && a->out_kind == CF_GEMM_OUT_ROWMAJOR;
-    const WsCandidate* best = nullptr;
-    double best_cost = 0.0;
-    for (const WsCandidate& c : kWsShapes) {
+    // k ranges: any row-major product (a->partials is not looked at here, so that the plan
+    // can ask for it).  Every range holds at least two stages and none is empty.
+    const int nk = a->K / WS_BK, cus = cu_count();
+    const bool may_split = a->out_kind != CF_GEMM_OUT_QKV && (long long)a->M * ntot < (1LL << 30);
+    const float bytes = ((float)a->M * (float)a->K + (float)a->K * (float)ntot) * 2.0f;
+    const float mn = (float)a->M * (float)ntot;
+    WsChoice best = none;
+    float best_cost = 0.0f;
+    for (int i = 0; i < kWsCount; i++) {
+        const WsCandidate& c = kWsShapes[i];
         // The Q|K|V scatter takes whole tiles; row-major outputs any rows and columns.
         if (a->out_kind == CF_GEMM_OUT_QKV && (a->M % c.bm != 0 || ntot % c.bn != 0)) continue;
         // The staged tile (fp32 with a residual, else fp16) fits in the rings.
         const unsigned staged = res32 ? (unsigned)c.bm * (c.bn + 4) * 4u : (unsigned)c.bm * (c.bn + 8) * 2u;
         const unsigned staged_vt = (unsigned)c.bn * (c.bm + 8) * 2u;     // v^T tiles, column-major
-        if (staged > c.lds || staged_vt > c.lds) continue;
-        if (c.bm == g_gemm_ws_bm && c.bn == g_gemm_ws_bn) return &c;   // an override that fits
-        const double cost = ws_cost(a->M, ntot, a->K, c.bm, c.bn, cu_count());
-        if (!best || cost < best_cost) {
-            best = &c;
-            best_cost = cost;
+        const unsigned lds = a->w_nk ? c.lds_nk : c.lds;
+        if (staged > lds || (a->out_kind == CF_GEMM_OUT_QKV && staged_vt > lds)) continue;
+        const bool forced = c.bm == g_gemm_ws_bm && c.bn == g_gemm_ws_bn;   // an override that fits
+        const long long tiles1 = (a->M + c.bm - 1LL) / c.bm * ((ntot + c.bn - 1) / c.bn);
+        if (tiles1 > 0x3fffffffLL) continue;
+        for (int ks = 1; ks <= kWsMaxSplit; ks++) {
+            if (ks > 1 && (!may_split || c.bm > 128 || tiles1 * ks > 4LL * cus)) break;
+            const int per = (nk + ks - 1) / ks, tiles = (int)tiles1 * ks, rounds = (tiles + cus - 1) / cus;
+            if (ks > 1 && (per < 2 || (ks - 1) * per >= nk)) continue;
+            if (ks > 1 && g_gemm_ws_ks != ks && (forced || g_gemm_ws_ks > 0)) continue;
+            // The deep rings leave one workgroup per CU, the shallow ones two or three.
+            if (c.depth == WS_DEEP ? rounds > 1 : c.depth == WS_SHALLOW && rounds == 1) continue;
+            float cost = ws_cost(bytes, mn, c.bm, c.bn, tiles, per, ks, rounds);
+            if (g_gemm_ws_ks == ks) cost -= 1e15f;
+            if (forced) cost -= 1e20f;
+            if (best.i < 0 || cost < best_cost) {
+                best = WsChoice{i, ks};
+                best_cost = cost;
+            }
         }
     }
     return best;
 }
 
-}  // namespace
-
-extern "C" void cf_gemm_set_stages(int32_t stages) { g_gemm_stages = stages; }
-
-extern "C" void cf_gemm_set_bk(int32_t bk) { g_gemm_bk = bk == 32 || bk == 64 ? bk : 0; }
-
-extern "C" void cf_gemm_set_ksplit(int32_t ks) { g_gemm_ksplit = ks == 1 || ks == 2 ? ks : 0; }
-
-extern "C" void cf_gemm_set_bn(int32_t bn) { g_gemm_bn = bn == 96 || bn == 128 || bn == 192 ? bn : 0; }
-
-extern "C" void cf_gemm_set_ws(int32_t mode) { g_gemm_ws = mode == 1 ? 1 : 0; }
-
-// The checks cf_launch_gemm runs before taking the wave-specialised kernel, for a
-// row-concatenated output (which only that kernel writes).
-extern "C" int32_t cf_gemm_rowcat_ok(const cf_gemm_args_t* a) {
-    if (a->out_kind != CF_GEMM_OUT_ROWCAT || a->nseg < 1 || a->nseg > 3 || a->M <= 0 || a->K <= 0) return 0;
-    Tiling t{};
-    t.a_vec = (a->K % 8 == 0) && ((uintptr_t)a->a % 16 == 0);
-    for (int s = 0; s < a->nseg; s++) t.w_vec[s] = (a->n[s] % 8 == 0) && ((uintptr_t)a->w[s] % 16 == 0);
-    t.epi_vec = (uintptr_t)a->out[0] % 16 == 0;
-    return ws_pick(a, t) ? 1 : 0;
-}
-
-extern "C" void cf_gemm_set_ws_shape(int32_t bm, int32_t bn) {
-    g_gemm_ws_bm = bm > 0 ? bm : 0;
-    g_gemm_ws_bn = bn > 0 ? bn : 0;
-}
-
-int g_gemm_group_m = 0;  // tuning override of the tile-order group height (0 = kGroupM)
-
-extern "C" void cf_gemm_set_group_m(int32_t group_m) { g_gemm_group_m = group_m > 0 ? group_m : 0; }
-
-extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
-    if (a->nseg < 1 || a->nseg > 3 || a->M <= 0 || a->K <= 0) return (int)hipErrorInvalidValue;
+Tiling gemm_tiling(const cf_gemm_args_t* a) {
     Tiling t{};
     // fp16 reads 8 halves at a time from A and W; fp32 reads 4 floats.
     const int vec = a->elem == CF_ELEM_F16 ? 8 : 4;
@@ -1440,19 +1557,75 @@ extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
     if (a->out_kind == CF_GEMM_OUT_ROWMAJOR) ev = ev && a->n[0] % 8 == 0;
     else if (a->out_kind == CF_GEMM_OUT_QKV) ev = ev && a->d % 8 == 0 && a->S % 8 == 0;
     t.epi_vec = ev;
+    return t;
+}
+
+bool gemm_args_ok(const cf_gemm_args_t* a) { return a->nseg >= 1 && a->nseg <= 3 && a->M > 0 && a->K > 0; }
+
+}  // namespace
+
+extern "C" void cf_gemm_set_stages(int32_t stages) { g_gemm_stages = stages; }
+
+extern "C" void cf_gemm_set_bk(int32_t bk) { g_gemm_bk = bk == 32 || bk == 64 ? bk : 0; }
+
+extern "C" void cf_gemm_set_ksplit(int32_t ks) { g_gemm_ksplit = ks == 1 || ks == 2 ? ks : 0; }
+
+extern "C" void cf_gemm_set_bn(int32_t bn) { g_gemm_bn = bn == 96 || bn == 128 || bn == 192 ? bn : 0; }
+
+extern "C" void cf_gemm_set_ws(int32_t mode) { g_gemm_ws = mode == 1 ? 1 : 0; }
+
+extern "C" size_t cf_gemm_plan(cf_gemm_args_t* a) {
+    a->plan = -1;
+    a->ksplit = 1;
+    if (!gemm_args_ok(a)) return 0;
+    const WsChoice c = ws_pick(a, gemm_tiling(a));
+    if (c.i < 0) return 0;
+    a->plan = c.i + 1;
+    a->ksplit = c.ks;
+    size_t ntot = 0;
+    for (int s = 0; s < a->nseg; s++) ntot += (size_t)a->n[s];
+    return c.ks > 1 ? (size_t)c.ks * (size_t)a->M * ntot : 0;
+}
+
+extern "C" void cf_gemm_set_ws_ksplit(int32_t ks) { g_gemm_ws_ks = ks > 0 && ks <= kWsMaxSplit ? ks : 0; }
+
+extern "C" void cf_gemm_set_ws_shape(int32_t bm, int32_t bn) {
+    g_gemm_ws_bm = bm > 0 ? bm : 0;
+    g_gemm_ws_bn = bn > 0 ? bn : 0;
+}
+
+int g_gemm_group_m = 0;  // tuning override of the tile-order group height (0 = kGroupM)
+
+extern "C" void cf_gemm_set_group_m(int32_t group_m) { g_gemm_group_m = group_m > 0 ? group_m : 0; }
+
+extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
+    if (!gemm_args_ok(a)) return (int)hipErrorInvalidValue;
+    Tiling t = gemm_tiling(a);
     t.group_m = g_gemm_group_m > 0 ? g_gemm_group_m : kGroupM;
-    if (a->out_kind == CF_GEMM_OUT_ROWCAT && !ws_pick(a, t)) return (int)hipErrorInvalidValue;
-    // The wave-specialised kernel where it applies (its tile chosen by the cost model).
-    if (const WsCandidate* c = ws_pick(a, t)) {
-        long long ntot = 0;
+    // The wave-specialised kernel where it applies (tile and k ranges by the cost model).
+    const WsChoice ws = a->plan == 0 ? ws_pick(a, t) : WsChoice{a->plan - 1, a->ksplit};
+    if ((a->out_kind == CF_GEMM_OUT_ROWCAT || a->w_nk) && ws.i < 0) return (int)hipErrorInvalidValue;
+    if (ws.i >= 0) {
+        const WsCandidate* c = &kWsShapes[ws.i];
+        int ntot = 0;
         for (int s = 0; s < a->nseg; s++) ntot += a->n[s];
+        cf_gemm_args_t args = *a;
+        args.ksplit = a->partials ? ws.ks : 1;
         const long long tiles_n = (ntot + c->bn - 1) / c->bn;
         t.n_tiles_m = (a->M + c->bm - 1) / c->bm;
         const long long blocks = (long long)t.n_tiles_m * tiles_n;
         if (blocks <= 0 || blocks > 0x7fffffffLL) return (int)hipErrorInvalidValue;
         set_order(t, (int)tiles_n);
-        const hipError_t e = c->launch(dim3((unsigned)blocks), (hipStream_t)stream, *a, t);
-        if (e != hipSuccess) return (int)e;
+        hipError_t e = c->launch(dim3((unsigned)blocks, (unsigned)args.ksplit), (hipStream_t)stream, args, t);
+        if (e == hipSuccess) e = hipGetLastError();
+        if (e != hipSuccess || args.ksplit == 1) return (int)e;
+        const dim3 g((unsigned)(((long long)a->M * (ntot / 4) + 63) / 64));
+        const FastDiv dr = fastdiv_make(ntot / 4);
+        hipStream_t st = (hipStream_t)stream;
+        if (args.ksplit <= 2) hipLaunchKernelGGL(gemm_splitk_sum<2>, g, dim3(64), 0, st, args, ntot, dr);
+        else if (args.ksplit <= 4) hipLaunchKernelGGL(gemm_splitk_sum<4>, g, dim3(64), 0, st, args, ntot, dr);
+        else if (args.ksplit <= 8) hipLaunchKernelGGL(gemm_splitk_sum<8>, g, dim3(64), 0, st, args, ntot, dr);
+        else hipLaunchKernelGGL(gemm_splitk_sum<kWsMaxSplit>, g, dim3(64), 0, st, args, ntot, dr);
         return (int)hipGetLastError();
     }
     // Full tiles with aligned rows take the pipelined direct-to-LDS kernel.  Its tile is

@@ -171,8 +171,8 @@ int32_t cf_gemv_fuses_rope(const cf_gemv_args_t* a);
  *                          M = B*S rows, W given as three segments.
  *   CF_GEMM_OUT_ROWCAT:   the nseg segments side by side in one row-major (M, sum n[s])
  *                          out[0], each with its own bias, no residual; fp16 on the
- *                          wave-specialised kernel only (cf_gemm_rowcat_ok says whether a
- *                          product can take it; cf_launch_gemm rejects it otherwise).
+ *                          wave-specialised kernel only (cf_gemm_plan gives plan > 0 for a
+ *                          product that can take it; cf_launch_gemm rejects it otherwise).
  * ------------------------------------------------------------------------------- */
 enum { CF_GEMM_OUT_ROWMAJOR = 0, CF_GEMM_OUT_QKV = 1, CF_GEMM_OUT_ROWCAT = 2 };
 
@@ -188,9 +188,20 @@ typedef struct {
     const void* residual;    /* row-major only, may be NULL */
     int32_t     B, S, H_q, H_kv, d;  /* QKV layout */
     int32_t     elem;        /* element type of a, w, bias, out, residual */
+    int32_t     w_nk;        /* 1: w[0] is (N, K) row-major (one segment; wave-specialised
+                                kernel only) */
+    int32_t     plan;        /* set by cf_gemm_plan: the wave-specialised kernel's tile
+                                (> 0) or another kernel (-1); 0 = the launch chooses */
+    int32_t     ksplit;      /* set by cf_gemm_plan: ranges of k with partial sums */
+    float*      partials;    /* workspace for those sums, or NULL (the launch then does not
+                                split k across workgroups) */
 } cf_gemm_args_t;
 
 int cf_launch_gemm(const cf_gemm_args_t* a, void* stream);
+/* Chooses the kernel (plan, ksplit) from the sizes and the pointers' alignment, and
+ * returns the floats of workspace for the sums over ranges of k (0 = none).  The pointers
+ * may be stand-ins of the same alignment. */
+size_t  cf_gemm_plan(cf_gemm_args_t* a);
 /* Tuning override of the fp16 direct-to-LDS GEMM's ring depth (3 or 4 stages; 0 =
  * automatic: 3, i.e. three workgroups per CU, when there are more than two tiles per CU). */
 void cf_gemm_set_stages(int32_t stages);
@@ -212,7 +223,8 @@ void cf_gemm_set_ws(int32_t mode);
 /* Tuning/test override of that kernel's tile (BM 256 or 128, BN among its widths; 0, 0 =
  * the cost model's choice).  A product the tile does not fit takes the cost model's. */
 void cf_gemm_set_ws_shape(int32_t bm, int32_t bn);
-int32_t cf_gemm_rowcat_ok(const cf_gemm_args_t* a);
+/* Test override of its split of k across workgroups (1..16; 0 = the cost model's). */
+void cf_gemm_set_ws_ksplit(int32_t ks);
 
 /* ---------------------------------------------------------------------------------
  * Prefill attention (flash style, online softmax): q (B, H_q, S, d), k (B, H_kv, S, d),

@@ -77,41 +77,64 @@ static int matmul_op(int elem, const void* inputs[], void* outputs[], const oper
     int64_t sa = batch > 1 ? p->stride_a : 0, sb = batch > 1 ? p->stride_b : 0;
     const int64_t sc = batch > 1 ? p->stride_c : 0;
 
-    /* Transposed operands are first made row-major in the workspace
+    cf_gemm_args_t g;
+    memset(&g, 0, sizeof(g));
+    g.M = (int32_t)M;
+    g.K = (int32_t)K;
+    g.nseg = 1;
+    g.bias[0] = inputs[2];
+    g.n[0] = (int32_t)N;
+    g.out_kind = CF_GEMM_OUT_ROWMAJOR;
+    g.elem = elem;
+
+    /* One plan for every slice: they differ in their pointers only, by strides that keep
+     * the alignment (else each launch chooses for itself, without k ranges).  B given as
+     * (N, K) goes to the GEMM as it is where that plan can take it; other transposed
+     * operands are first made row-major in the workspace, 256-byte aligned
      * (matmul_cuda.cu:320-352 transposes into per-call allocations). */
-    if (p->transpose_a || p->transpose_b) {
-        size_t cur = 0;
-        const size_t off_a = p->transpose_a ? cf_ws_take(&cur, (size_t)batch * M * K * esz) : 0;
-        const size_t off_b = p->transpose_b ? cf_ws_take(&cur, (size_t)batch * K * N * esz) : 0;
-        char* ws = (char*)gpu_workspace_get_stream(st, cur);
-        if (!ws) return -1;
-        int rc;
-        if (p->transpose_a) {
-            if ((rc = cf_launch_transpose(A, ws + off_a, K, M, batch, sa, M * K, (int32_t)esz, st)) != 0) return rc;
-            A = ws + off_a;
-            sa = M * K;
-        }
-        if (p->transpose_b) {
-            if ((rc = cf_launch_transpose(B, ws + off_b, N, K, batch, sb, K * N, (int32_t)esz, st)) != 0) return rc;
-            B = ws + off_b;
-            sb = K * N;
+    const int ta = p->transpose_a;
+    const int one_plan = batch == 1 || ((uint64_t)((ta ? M * K : sa) * esz) % 16 == 0 &&
+                                        (uint64_t)(sb * esz) % 16 == 0 && (uint64_t)(sc * esz) % 16 == 0);
+    const void* const stand_in = (const void*)(uintptr_t)256;
+    int flip_b = p->transpose_b;
+    size_t part = 0;                 /* partial sums, shared by the slices (one after another) */
+    if (one_plan) {
+        g.a = ta ? stand_in : A;
+        g.w[0] = B;
+        g.out[0] = outputs[0];
+        g.w_nk = flip_b;
+        part = cf_gemm_plan(&g);
+        if (flip_b && g.plan < 0) {
+            g.w_nk = 0;
+            g.plan = 0;
+            g.ksplit = 1;
+        } else {
+            flip_b = 0;
         }
     }
+    size_t cur = 0;
+    const size_t off_a = ta ? cf_ws_take(&cur, (size_t)batch * M * K * esz) : 0;
+    const size_t off_b = flip_b ? cf_ws_take(&cur, (size_t)batch * K * N * esz) : 0;
+    const size_t off_p = cf_ws_take(&cur, part * sizeof(float));
+    char* ws = NULL;
+    if (cur > 0 && !(ws = (char*)gpu_workspace_get_stream(st, cur))) return -1;
+    if (part > 0) g.partials = (float*)(ws + off_p);
+    int rc;
+    if (ta) {
+        if ((rc = cf_launch_transpose(A, ws + off_a, K, M, batch, sa, M * K, (int32_t)esz, st)) != 0) return rc;
+        A = ws + off_a;
+        sa = M * K;
+    }
+    if (flip_b) {
+        if ((rc = cf_launch_transpose(B, ws + off_b, N, K, batch, sb, K * N, (int32_t)esz, st)) != 0) return rc;
+        B = ws + off_b;
+        sb = K * N;
+    }
     for (int64_t bi = 0; bi < batch; bi++) {
-        cf_gemm_args_t g;
-        memset(&g, 0, sizeof(g));
         g.a = A + (size_t)(bi * sa) * esz;
-        g.M = (int32_t)M;
-        g.K = (int32_t)K;
-        g.nseg = 1;
         g.w[0] = B + (size_t)(bi * sb) * esz;
-        g.bias[0] = inputs[2];
-        g.n[0] = (int32_t)N;
-        g.out_kind = CF_GEMM_OUT_ROWMAJOR;
         g.out[0] = (char*)outputs[0] + (size_t)(bi * sc) * esz;
-        g.elem = elem;
-        const int rc = cf_launch_gemm(&g, st);
-        if (rc != 0) return rc;
+        if ((rc = cf_launch_gemm(&g, st)) != 0) return rc;
     }
     return 0;
 }

@@ -56,8 +56,26 @@ static void fused_carve(const fused_shape_t* sh, size_t esz, size_t* cur, size_t
     off[3] = cf_ws_take(cur, (size_t)(sh->B * sh->S * sh->D) * esz);
 }
 
-static void fused_fill(int elem, const void* inputs[], void* outputs[], const operator_params_t* params,
-                       const fused_shape_t* sh, char* data, const size_t off[4], fused_plan_t* pl);
+/* Returns the bytes of the two products' partial sums (shared: they run one after the
+ * other). */
+static size_t fused_fill(int elem, const void* inputs[], void* outputs[], const operator_params_t* params,
+                         const fused_shape_t* sh, const size_t off[4], fused_plan_t* pl);
+
+/* The plan is made before the workspace is known, with its areas at stand-in addresses
+ * from FUSED_BASE on (256-byte aligned, as the workspace is): only sizes and alignment
+ * decide.  fused_rebase then moves those addresses to the workspace. */
+#define FUSED_BASE ((char*)(uintptr_t)256)
+
+static void rebase(const void** p, char* data) { if (*p) *p = data + ((uintptr_t)*p - (uintptr_t)FUSED_BASE); }
+
+static void fused_rebase(fused_plan_t* pl, char* data) {
+    for (int i = 0; i < 3; i++) rebase((const void**)&pl->qkv.out[i], data);
+    rebase(&pl->attn.q, data);
+    rebase(&pl->attn.k, data);
+    rebase(&pl->attn.vt, data);
+    rebase((const void**)&pl->attn.o, data);
+    rebase(&pl->wo.a, data);
+}
 
 static int fused_plan(int elem, const void* inputs[], void* outputs[], const operator_params_t* params,
                       void* st, fused_plan_t* pl) {
@@ -67,14 +85,18 @@ static int fused_plan(int elem, const void* inputs[], void* outputs[], const ope
     if (fused_shape(params, &sh) != 0) return -1;
     size_t cur = 0, off[4];
     fused_carve(&sh, elem == CF_ELEM_F16 ? 2 : 4, &cur, off);
+    const size_t part = fused_fill(elem, inputs, outputs, params, &sh, off, pl);
+    const size_t off_p = cf_ws_take(&cur, part);
     char* data = (char*)gpu_workspace_get_stream(st, cur);
     if (!data) return -1;
-    fused_fill(elem, inputs, outputs, params, &sh, data, off, pl);
+    fused_rebase(pl, data);
+    if (part > 0) pl->qkv.partials = pl->wo.partials = (float*)(data + off_p);
     return 0;
 }
 
-static void fused_fill(int elem, const void* inputs[], void* outputs[], const operator_params_t* params,
-                       const fused_shape_t* sh, char* data, const size_t off[4], fused_plan_t* pl) {
+static size_t fused_fill(int elem, const void* inputs[], void* outputs[], const operator_params_t* params,
+                         const fused_shape_t* sh, const size_t off[4], fused_plan_t* pl) {
+    char* const data = FUSED_BASE;
     const mha_fused_params_t* p = (const mha_fused_params_t*)params;
     const int64_t B = sh->B, S = sh->S, D = sh->D, H = sh->H, d = sh->d, H_kv = sh->H_kv, kvd = sh->kvd;
     const size_t off_q = off[0], off_k = off[1], off_v = off[2], off_o = off[3];
@@ -108,6 +130,7 @@ static void fused_fill(int elem, const void* inputs[], void* outputs[], const op
     /* The row-concatenated layout: one (B*S, (H + 2 H_kv) d) matrix from the start of the
      * q area; the q, k and v areas follow one another (each start rounded up to 256 bytes),
      * so together they hold its B*S*(D + 2 kvd) elements. */
+    size_t part_q = 0;
     if (g_rowcat && elem == CF_ELEM_F16) {
         cf_gemm_args_t rc = *g;
         rc.out_kind = CF_GEMM_OUT_ROWCAT;
@@ -117,11 +140,15 @@ static void fused_fill(int elem, const void* inputs[], void* outputs[], const op
         fr.q = data + off_q;
         fr.k = fr.vt = NULL;
         fr.qkv_ld = (int32_t)(D + 2 * kvd);
-        if (cf_gemm_rowcat_ok(&rc) && cf_flash_rowcat_ok(&fr)) {
-            *g = rc;
-            *f = fr;
+        if (cf_flash_rowcat_ok(&fr)) {
+            part_q = cf_gemm_plan(&rc);
+            if (rc.plan > 0) {
+                *g = rc;
+                *f = fr;
+            }
         }
     }
+    if (g->plan == 0) part_q = cf_gemm_plan(g);
 
     cf_gemm_args_t* o = &pl->wo;
     o->a = data + off_o;
@@ -133,6 +160,8 @@ static void fused_fill(int elem, const void* inputs[], void* outputs[], const op
     o->out[0] = outputs[0];
     o->residual = (p->has_residual && inputs[1]) ? inputs[1] : NULL;
     o->elem = elem;
+    const size_t part_o = cf_gemm_plan(o);
+    return (part_q > part_o ? part_q : part_o) * sizeof(float);
 }
 
 static int fused_launch(const fused_plan_t* pl, int which, void* st) {
@@ -211,18 +240,29 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
     off_y = cf_ws_take(&cur, (size_t)BSD * 2);
     fused_carve(&sh, 2, &cur, off);
     void* st = cf_stream_of(stream);
+    /* The fp16 copies are 256-byte aligned whatever the caller's buffers are. */
+    const void* in16[10];
+    for (int i = 0; i < 10; i++) in16[i] = inputs[i] && n_in[i] ? FUSED_BASE + off_in[i] : NULL;
+    void* out16[1] = {FUSED_BASE + off_y};
+    fused_plan_t pl;
+    const size_t part = fused_fill(CF_ELEM_F16, in16, out16, params, &sh, off, &pl);
+    const size_t off_p = cf_ws_take(&cur, part);
     char* data = (char*)gpu_workspace_get_stream(st, cur);
     if (!data) return -1;
-    const void* in16[10];
-    for (int i = 0; i < 10; i++) {
-        in16[i] = NULL;
-        if (!inputs[i] || n_in[i] == 0) continue;
-        if (cf_launch_cast(inputs[i], data + off_in[i], n_in[i], CF_CAST_F32_F16, st) != 0) return -1;
-        in16[i] = data + off_in[i];
+    for (int i = 0; i < 10; i++)
+        if (in16[i] && cf_launch_cast(inputs[i], data + off_in[i], n_in[i], CF_CAST_F32_F16, st) != 0) return -1;
+    fused_rebase(&pl, data);
+    /* Here the operands, the residual and Y are in the workspace too. */
+    rebase(&pl.qkv.a, data);
+    for (int i = 0; i < 3; i++) {
+        rebase(&pl.qkv.w[i], data);
+        rebase(&pl.qkv.bias[i], data);
     }
-    void* out16[1] = {data + off_y};
-    fused_plan_t pl;
-    fused_fill(CF_ELEM_F16, in16, out16, params, &sh, data, off, &pl);
+    rebase(&pl.wo.w[0], data);
+    rebase(&pl.wo.bias[0], data);
+    rebase(&pl.wo.residual, data);
+    rebase((const void**)&pl.wo.out[0], data);
+    if (part > 0) pl.qkv.partials = pl.wo.partials = (float*)(data + off_p);
     for (int k = 0; k < 3; k++)
         if (fused_launch(&pl, k, st) != 0) return -1;
     return cf_launch_cast(data + off_y, outputs[0], BSD, CF_CAST_F16_F32, st);

@@ -193,6 +193,36 @@ def test_matmul_f16_tile_ends(gpu, native, bm, bn, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("M,N,K,bm,bn,ks", [
+    (1, 72, 1024, 64, 64, 8), (16, 200, 1088, 64, 128, 3), (65, 64, 640, 64, 64, 5), (130, 328, 512, 128, 96, 2),
+    (17, 136, 4096, 64, 64, 16), (300, 264, 192, 256, 64, 1), (130, 72, 192, 64, 128, 1)])
+def test_matmul_f16_k_ranges(gpu, native, nk, M, N, K, bm, bn, ks):
+    """Split sums over ranges of k (uneven last ranges, cut row and column tiles) and W
+    given as (N, K), forced tile by tile, against float64 and, without a forced tile, for
+    the cost model's choice; nothing written past the result."""
+    import cudaforge_amd as cf
+    A = O.round_f16(O.normal((M, K), M + N))
+    B = O.round_f16(O.normal((K, N), K + 1, 0.0, 1.0 / np.sqrt(K)))
+    bias = O.round_f16(O.normal((N,), 5, 0.0, 0.1))
+    want = A.astype(np.float64) @ B.astype(np.float64) + bias
+    p = cf.MatmulParams(M, N, K, False, nk, 1, 0, 0, 0, 0)
+    for force in (True, False):
+        C = cf.DeviceBuffer.from_numpy(np.full(M * N + 1024, 7.0, np.float16))
+        try:
+            if force:
+                native.cf_gemm_set_ws_shape(bm, bn)
+                native.cf_gemm_set_ws_ksplit(ks)
+            assert cf.call_op("matmul_f16_cuda", [dev(A, True), dev(B.T if nk else B, True), dev(bias, True)], [C], p) == 0
+            got = C.download().astype(np.float32)
+        finally:
+            native.cf_gemm_set_ws_shape(0, 0)
+            native.cf_gemm_set_ws_ksplit(0)
+        assert max_abs(want, got[:M * N].reshape(M, N)) <= 4e-3      # one fp16 rounding of values below 8
+        assert np.all(got[M * N:] == 7.0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])
 def test_matmul_cuda_transposed_batched(gpu, f16, ta, tb):
