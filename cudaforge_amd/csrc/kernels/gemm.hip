@@ -830,7 +830,7 @@ struct WsEpi {
     const CF_GLOBAL _Float16* bias1;
     const CF_GLOBAL _Float16* bias2;
     const CF_GLOBAL _Float16* res;
-    int S, Hq, Hkv, d, n0w;
+    int S, Hq, Hkv, d, n0w, f32;
     // Per-segment pointers as the first one plus a selected distance: a select among the
     // pointers themselves is turned into an indexed load of the struct, which then lives
     // in scratch memory.
@@ -857,11 +857,12 @@ __device__ __forceinline__ WsEpi ws_epi(const cf_gemm_args_t& a) {
     e.Hq = a.H_q;
     e.Hkv = a.H_kv;
     e.d = a.d;
+    e.f32 = a.out_f32;
     e.n0w = a.out_kind == CF_GEMM_OUT_ROWCAT ? a.n[0] + a.n[1] + a.n[2] : a.n[0];
     // Empty asm that "modifies" every field: the loads happen here, not where first used.
     asm volatile("" : "+s"(e.out0), "+s"(e.out1), "+s"(e.out2), "+s"(e.bias0), "+s"(e.bias1), "+s"(e.bias2),
                  "+s"(e.res));
-    asm volatile("" : "+s"(e.S), "+s"(e.Hq), "+s"(e.Hkv), "+s"(e.d), "+s"(e.n0w));
+    asm volatile("" : "+s"(e.S), "+s"(e.Hq), "+s"(e.Hkv), "+s"(e.d), "+s"(e.n0w), "+s"(e.f32));
     return e;
 }
 #pragma clang diagnostic pop
@@ -1196,6 +1197,17 @@ void gemm_f16_ws(cf_gemm_args_t a, Tiling t) {
     ws_store<BM, BN, EPI>(epi, start, a.nseg, m0, n0, min(BM, a.M - m0), min(BN, ntot - n0), tid, smem, vt_tile);
 }
 
+// Eight consecutive row-major results, as fp16 or widened to fp32 (out_f32).
+__device__ __forceinline__ void ws_put8(const WsEpi& e, size_t off, h8_t v) {
+    if (e.f32) {
+        CF_GLOBAL float* const o = (CF_GLOBAL float*)e.out0 + off;
+        *(CF_GLOBAL f4_t*)o = f4_t{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+        *(CF_GLOBAL f4_t*)(o + 4) = f4_t{(float)v[4], (float)v[5], (float)v[6], (float)v[7]};
+    } else {
+        *(CF_GLOBAL h8_t*)(e.out0 + off) = v;
+    }
+}
+
 // Store phase of gemm_f16_ws (all 512 threads): the staged tile goes out as 16-byte chunks,
 // 8 columns of one row (row-major C, head-major q and k; consecutive threads along the
 // row) or, for v^T columns, 8 rows of one column read down the staged column.  Each pass
@@ -1206,9 +1218,9 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
     constexpr int CPR = BN / 8, NCH = BM * CPR, IT = (NCH + 511) / 512;
     constexpr bool qkv = EPI == WS_EPI_QKV;
     const WsRows wr = ws_rows(e, m0);
-    // Whole tiles skip the end-of-matrix tests (with them, BERT-base's output
+    // Whole tiles of fp16 results skip the end-of-matrix tests (with them, BERT-base's output
     // projection measured 9.0 us, without 8.45).
-    const bool whole = rows == BM && cols == BN;
+    const bool whole = rows == BM && cols == BN && !e.f32;
     if constexpr (EPI == WS_EPI_ROWMAJOR) {
         // Row-major C: consecutive threads along a row.
         if (whole) {
@@ -1227,7 +1239,7 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
             const int id = tid + 512 * it;
             const int r = id / CPR, c8 = id - r * CPR;
             if (r < rows && 8 * c8 < cols)         // rows <= BM: also the end of the tile
-                *(CF_GLOBAL h8_t*)(e.out0 + (size_t)(m0 + r) * e.n0w + n0 + 8 * c8) = *(const h8_t*)(smem + r * (BN + 8) + 8 * c8);
+                ws_put8(e, (size_t)(m0 + r) * e.n0w + n0 + 8 * c8, *(const h8_t*)(smem + r * (BN + 8) + 8 * c8));
         }
         return;
     }
@@ -1272,7 +1284,8 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
                 h8_t v;
 #pragma unroll
                 for (int k = 0; k < 8; k++) v[k] = (_Float16)(f[k] + (float)rv[it][k]);
-                *(CF_GLOBAL h8_t*)(e.out0 + off[it]) = v;
+                if constexpr (W) *(CF_GLOBAL h8_t*)(e.out0 + off[it]) = v;
+                else ws_put8(e, off[it], v);
             }
         };
         if (whole) add_and_store(std::true_type{});
@@ -1344,7 +1357,8 @@ void gemm_splitk_sum(cf_gemm_args_t a, int ntot, FastDiv div_row) {
     h4_t o;
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = (_Float16)(s[e] + (float)b[e] + (float)r[e]);
-    *(h4_t*)((_Float16*)a.out[0] + (size_t)m * ntot + n) = o;
+    if (a.out_f32) *(f4_t*)((float*)a.out[0] + (size_t)m * ntot + n) = __builtin_convertvector(o, f4_t);
+    else *(h4_t*)((_Float16*)a.out[0] + (size_t)m * ntot + n) = o;
 }
 
 // Cost model of the wave-specialised kernel, in CU clocks, fitted to a sweep of every tile
@@ -1605,6 +1619,7 @@ extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
     // The wave-specialised kernel where it applies (tile and k ranges by the cost model).
     const WsChoice ws = a->plan == 0 ? ws_pick(a, t) : WsChoice{a->plan - 1, a->ksplit};
     if ((a->out_kind == CF_GEMM_OUT_ROWCAT || a->w_nk) && ws.i < 0) return (int)hipErrorInvalidValue;
+    if (a->out_f32 && (ws.i < 0 || a->out_kind != CF_GEMM_OUT_ROWMAJOR)) return (int)hipErrorInvalidValue;
     if (ws.i >= 0) {
         const WsCandidate* c = &kWsShapes[ws.i];
         int ntot = 0;

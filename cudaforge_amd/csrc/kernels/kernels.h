@@ -190,6 +190,8 @@ typedef struct {
     int32_t     elem;        /* element type of a, w, bias, out, residual */
     int32_t     w_nk;        /* 1: w[0] is (N, K) row-major (one segment; wave-specialised
                                 kernel only) */
+    int32_t     out_f32;     /* 1: out[0] takes the fp16 results widened to fp32 (row-major,
+                                wave-specialised kernel only) */
     int32_t     plan;        /* set by cf_gemm_plan: the wave-specialised kernel's tile
                                 (> 0) or another kernel (-1); 0 = the launch chooses */
     int32_t     ksplit;      /* set by cf_gemm_plan: ranges of k with partial sums */
@@ -293,6 +295,16 @@ int cf_launch_layernorm(const cf_layernorm_args_t* a, void* stream);
  * f32 -> f16 rounds to nearest even, f32 -> i64 truncates toward zero. */
 enum { CF_CAST_I64_F32 = 0, CF_CAST_F32_I64 = 1, CF_CAST_F32_F16 = 2, CF_CAST_F16_F32 = 3 };
 int cf_launch_cast(const void* in, void* out, int64_t n, int32_t kind, void* stream);
+
+/* Up to CF_CAST_MANY arrays f32 -> f16 (nearest even) in one launch; entries with n = 0 are
+ * skipped.  16-byte aligned arrays are read and written 16 bytes at a time. */
+#define CF_CAST_MANY 10
+typedef struct {
+    const void* in[CF_CAST_MANY];
+    void*       out[CF_CAST_MANY];
+    int64_t     n[CF_CAST_MANY];
+} cf_cast_many_args_t;
+int cf_launch_cast_many(const cf_cast_many_args_t* a, void* stream);
 
 /* out (cols, rows) = in (rows, cols)^T for `batch` slices (strides in elements);
  * elem_bytes 2 or 4. */

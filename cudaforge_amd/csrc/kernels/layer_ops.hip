@@ -124,7 +124,40 @@ hipError_t launch_layernorm(const cf_layernorm_args_t& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Cast: grid-stride elementwise.
+// Cast: grid-stride elementwise.  Between f32 and f16, eight elements per thread with
+// 16-byte accesses where both ends are aligned (`vec`; the last n % 8 one by one).
+template <typename I, typename O>
+__device__ __forceinline__ void cast8(const I* __restrict__ in, O* __restrict__ out, int64_t i, int64_t n, bool vec) {
+    typedef I i8_t __attribute__((ext_vector_type(8)));
+    typedef O o8_t __attribute__((ext_vector_type(8)));
+    if (vec && i + 8 <= n) {
+        *(o8_t*)(out + i) = __builtin_convertvector(*(const i8_t*)(in + i), o8_t);
+    } else {
+        for (int64_t j = i; j < i + 8 && j < n; j++) out[j] = (O)in[j];
+    }
+}
+template <typename I, typename O>
+__global__ __launch_bounds__(256) void cast8_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n, bool vec) {
+    for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (int64_t)gridDim.x * 2048)
+        cast8(in, out, i, n, vec);
+}
+
+// Several f32 -> f16 arrays in one launch (the mixed-precision prefill's ten operands, whose
+// ten launches of 1.5-3.2 us took longer than its products): entry e owns workgroups
+// first[e] .. first[e+1] - 1 of 2048 elements each.
+struct CastMany {
+    cf_cast_many_args_t a;
+    unsigned first[CF_CAST_MANY + 1];
+    unsigned vec;                      // bit e: entry e's ends are aligned
+};
+__global__ __launch_bounds__(256) void cast_many_kernel(CastMany c) {
+    int e = 0;
+#pragma unroll
+    for (int k = 1; k < CF_CAST_MANY; k++) e += blockIdx.x >= c.first[k] ? 1 : 0;
+    const int64_t i = ((int64_t)(blockIdx.x - c.first[e]) * 256 + threadIdx.x) * 8;
+    if (i < c.a.n[e]) cast8((const float*)c.a.in[e], (_Float16*)c.a.out[e], i, c.a.n[e], (c.vec >> e) & 1u);
+}
+
 template <typename I, typename O>
 __global__ __launch_bounds__(256) void cast_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
@@ -168,14 +201,33 @@ extern "C" int cf_launch_cast(const void* in, void* out, int64_t n, int32_t kind
     if (!in || !out || n < 0) return (int)hipErrorInvalidValue;
     if (n == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 g(grid_1d(n)), b(256);
+    const dim3 g(grid_1d(n)), g8(grid_1d((n + 7) / 8)), b(256);
+    const bool vec = ((uintptr_t)in | (uintptr_t)out) % 16 == 0;
     switch (kind) {
         case CF_CAST_I64_F32: hipLaunchKernelGGL((cast_kernel<int64_t, float>), g, b, 0, s, (const int64_t*)in, (float*)out, n); break;
         case CF_CAST_F32_I64: hipLaunchKernelGGL((cast_kernel<float, int64_t>), g, b, 0, s, (const float*)in, (int64_t*)out, n); break;
-        case CF_CAST_F32_F16: hipLaunchKernelGGL((cast_kernel<float, _Float16>), g, b, 0, s, (const float*)in, (_Float16*)out, n); break;
-        case CF_CAST_F16_F32: hipLaunchKernelGGL((cast_kernel<_Float16, float>), g, b, 0, s, (const _Float16*)in, (float*)out, n); break;
+        case CF_CAST_F32_F16: hipLaunchKernelGGL((cast8_kernel<float, _Float16>), g8, b, 0, s, (const float*)in, (_Float16*)out, n, vec); break;
+        case CF_CAST_F16_F32: hipLaunchKernelGGL((cast8_kernel<_Float16, float>), g8, b, 0, s, (const _Float16*)in, (float*)out, n, vec); break;
         default: return (int)hipErrorInvalidValue;
     }
+    return (int)hipGetLastError();
+}
+
+extern "C" int cf_launch_cast_many(const cf_cast_many_args_t* a, void* stream) {
+    CastMany c;
+    c.a = *a;
+    c.vec = 0;
+    unsigned long long at = 0;
+    for (int e = 0; e < CF_CAST_MANY; e++) {
+        c.first[e] = (unsigned)at;
+        if (a->n[e] < 0 || (a->n[e] > 0 && (!a->in[e] || !a->out[e]))) return (int)hipErrorInvalidValue;
+        if (((uintptr_t)a->in[e] | (uintptr_t)a->out[e]) % 16 == 0) c.vec |= 1u << e;
+        at += ((unsigned long long)a->n[e] + 2047) / 2048;
+        if (at > 0x7fffffffULL) return (int)hipErrorInvalidValue;
+    }
+    c.first[CF_CAST_MANY] = (unsigned)at;
+    if (at == 0) return 0;
+    hipLaunchKernelGGL(cast_many_kernel, dim3((unsigned)at), dim3(256), 0, (hipStream_t)stream, c);
     return (int)hipGetLastError();
 }
 

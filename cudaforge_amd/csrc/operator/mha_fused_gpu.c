@@ -249,8 +249,13 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
     const size_t off_p = cf_ws_take(&cur, part);
     char* data = (char*)gpu_workspace_get_stream(st, cur);
     if (!data) return -1;
-    for (int i = 0; i < 10; i++)
-        if (in16[i] && cf_launch_cast(inputs[i], data + off_in[i], n_in[i], CF_CAST_F32_F16, st) != 0) return -1;
+    cf_cast_many_args_t c;
+    for (int i = 0; i < 10; i++) {
+        c.in[i] = inputs[i];
+        c.out[i] = data + off_in[i];
+        c.n[i] = in16[i] ? n_in[i] : 0;
+    }
+    if (cf_launch_cast_many(&c, st) != 0) return -1;
     fused_rebase(&pl, data);
     /* Here the operands, the residual and Y are in the workspace too. */
     rebase(&pl.qkv.a, data);
@@ -263,9 +268,15 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
     rebase(&pl.wo.residual, data);
     rebase((const void**)&pl.wo.out[0], data);
     if (part > 0) pl.qkv.partials = pl.wo.partials = (float*)(data + off_p);
+    /* The output product widens Y as it stores it, where its kernel can (aligned Y). */
+    const int wide = pl.wo.plan > 0 && (uintptr_t)outputs[0] % 16 == 0;
+    if (wide) {
+        pl.wo.out[0] = outputs[0];
+        pl.wo.out_f32 = 1;
+    }
     for (int k = 0; k < 3; k++)
         if (fused_launch(&pl, k, st) != 0) return -1;
-    return cf_launch_cast(data + off_y, outputs[0], BSD, CF_CAST_F16_F32, st);
+    return wide ? 0 : cf_launch_cast(data + off_y, outputs[0], BSD, CF_CAST_F16_F32, st);
 }
 
 int causal_mask_f32_cuda(const void* inputs[], void* outputs[],

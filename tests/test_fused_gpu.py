@@ -81,6 +81,26 @@ def test_fused_f16_entry_takes_float_buffers(gpu, B, S, H, H_kv, d, causal, resi
     assert max_abs(c16.oracle(), got) <= TOL16
 
 
+@pytest.mark.parametrize("B,S,H,H_kv,d,skew_in,skew_out", [
+    (1, 8, 12, 12, 64, 0, 0), (1, 8, 12, 12, 64, 4, 0), (3, 37, 4, 2, 128, 0, 4), (1, 5, 3, 3, 17, 8, 8)])
+def test_fused_f16_entry_small_and_misaligned(gpu, B, S, H, H_kv, d, skew_in, skew_out):
+    """mha_fused_f16_cuda on a few tokens, its float buffers at any 4-byte address and with
+    lengths that are no multiple of 8: the casts' element-wise ends and Y stored by the
+    output product or, where it cannot, widened afterwards."""
+    import cudaforge_amd as cf
+    c32 = FusedCase(B, S, H, H_kv, d, seed=40 + S, f16=False, residual=True, bias_std=0.02)
+    c16 = FusedCase(B, S, H, H_kv, d, seed=40 + S, f16=True, residual=True, bias_std=0.02)
+    k = skew_in // 4
+    bufs = [dev(np.concatenate([np.zeros(k, np.float32), a.ravel()])) for a in c32.arrays()]
+    Y = cf.DeviceBuffer.from_numpy(np.full(B * S * H * d + 64, 7.0, np.float32))
+    assert cf.call_op("mha_fused_f16_cuda", [b.ptr + skew_in for b in bufs], [Y.ptr + skew_out],
+                      c32.params(cf.MhaFusedParams)) == 0
+    got = Y.download()
+    n = skew_out // 4
+    assert np.array_equal(got[n:n + B * S * H * d].reshape(B, S, H * d), run_fused_gpu(c16))
+    assert np.all(got[:n] == 7.0) and np.all(got[n + B * S * H * d:] == 7.0)
+
+
 def test_config3_bert_base_full_size(gpu):
     """B=8, S=512, D=768, 12x64, fp16, no mask.  Every row of the
     full-size run against a float64 evaluation of the same math, and batch rows 0 and 7
