@@ -20,7 +20,8 @@
 //       one pass without a residual, fp32 in two with one) so stores are 16 bytes along
 //       the destination's contiguous direction.
 // fp32: 128x128x16 tile with v_mfma_f32_16x16x4_f32, both tiles staged k-major so each
-//       operand is one conflict-free ds_read_b32 (the FP32 operator's parity path).
+//       operand is one conflict-free ds_read_b32: the shapes that gemm_x3 and gemm_f32_ws
+//       do not take (K % 32, widths or addresses off their alignment).
 // Tile edges are zero-filled on load and masked on store.
 
 #include <hip/hip_runtime.h>
@@ -32,6 +33,7 @@
 
 #include "kernels.h"
 #include "cdna4.h"
+#include "gemm_x3.h"
 
 namespace {
 
@@ -1333,7 +1335,7 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
 // Sum of gemm_f16_ws's k ranges: KS >= a.ksplit partials of four columns of one row per
 // thread, all loaded before the first add (the range index clamped, the surplus left out),
 // plus bias and residual in fp32 and one rounding.
-template <int KS>
+template <typename T, int KS>
 __global__ __launch_bounds__(64)
 void gemm_splitk_sum(cf_gemm_args_t a, int ntot, FastDiv div_row) {
     const int id = blockIdx.x * 64 + threadIdx.x;          // four columns: M * ntot / 4 < 2^31
@@ -1346,19 +1348,20 @@ void gemm_splitk_sum(cf_gemm_args_t a, int ntot, FastDiv div_row) {
     for (int k = 0; k < KS; k++) v[k] = *(const f4_t*)(p + (size_t)min(k, a.ksplit - 1) * plane);
     const int n1 = a.n[0], n2 = n1 + (a.nseg > 1 ? a.n[1] : 0);
     const int seg = a.nseg > 2 && n >= n2 ? 2 : a.nseg > 1 && n >= n1 ? 1 : 0;
-    const _Float16* bias = (const _Float16*)(seg == 2 ? a.bias[2] : seg == 1 ? a.bias[1] : a.bias[0]);
+    typedef T v4_t __attribute__((ext_vector_type(4)));
+    const T* bias = (const T*)(seg == 2 ? a.bias[2] : seg == 1 ? a.bias[1] : a.bias[0]);
     const int col = n - (seg == 2 ? n2 : seg == 1 ? n1 : 0);
-    const h4_t b = bias ? *(const h4_t*)(bias + col) : h4_t{0, 0, 0, 0};
-    const h4_t r = a.residual ? *(const h4_t*)((const _Float16*)a.residual + (size_t)m * ntot + n) : h4_t{0, 0, 0, 0};
+    const v4_t b = bias ? *(const v4_t*)(bias + col) : v4_t{0, 0, 0, 0};
+    const v4_t r = a.residual ? *(const v4_t*)((const T*)a.residual + (size_t)m * ntot + n) : v4_t{0, 0, 0, 0};
     f4_t s = v[0];
 #pragma unroll
     for (int k = 1; k < KS; k++)
         if (k < a.ksplit) s += v[k];
-    h4_t o;
+    v4_t o;
 #pragma unroll
-    for (int e = 0; e < 4; e++) o[e] = (_Float16)(s[e] + (float)b[e] + (float)r[e]);
+    for (int e = 0; e < 4; e++) o[e] = (T)(s[e] + (float)b[e] + (float)r[e]);
     if (a.out_f32) *(f4_t*)((float*)a.out[0] + (size_t)m * ntot + n) = __builtin_convertvector(o, f4_t);
-    else *(h4_t*)((_Float16*)a.out[0] + (size_t)m * ntot + n) = o;
+    else *(v4_t*)((T*)a.out[0] + (size_t)m * ntot + n) = o;
 }
 
 // Cost model of the wave-specialised kernel, in CU clocks, fitted to a sweep of every tile
@@ -1588,10 +1591,48 @@ extern "C" void cf_gemm_set_bn(int32_t bn) { g_gemm_bn = bn == 96 || bn == 128 |
 
 extern "C" void cf_gemm_set_ws(int32_t mode) { g_gemm_ws = mode == 1 ? 1 : 0; }
 
+template <typename T>
+static void splitk_sum(const cf_gemm_args_t& a, int ntot, hipStream_t st) {
+    const dim3 g((unsigned)(((long long)a.M * (ntot / 4) + 63) / 64));
+    const FastDiv dr = fastdiv_make(ntot / 4);
+    if (a.ksplit <= 2) hipLaunchKernelGGL((gemm_splitk_sum<T, 2>), g, dim3(64), 0, st, a, ntot, dr);
+    else if (a.ksplit <= 4) hipLaunchKernelGGL((gemm_splitk_sum<T, 4>), g, dim3(64), 0, st, a, ntot, dr);
+    else if (a.ksplit <= 8) hipLaunchKernelGGL((gemm_splitk_sum<T, 8>), g, dim3(64), 0, st, a, ntot, dr);
+    else hipLaunchKernelGGL((gemm_splitk_sum<T, kWsMaxSplit>), g, dim3(64), 0, st, a, ntot, dr);
+}
+
+int gemm_splitk_sum_launch(const cf_gemm_args_t* a, hipStream_t st) {
+    int ntot = 0;
+    for (int s = 0; s < a->nseg; s++) ntot += a->n[s];
+    if (a->elem == CF_ELEM_F32) splitk_sum<float>(*a, ntot, st);
+    else splitk_sum<_Float16>(*a, ntot, st);
+    return (int)hipGetLastError();
+}
+
+constexpr int kPlanX3 = 1000, kPlanF32 = 2000;    // plans from here on: gemm_x3's, gemm_f32_ws's tiles
+
 extern "C" size_t cf_gemm_plan(cf_gemm_args_t* a) {
     a->plan = -1;
     a->ksplit = 1;
     if (!gemm_args_ok(a)) return 0;
+    if (a->elem == CF_ELEM_F32) {
+        // FP32: the bf16-MFMA product where the MFMA time it saves outweighs splitting the
+        // operands (16 bytes of memory traffic per element of W against 4), else the fp32
+        // MFMA one, by their cost models: 300 x 4096 x 1024 33 and 35 us, 256 x 4096 x 4096 75
+        // and 85, 320 x 768 x 3072 24 and 20, 16 x 4096 x 14336 183 and 36.
+        int ks_x3 = 1, ks_f = 1;
+        float clk_x3 = 0.0f, clk_f = 0.0f;
+        const int x3 = gemm_x3_pick(a, &ks_x3, &clk_x3), f = gemm_f32_ws_pick(a, &ks_f, &clk_f);
+        if (x3 >= 0 && (f < 0 || clk_x3 < clk_f)) {
+            a->plan = kPlanX3 + x3;
+            a->ksplit = ks_x3;
+            return gemm_x3_floats(a);
+        }
+        if (f < 0) return 0;
+        a->plan = kPlanF32 + f;
+        a->ksplit = ks_f;
+        return gemm_f32_ws_floats(a);
+    }
     const WsChoice c = ws_pick(a, gemm_tiling(a));
     if (c.i < 0) return 0;
     a->plan = c.i + 1;
@@ -1614,10 +1655,12 @@ extern "C" void cf_gemm_set_group_m(int32_t group_m) { g_gemm_group_m = group_m 
 
 extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
     if (!gemm_args_ok(a)) return (int)hipErrorInvalidValue;
+    if (a->plan >= kPlanF32) return gemm_f32_ws_launch(a, a->plan - kPlanF32, (hipStream_t)stream);
+    if (a->plan >= kPlanX3 && a->partials) return gemm_x3_launch(a, a->plan - kPlanX3, (hipStream_t)stream);
     Tiling t = gemm_tiling(a);
     t.group_m = g_gemm_group_m > 0 ? g_gemm_group_m : kGroupM;
     // The wave-specialised kernel where it applies (tile and k ranges by the cost model).
-    const WsChoice ws = a->plan == 0 ? ws_pick(a, t) : WsChoice{a->plan - 1, a->ksplit};
+    const WsChoice ws = a->plan == 0 || a->plan >= kPlanX3 ? ws_pick(a, t) : WsChoice{a->plan - 1, a->ksplit};
     if ((a->out_kind == CF_GEMM_OUT_ROWCAT || a->w_nk) && ws.i < 0) return (int)hipErrorInvalidValue;
     if (a->out_f32 && (ws.i < 0 || a->out_kind != CF_GEMM_OUT_ROWMAJOR)) return (int)hipErrorInvalidValue;
     if (ws.i >= 0) {
@@ -1634,14 +1677,7 @@ extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
         hipError_t e = c->launch(dim3((unsigned)blocks, (unsigned)args.ksplit), (hipStream_t)stream, args, t);
         if (e == hipSuccess) e = hipGetLastError();
         if (e != hipSuccess || args.ksplit == 1) return (int)e;
-        const dim3 g((unsigned)(((long long)a->M * (ntot / 4) + 63) / 64));
-        const FastDiv dr = fastdiv_make(ntot / 4);
-        hipStream_t st = (hipStream_t)stream;
-        if (args.ksplit <= 2) hipLaunchKernelGGL(gemm_splitk_sum<2>, g, dim3(64), 0, st, args, ntot, dr);
-        else if (args.ksplit <= 4) hipLaunchKernelGGL(gemm_splitk_sum<4>, g, dim3(64), 0, st, args, ntot, dr);
-        else if (args.ksplit <= 8) hipLaunchKernelGGL(gemm_splitk_sum<8>, g, dim3(64), 0, st, args, ntot, dr);
-        else hipLaunchKernelGGL(gemm_splitk_sum<kWsMaxSplit>, g, dim3(64), 0, st, args, ntot, dr);
-        return (int)hipGetLastError();
+        return gemm_splitk_sum_launch(&args, (hipStream_t)stream);
     }
     // Full tiles with aligned rows take the pipelined direct-to-LDS kernel.  Its tile is
     // 128 columns wide unless that leaves CUs idle and 96 columns fills more of them

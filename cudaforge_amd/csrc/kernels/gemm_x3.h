@@ -1,0 +1,23 @@
+// gemm_x3.h — the FP32 product on bf16 MFMA (gemm_x3.hip), chosen by cf_gemm_plan.
+#ifndef CF_GEMM_X3_H_
+#define CF_GEMM_X3_H_
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+#include "kernels.h"
+
+// The tile for this product (an index for gemm_x3_launch), or -1 where it does not apply.
+// *ks: the ranges of k its workgroups sum; *clk: its estimated time in CU clocks.
+int gemm_x3_pick(const cf_gemm_args_t* a, int* ks, float* clk);
+// Workspace floats (a->partials) of a launch with a->ksplit ranges.
+size_t gemm_x3_floats(const cf_gemm_args_t* a);
+int gemm_x3_launch(const cf_gemm_args_t* a, int pick, hipStream_t st);
+// FP32 products of few rows on the fp32 MFMA (gemm_f32_ws.hip), likewise.
+int gemm_f32_ws_pick(const cf_gemm_args_t* a, int* ks, float* clk);
+size_t gemm_f32_ws_floats(const cf_gemm_args_t* a);
+int gemm_f32_ws_launch(const cf_gemm_args_t* a, int pick, hipStream_t st);
+// Sums a->ksplit ranges of fp32 partial sums at a->partials into out[0] (gemm.hip).
+int gemm_splitk_sum_launch(const cf_gemm_args_t* a, hipStream_t st);
+
+#endif  // CF_GEMM_X3_H_

@@ -1,0 +1,378 @@
+// gemm_x3.hip — FP32 products on the bf16 matrix cores (gfx950).
+//
+// The fp32 MFMA runs at 1/16 of the bf16 one's rate (157 against 2500 TFLOP/s), so large
+// FP32 products are computed from an exact three-way split: x = h + m + l, each a bf16
+// holding 8 of x's 24 significant bits (h the top ones by truncation, m and l what is
+// left, every subtraction exact), and
+//   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh) + O(2^-24 a b),
+// six bf16 MFMAs with fp32 accumulation for one fp32 product at 1/6 of 2500 TFLOP/s.  The
+// three dropped terms are below 2^-23.4 |a b| together; what an fp32 sum over K of a few
+// hundred loses to rounding is larger, and a 32-k MFMA rounds its running sum an eighth as
+// often as the 4-k fp32 one.  Relative 2-norm error against float64, N(0, 1) x N(0, 0.02),
+// fp32 MFMA kernel -> this one: K = 768 5.0e-7 -> 4.2e-7, 3072 9.9e-7 -> 8.7e-7, 14336 2.1e-6 ->
+// 2.1e-6 (1.0e-6 with ranges of k); all-positive operands 4.2e-7 -> 3.7e-7.
+// Times, the 128 x 128 fp32 MFMA kernel (gemm.hip) -> this one with the splitting launch:
+// 4096 x 2304 x 768 170 -> 76 us, 4096 x 768 x 3072 240 -> 105, 2048 x 1024 x 4096 381 -> 100.
+// What bounds it: six MFMAs per product at the rate the chip holds with every CU busy (1.4
+// PFLOP/s of bf16 on 256 x 144 tiles, against 2.5 nominal; one tile on an idle chip runs its
+// stages within 20 % of the MFMA time), plus about 11 us of splitting at that shape.
+//
+// 1. split_kernel writes both operands' parts in MFMA fragment order: units of 16 rows (of
+//    A, or columns of W) x 32 k, 1 KB each, lane (lr, lq)'s 16 bytes at lane * 16 = row lr,
+//    k 8 lq .. +7.  A unit is one direct-to-LDS load instruction of contiguous memory and
+//    one conflict-free ds_read_b128, whatever the layout of the operand was.
+// 2. gemm_x3: 4 loader and 4 compute waves as in gemm_f16_ws, 32-k stages of (BM + BN) / 16
+//    x 3 units.
+// Infinities and NaN cannot be split (inf - inf); split_kernel reports any by writing the
+// call's number to a flag word, and gemm_x3 then computes its tile from the original
+// operands on the fp32 MFMA, with the results the fp32 kernel would have.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <atomic>
+
+#include "kernels.h"
+#include "cdna4.h"
+#include "gemm_f32_store.h"
+#include "gemm_x3.h"
+
+namespace {
+
+using namespace cdna4;
+
+typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
+constexpr int kUnit = 512;                 // halves per unit (16 rows x 32 k)
+
+struct X3Args {
+    cf_gemm_args_t g;
+    uint16_t* ap;                          // A's parts, [row tile][k tile][3] units
+    uint16_t* wp;                          // W's, [column tile][k tile][3], segments side by side
+    uint32_t* flag;                        // == call: an operand is not finite
+    uint32_t  call;
+    int       mt, nt, kt;                  // tiles of 16 rows, 16 columns, 32 k
+    int       tiles_m, tiles_n;
+    int       ks, per;                     // ranges of k (blockIdx.y) and their 32-k stages
+    float*    part;                        // ks > 1: sums [range][M][columns]
+};
+
+// The three parts of x, as the upper halves of three floats.
+__device__ __forceinline__ void split3(float x, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = __float_as_uint(x) & 0xffff0000u;
+    const float r = x - __uint_as_float(h);
+    m = __float_as_uint(r) & 0xffff0000u;
+    l = __float_as_uint(r - __uint_as_float(m));          // at most 8 bits: its lower half is zero
+}
+__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
+
+// One unit per wave: lane (lr, lq) takes row lr's k 8 lq .. +7.  Workgroups 0 .. (A's row
+// tiles x k tile groups) - 1 split A, the rest W.  Bound by memory (4 bytes in, 6 out).
+__global__ __launch_bounds__(256)
+void split_kernel(X3Args x, int a_wgs) {
+    const cf_gemm_args_t& a = x.g;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+    const int K = a.K, kg = (x.kt + 3) / 4;               // k tile groups of 4 (one per wave)
+    int id = blockIdx.x;
+    const bool is_w = id >= a_wgs;
+    if (is_w) id -= a_wgs;
+    const int t = id / kg, kt = (id - t * kg) * 4 + wave;
+    if (kt >= x.kt) return;
+    const int k0 = 32 * kt + 8 * lq;
+    float v[8];
+    uint16_t* dst;
+    if (!is_w || a.w_nk) {
+        // Rows contiguous along k: A, or W given as (N, K).
+        const int rows = is_w ? a.n[0] : a.M;
+        const float* src = (const float*)(is_w ? a.w[0] : a.a) + (size_t)min(16 * t + lr, rows - 1) * K + k0;
+        const f4_t v0 = *(const f4_t*)src, v1 = *(const f4_t*)(src + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) { v[e] = v0[e]; v[4 + e] = v1[e]; }
+        dst = is_w ? x.wp : x.ap;
+    } else {
+        // W (K, N): eight rows of one column; segment widths are multiples of 16.
+        const Segs sg = load_segs(a);
+        const int c = 16 * t, seg = sg.of(c), N = sg.width(seg);
+        const CF_GLOBAL float* src = sg.w.at(seg) + (size_t)k0 * N + (c - sg.start(seg)) + lr;
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = src[(size_t)e * N];
+        dst = x.wp;
+    }
+    uint32_t h[8], m[8], l[8];
+    bool bad = false;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        bad = bad || (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
+        split3(v[e], h[e], m[e], l[e]);
+    }
+    if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) *x.flag = x.call;
+    uint4* const o = (uint4*)(dst + (size_t)(t * x.kt + kt) * (3 * kUnit)) + lane;
+    o[0] = uint4{pack_hi(h[0], h[1]), pack_hi(h[2], h[3]), pack_hi(h[4], h[5]), pack_hi(h[6], h[7])};
+    o[64] = uint4{pack_hi(m[0], m[1]), pack_hi(m[2], m[3]), pack_hi(m[4], m[5]), pack_hi(m[6], m[7])};
+    o[128] = uint4{pack_hi(l[0], l[1]), pack_hi(l[2], l[3]), pack_hi(l[4], l[5]), pack_hi(l[6], l[7])};
+}
+
+// NCW compute waves, WMC of them along M.  Two per SIMD (8) where the tile divides among
+// them: one's MFMAs cover the other's LDS reads.
+template <int BM, int BN, int NCW, int WMC>
+struct X3Shape {
+    static constexpr int WM = BM / WMC, WN = BN * WMC / NCW;   // rows and columns of a compute wave
+    static constexpr int MI = WM / 16, NJ = WN / 16;
+    static constexpr int AU = BM / 16 * 3, WU = BN / 16 * 3, U = AU + WU;   // units per stage
+    static constexpr int PW = (U + 3) / 4;            // load instructions per loader wave, at most
+    static constexpr int ST = U * kUnit;              // halves per stage
+    static_assert(WM % 16 == 0 && BN * WMC % (16 * NCW) == 0, "wave tile");
+};
+template <int BM, int BN, int NCW, int WMC, int S>
+constexpr unsigned x3_lds_bytes() { return (unsigned)S * X3Shape<BM, BN, NCW, WMC>::ST * 2u; }
+
+// The product.  Stages of 32 k; a compute wave owns MI x NJ tiles of 16 x 16 and runs 6 MI
+// MFMAs per 16 columns and stage, the smallest terms first.  Results go out straight from
+// the accumulators (C^T: four consecutive columns per lane, 16 bytes).
+template <int BM, int BN, int NCW, int WMC, int S>
+__global__ __launch_bounds__(64 * (NCW + 4), 1)
+void gemm_x3(X3Args x) {
+    using SH = X3Shape<BM, BN, NCW, WMC>;
+    constexpr int MI = SH::MI, NJ = SH::NJ, U = SH::U, AU = SH::AU, PW = SH::PW, ST = SH::ST;
+    extern __shared__ __attribute__((aligned(16))) uint16_t smem_x3[];
+    const cf_gemm_args_t& a = x.g;
+    int tm, tn;
+    xcd_tile((int)blockIdx.x, x.tiles_m, x.tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN, K = a.K;
+    const int kt0 = (int)blockIdx.y * x.per, nk = min(x.kt - kt0, x.per);    // no range is empty
+    const Segs sg = load_segs(a);
+    const int ntot = sg.total;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool slow = (uint32_t)__builtin_amdgcn_readfirstlane((int)*(const volatile uint32_t*)x.flag) == x.call;
+
+    if (wave >= NCW) {
+        if (slow) return;                                  // the compute waves use no barrier then
+        const int cw = wave & 3;
+        uint32_t off[PW];
+        int nu = 0;
+#pragma unroll
+        for (int v = 0; v < PW; v++) {
+            const int u = cw + 4 * v;
+            nu += u < U ? 1 : 0;
+            const int tl = u < AU ? min(m0 / 16 + u / 3, x.mt - 1) : min(n0 / 16 + min(u - AU, SH::WU - 1) / 3, x.nt - 1);
+            off[v] = (uint32_t)tl * (uint32_t)x.kt * 3072u + (uint32_t)(u % 3) * 1024u + (uint32_t)lane * 16u;
+        }
+        const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_offset(smem_x3) + (uint32_t)cw * 1024u);
+        auto issue = [&](int kt, int stage) {
+            const uint16_t* ab = x.ap + (size_t)(kt0 + kt) * (3 * kUnit);
+            const uint16_t* wb = x.wp + (size_t)(kt0 + kt) * (3 * kUnit);
+            const uint32_t so = lds0 + (uint32_t)stage * (ST * 2u);
+#pragma unroll
+            for (int v = 0; v < PW; v++)
+                if (v < nu) lds_dma16_s(off[v], cw + 4 * v < AU ? ab : wb, so + 4096u * v);
+        };
+        auto wait = [&](int ahead) {
+            if (nu == PW) wait_ahead<PW, S - 2>(ahead);
+            else wait_ahead<PW - 1, S - 2>(ahead);
+        };
+        for (int s = 0; s < S - 1 && s < nk; s++) issue(s, s);
+        wait(min(S - 2, nk - 1));
+        ring_barrier();
+        for_each_stage<S>(nk, [&](int kt, auto stage_c) {
+            constexpr int stage = decltype(stage_c)::value;
+            if (kt + S - 1 < nk) issue(kt + S - 1, (stage + S - 1) % S);
+            if (kt + 1 < nk) wait(min(S - 2, nk - 2 - kt));
+            ring_barrier();
+        });
+        return;
+    }
+
+    const int wm = SH::WM * (wave % WMC), wn = SH::WN * (wave / WMC);
+    f4_t acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+
+    if (!slow) {
+        const uint16_t* const a_rd = smem_x3 + (wm / 16) * (3 * kUnit) + lane * 8;
+        const uint16_t* const w_rd = smem_x3 + (AU + (wn / 16) * 3) * kUnit + lane * 8;
+        ring_barrier();
+        for_each_stage<S>(nk, [&](int, auto stage_c) {
+            constexpr int stage = decltype(stage_c)::value;
+            b8_t af[MI][3];
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) af[i][p] = *(const b8_t*)(a_rd + stage * ST + (3 * i + p) * kUnit);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                b8_t bf[3];
+#pragma unroll
+                for (int p = 0; p < 3; p++) bf[p] = *(const b8_t*)(w_rd + stage * ST + (3 * j + p) * kUnit);
+                constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int q = 0; q < 6; q++)
+#pragma unroll
+                    for (int i = 0; i < MI; i++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[PB[q]], af[i][PA[q]], acc[i][j], 0, 0, 0);
+            }
+            ring_barrier();
+        });
+    } else {
+        // From the original operands: lane (lr, lq) loads row (column) lr's k0 + lq.
+        const float* ar[MI];
+        const CF_GLOBAL float* wr[NJ];
+        size_t wst[NJ];
+#pragma unroll
+        for (int i = 0; i < MI; i++) ar[i] = (const float*)a.a + (size_t)min(m0 + wm + 16 * i + lr, a.M - 1) * K + 32 * kt0 + lq;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int c = min(n0 + wn + 16 * j + lr, ntot - 1);
+            const int seg = sg.of(c), N = sg.width(seg), col = c - sg.start(seg);
+            wr[j] = sg.w.at(seg) + (a.w_nk ? (size_t)col * K + 32 * kt0 + lq : (size_t)(32 * kt0 + lq) * N + col);
+            wst[j] = a.w_nk ? 4 : (size_t)4 * N;
+        }
+        for (int k = 0; k < 32 * nk; k += 4) {
+            float av[MI];
+#pragma unroll
+            for (int i = 0; i < MI; i++) av[i] = ar[i][k];
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                const float bv = *wr[j];
+                wr[j] += wst[j];
+#pragma unroll
+                for (int i = 0; i < MI; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av[i], acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+
+    store_f32_ct<MI, NJ>(a, sg, m0 + wm, n0 + wn, lr, lq, acc,
+                         x.ks > 1 ? x.part + (size_t)blockIdx.y * a.M * ntot : nullptr);
+}
+
+template <int BM, int BN, int NCW, int WMC, int S>
+hipError_t launch_x3(dim3 grid, hipStream_t st, const X3Args& x) {
+    constexpr unsigned lds = x3_lds_bytes<BM, BN, NCW, WMC, S>();
+    static std::atomic<uint64_t> raised{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev >= 64 || !((raised.load(std::memory_order_acquire) >> dev) & 1u)) {
+        e = hipFuncSetAttribute((const void*)gemm_x3<BM, BN, NCW, WMC, S>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        if (dev < 64) raised.fetch_or(1ull << dev, std::memory_order_release);
+    }
+    hipLaunchKernelGGL((gemm_x3<BM, BN, NCW, WMC, S>), grid, dim3(64 * (NCW + 4)), lds, st, x);
+    return hipSuccess;
+}
+
+struct X3Candidate {
+    int bm, bn;
+    hipError_t (*launch)(dim3, hipStream_t, const X3Args&);
+};
+const X3Candidate kX3Shapes[] = {
+    {256, 160, launch_x3<256, 160, 8, 4, 2>}, {256, 144, launch_x3<256, 144, 4, 4, 2>},
+    {256, 128, launch_x3<256, 128, 8, 4, 2>}, {256, 96, launch_x3<256, 96, 8, 4, 2>},
+    {256, 64, launch_x3<256, 64, 8, 4, 2>},   {128, 192, launch_x3<128, 192, 8, 2, 2>},
+    {128, 128, launch_x3<128, 128, 8, 2, 3>}, {128, 96, launch_x3<128, 96, 8, 4, 3>},
+    {128, 64, launch_x3<128, 64, 8, 4, 4>},   {64, 64, launch_x3<64, 64, 8, 2, 6>},
+};
+constexpr int kX3Count = (int)(sizeof(kX3Shapes) / sizeof(kX3Shapes[0]));
+constexpr int kX3MaxSplit = 16;
+int g_x3_mode = 0, g_x3_bm = 0, g_x3_bn = 0, g_x3_ks = 0;
+
+}  // namespace
+
+extern "C" void cf_gemm_set_x3(int32_t mode, int32_t bm, int32_t bn, int32_t ks) {
+    g_x3_mode = mode;
+    g_x3_ks = ks;
+    g_x3_bm = bm;
+    g_x3_bn = bn;
+}
+
+int gemm_x3_pick(const cf_gemm_args_t* a, int* ks_out, float* clk) {
+    if (g_x3_mode == 1 || a->elem != CF_ELEM_F32 || a->out_f32) return -1;
+    if (a->K % 32 != 0 || (uintptr_t)a->a % 16 != 0) return -1;
+    if (a->w_nk && (a->nseg != 1 || a->out_kind != CF_GEMM_OUT_ROWMAJOR || (uintptr_t)a->w[0] % 16 != 0)) return -1;
+    if (a->out_kind == CF_GEMM_OUT_QKV && a->d % 4 != 0) return -1;
+    uintptr_t al = (uintptr_t)a->residual;
+    long long ntot = 0;
+    for (int s = 0; s < a->nseg; s++) {
+        if (a->n[s] % 16 != 0) return -1;
+        ntot += a->n[s];
+        al |= (uintptr_t)a->bias[s];
+        if (s == 0 || a->out_kind == CF_GEMM_OUT_QKV) al |= (uintptr_t)a->out[s];
+    }
+    if (al % 16 != 0) return -1;
+    const long long mt = (a->M + 15LL) / 16, nt = ntot / 16, kt = a->K / 32;
+    // 32-bit unit offsets, and the splitting grid.
+    if (mt * kt * 3072 >= (1LL << 32) || nt * kt * 3072 >= (1LL << 32)) return -1;
+    const bool may_split = a->out_kind != CF_GEMM_OUT_QKV && (long long)a->M * ntot < (1LL << 30);
+    const int cus = cu_count();
+    int best = -1;
+    *ks_out = 1;
+    float best_cost = 0.0f;
+    for (int i = 0; i < kX3Count; i++) {
+        const X3Candidate& c = kX3Shapes[i];
+        const long long tiles = (a->M + c.bm - 1LL) / c.bm * ((ntot + c.bn - 1) / c.bn);
+        if (tiles > 0x7fffffffLL) continue;
+        // Measured per 32-k stage with every CU busy: 450 clk plus 2900 FLOP/clk of MFMA
+        // work (1.4-1.6 PFLOP/s over the chip; torch's bf16 8192^3 product ran at 1.2 here),
+        // for tiles of 64 x 64 to 256 x 160 within 6 %; about 4000 clk per tile around it.
+        // Ranges of k add a second launch (8900 clk) and the sums' way through memory.
+        const float stage = 450.0f + (float)(c.bm * c.bn) * (32.0f * 2.0f * 6.0f / 2900.0f);
+        for (int ks = 1; ks <= kX3MaxSplit; ks++) {
+            const int per = (int)((kt + ks - 1) / ks);
+            if (ks > 1 && (!may_split || tiles * ks > 2LL * cus || per < 4)) break;
+            if (ks > 1 && (long long)(ks - 1) * per >= kt) continue;
+            float cost = (float)((tiles * ks + cus - 1) / cus) * (stage * (float)per + 4000.0f);
+            if (ks > 1) cost += 8900.0f + (float)ks * (float)a->M * (float)ntot * (8.0f / 1900.0f);
+            if (c.bm == g_x3_bm && c.bn == g_x3_bn && (g_x3_ks == 0 ? ks == 1 : ks == g_x3_ks)) cost = -1.0f;
+            if (best < 0 || cost < best_cost) {
+                best = i;
+                best_cost = cost;
+                *ks_out = ks;
+            }
+        }
+    }
+    // ... and the splitting launch: 10 bytes of traffic per operand element.
+    *clk = best_cost + 8900.0f + ((float)a->M * (float)a->K + (float)a->K * (float)ntot) * (10.0f / 2100.0f);
+    if (g_x3_mode == 2) *clk = 0.0f;
+    return best;
+}
+
+size_t gemm_x3_floats(const cf_gemm_args_t* a) {
+    size_t ntot = 0;
+    for (int s = 0; s < a->nseg; s++) ntot += (size_t)a->n[s];
+    const size_t units = ((size_t)(a->M + 15) / 16 + ntot / 16) * (size_t)(a->K / 32) * 3;
+    // The flag's 256 bytes, then 1 KB per unit, then the ranges' sums.
+    return 64 + units * 256 + (a->ksplit > 1 ? (size_t)a->ksplit * (size_t)a->M * ntot : 0);
+}
+
+int gemm_x3_launch(const cf_gemm_args_t* a, int pick, hipStream_t st) {
+    static std::atomic<uint32_t> calls{0};
+    X3Args x;
+    x.g = *a;
+    int ntot = 0;
+    for (int s = 0; s < a->nseg; s++) ntot += a->n[s];
+    x.mt = (a->M + 15) / 16;
+    x.nt = ntot / 16;
+    x.kt = a->K / 32;
+    x.flag = (uint32_t*)a->partials;
+    x.call = calls.fetch_add(1, std::memory_order_relaxed) + 1;
+    x.ap = (uint16_t*)(a->partials + 64);
+    x.wp = x.ap + (size_t)x.mt * x.kt * (3 * kUnit);
+    const X3Candidate& c = kX3Shapes[pick];
+    x.tiles_m = (a->M + c.bm - 1) / c.bm;
+    x.tiles_n = (ntot + c.bn - 1) / c.bn;
+    const int kg = (x.kt + 3) / 4;
+    const long long wgs = (long long)(x.mt + x.nt) * kg;
+    if (wgs > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(split_kernel, dim3((unsigned)wgs), dim3(256), 0, st, x, x.mt * kg);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return (int)e;
+    x.ks = a->ksplit;
+    x.per = (x.kt + x.ks - 1) / x.ks;
+    x.part = (float*)(x.wp + (size_t)x.nt * x.kt * (3 * kUnit));
+    e = c.launch(dim3((unsigned)(x.tiles_m * x.tiles_n), (unsigned)x.ks), st, x);
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e != hipSuccess || x.ks == 1) return (int)e;
+    x.g.partials = x.part;
+    return gemm_splitk_sum_launch(&x.g, st);
+}

@@ -195,14 +195,21 @@ typedef struct {
     int32_t     plan;        /* set by cf_gemm_plan: the wave-specialised kernel's tile
                                 (> 0) or another kernel (-1); 0 = the launch chooses */
     int32_t     ksplit;      /* set by cf_gemm_plan: ranges of k with partial sums */
-    float*      partials;    /* workspace for those sums, or NULL (the launch then does not
-                                split k across workgroups) */
+    float*      partials;    /* workspace of the size cf_gemm_plan gave, or NULL (the launch
+                                then takes a kernel that needs none) */
 } cf_gemm_args_t;
 
 int cf_launch_gemm(const cf_gemm_args_t* a, void* stream);
+/* FP32 products on bf16 MFMA (gemm_x3.hip): mode 0 = where the cost model says so, 1 = never, 2 =
+ * wherever the shape allows it; bm, bn force a tile with ks ranges of k (0 = the cost
+ * model's; ks 0 = 1).  cf_gemm_set_f32: the same of the fp32 MFMA kernel for the products
+ * that leaves (mode 1 = never).  Tests and measurements. */
+void    cf_gemm_set_f32(int32_t mode, int32_t bm, int32_t bn, int32_t ks);
+void    cf_gemm_set_x3(int32_t mode, int32_t bm, int32_t bn, int32_t ks);
 /* Chooses the kernel (plan, ksplit) from the sizes and the pointers' alignment, and
- * returns the floats of workspace for the sums over ranges of k (0 = none).  The pointers
- * may be stand-ins of the same alignment. */
+ * returns the floats of workspace it needs in `partials` (0 = none): sums over ranges of
+ * k, or the split operands of an FP32 product.  The pointers may be stand-ins of the same
+ * alignment. */
 size_t  cf_gemm_plan(cf_gemm_args_t* a);
 /* Tuning override of the fp16 direct-to-LDS GEMM's ring depth (3 or 4 stages; 0 =
  * automatic: 3, i.e. three workgroups per CU, when there are more than two tiles per CU). */

@@ -101,6 +101,20 @@ def test_fused_f16_entry_small_and_misaligned(gpu, B, S, H, H_kv, d, skew_in, sk
     assert np.all(got[:n] == 7.0) and np.all(got[n + B * S * H * d:] == 7.0)
 
 
+@pytest.mark.parametrize("kernel", ["x3", "f32"])
+@pytest.mark.parametrize("B,S,H,H_kv,d,causal", [(2, 131, 6, 2, 64, True), (1, 8, 4, 4, 32, False), (3, 77, 4, 2, 128, False)])
+def test_fused_f32_products(gpu, native, kernel, B, S, H, H_kv, d, causal):
+    """The FP32 op with its projections (Q|K|V scattered head-major, output with residual) on
+    each of the two FP32 product kernels, tokens no multiple of any tile."""
+    c = FusedCase(B, S, H, H_kv, d, seed=S + d, causal=causal, residual=True, bias_std=0.02)
+    try:
+        native.cf_gemm_set_x3(2 if kernel == "x3" else 1, 0, 0, 0)
+        got = run_fused_gpu(c)
+    finally:
+        native.cf_gemm_set_x3(0, 0, 0, 0)
+    assert max_abs(c.oracle(), got) <= TOL32
+
+
 def test_config3_bert_base_full_size(gpu):
     """B=8, S=512, D=768, 12x64, fp16, no mask.  Every row of the
     full-size run against a float64 evaluation of the same math, and batch rows 0 and 7

@@ -222,6 +222,86 @@ def test_matmul_f16_k_ranges(gpu, native, nk, M, N, K, bm, bn, ks):
         assert np.all(got[M * N:] == 7.0)
 
 
+def _mm_f32_run(native, A, B, bias, nk, kernel, bm, bn, ks):
+    """One FP32 product, forced onto "x3" (bf16 MFMA on split operands) or "f32" (the few-row
+    fp32 MFMA kernel) at a tile and number of k ranges; nothing may be written past it."""
+    import cudaforge_amd as cf
+    (M, K), N = A.shape, B.shape[1]
+    C = cf.DeviceBuffer.from_numpy(np.full(M * N + 1024, 7.0, np.float32))
+    p = cf.MatmulParams(M, N, K, False, nk, 1, 0, 0, 0, 0)
+    try:
+        if kernel == "x3":
+            native.cf_gemm_set_x3(2, bm, bn, ks)
+        elif kernel == "f32":
+            native.cf_gemm_set_x3(1, 0, 0, 0)
+            native.cf_gemm_set_f32(0, bm, bn, ks)
+        elif kernel == "general":
+            native.cf_gemm_set_x3(1, 0, 0, 0)
+            native.cf_gemm_set_f32(1, 0, 0, 0)
+        slots = [dev(A), dev(B.T if nk else B), None if bias is None else dev(bias)]
+        assert cf.call_op("matmul_f32_cuda", slots, [C], p) == 0
+        got = C.download()
+    finally:
+        native.cf_gemm_set_x3(0, 0, 0, 0)
+        native.cf_gemm_set_f32(0, 0, 0, 0)
+    assert np.all(got[M * N:] == 7.0)
+    return got[:M * N].reshape(M, N)
+
+
+X3_TILES = [(256, 160), (256, 144), (256, 128), (256, 96), (256, 64), (128, 192), (128, 128), (128, 96), (128, 64),
+            (64, 64)]
+F32_TILES = [(16, 64), (32, 64), (64, 64), (32, 32), (128, 64), (16, 128)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("kernel,bm,bn", [("x3", *t) for t in X3_TILES] + [("f32", *t) for t in F32_TILES])
+def test_matmul_f32_tiles(gpu, native, nk, kernel, bm, bn):
+    """Each FP32 tile with its last rows and columns cut, one and several ranges of k (the
+    last one shorter), W in both layouts, against float64.  Bound per element: the sum of K
+    products rounded once per step at most, K * 2^-24 * sum |a b|, ten times what is seen."""
+    for M, N, K, ks in ((1, 16, 32, 1), (130, 208, 352, 1), (277, 176, 3104, 3), (64, 64, 4096, 4)):
+        A, B = O.normal((M, K), M + N), O.normal((K, N), K + 1, 0.0, 1.0 / np.sqrt(K))
+        bias = O.normal((N,), 5, 0.0, 0.1)
+        want = A.astype(np.float64) @ B.astype(np.float64) + bias
+        bound = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64) * (K ** 0.5 * 2.0 ** -24) + 2.0 ** -22
+        got = _mm_f32_run(native, A, B, bias, nk, kernel, bm, bn, ks)
+        assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.gpu
+def test_matmul_f32_split_operands_keep_precision_and_range(gpu, native):
+    """The bf16-MFMA product is no further from float64 than the general fp32 kernel, also
+    for operands spread over 40 binary orders, at the largest and smallest exponents and
+    with exact cancellation; infinities and NaN give what the fp32 kernel gives."""
+    rng = np.random.default_rng(3)
+
+    def err(y, want):
+        return float(np.linalg.norm(y - want) / np.linalg.norm(want))
+
+    M, N, K = 320, 192, 768
+    a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    spread = np.exp2(rng.integers(-20, 20, (M, K))).astype(np.float32)
+    for A, B in ((a, b), (np.abs(a), np.abs(b)), (a * spread, b), (a * np.float32(2.0 ** 100), b * np.float32(2.0 ** -90)),
+                 (a * np.float32(1e-30), b * np.float32(1e-4)), (np.concatenate([a, -a], 1), np.concatenate([b, b], 0))):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        x3 = _mm_f32_run(native, A, B, None, False, "x3", 0, 0, 0)
+        if not want.any():
+            assert np.abs(x3).max() <= 1e-3                    # the cancelled sums' rounding
+            continue
+        assert err(x3, want) <= max(1.2 * err(_mm_f32_run(native, A, B, None, False, "general", 0, 0, 0), want), 2e-7)
+    A, B = a.copy(), b.copy()
+    A[5, 7], A[300, 100], B[3, 9] = np.inf, np.nan, -np.inf
+    for nk in (False, True):
+        x3, ref = (_mm_f32_run(native, A, B, None, nk, k, 0, 0, 0) for k in ("x3", "general"))
+        assert np.array_equal(np.isnan(x3), np.isnan(ref)) and np.array_equal(np.isinf(x3), np.isinf(ref))
+        ok = np.isfinite(ref)
+        assert np.array_equal(np.sign(x3[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
+        assert max_abs(x3[ok], ref[ok]) <= 1e-3
+    # The next call is finite again.
+    assert err(_mm_f32_run(native, a, b, None, False, "x3", 0, 0, 0), a.astype(np.float64) @ b.astype(np.float64)) <= 1e-6
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])
