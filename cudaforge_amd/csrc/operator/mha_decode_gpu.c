@@ -84,6 +84,14 @@ static void plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t
          * 1-17 % faster than one split per CU slot. */
         if (spread) target *= 4;
         int64_t n = cf_ceil_div(target, units);
+        /* Short contexts in one split, which writes O itself: the merge launch costs about
+         * 3.2 us, more than splitting saves.  One split against the plan above (core op,
+         * B = 6, 16 heads of 64, fp16): 128 positions 3.7 and 6.4 us, 256 5.1 and 6.1, 384 6.4
+         * and 6.4; fp32, whose split walks 64 positions at a time without reading ahead, 192
+         * 5.5 and 7.0 (and 257 7.8 against 7.3 inside the decode op, 12 heads); heads of 128
+         * move twice the bytes per position in groups of four: 64 positions 5.5 and 7.2 us,
+         * 128 7.8 and 7.3. */
+        if (fast && t_max <= (s->d > 64 ? 64 : elem == CF_ELEM_F16 ? 320 : 192)) n = 1;
         const int64_t nmax = cf_ceil_div(t_max, q);
         if (n > nmax) n = nmax;
         if (n < 1) n = 1;

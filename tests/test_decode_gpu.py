@@ -302,6 +302,27 @@ def test_config4_ragged_full_size(gpu):
     assert max_abs(ref, got) <= TOL16
 
 
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("H,H_kv,d,T", [(4, 4, 64, 64), (4, 2, 64, 320), (4, 4, 64, 321), (8, 2, 128, 64), (8, 2, 128, 65), (4, 4, 64, 192),
+                                        (8, 1, 64, 319)])
+def test_short_context_in_one_split(gpu, native, f16, H, H_kv, d, T):
+    """Contexts up to the length that runs as one split (no merge) and one position past
+    it, against float64 and against splits of 64 positions."""
+    from helpers import attn_ref64_all
+    Q, K, V = (O.normal(s, 610 + i) for i, s in enumerate([(3, H, d), (3, T, H_kv, d), (3, T, H_kv, d)]))
+    if f16:
+        Q, K, V = O.round_f16(Q), O.round_f16(K), O.round_f16(V)
+    ref = attn_ref64_all(Q, K, V, np.full(3, T, np.int32), H_kv, float(1 / np.sqrt(d)))
+    got = run_decode_attn_gpu(Q, K, V, T - 1, H_kv, f16)
+    try:
+        native.mha_decode_set_split_chunk(64)
+        split = run_decode_attn_gpu(Q, K, V, T - 1, H_kv, f16)
+    finally:
+        native.mha_decode_set_split_chunk(0)
+    tol = TOL16 if f16 else TOL32
+    assert max_abs(ref, got) <= tol and max_abs(split, got) <= tol
+
+
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1], [4096, 1, 17, 2999], [33] * 64, [1] * 63 + [5000],
                                   [16, 4080, 16, 4080], [257, 4095, 1000, 3]])
 def test_balanced_ragged_partition(gpu, native, lens):
