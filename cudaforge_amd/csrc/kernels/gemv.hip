@@ -9,7 +9,9 @@
 //   MFMA cols  <- batch rows m       (B operand = X, k-contiguous rows of X)
 //   MFMA k     <- reduction index k
 //
-// Two kernels:
+// Kernels:
+// * gemv_one (weights of a few MB, up to 16 rows) and gemv_small (a few rows, shapes that
+//   leaves): one pass over K and no second launch, see there.
 // * gemv_f16_dma (fp16, K % 32 == 0, every segment width % 64 == 0, 16-byte aligned):
 //   one wave per 64/128/256 columns and K chunk, W and X streamed by DMA into an LDS
 //   ring and multiplied as Y = X . W on MFMA (see the kernel); the K split is planned
@@ -61,6 +63,7 @@ struct Tiles {
     int ks;                           // K chunks (workgroups along K)
     int dma;                          // fp16 DMA path: its tile width (64/128/256), else 0
     int small;                        // one-pass kernel for small projections (gemv_small)
+    int one;                          // one-pass kernel of up to 16 rows: its columns (gemv_one)
     // The K-chunk sum's divisors, set by the launcher: column tiles, lanes per row
     // (bn / 4), and the RoPE head size (2 without RoPE).
     FastDiv div_tiles, div_lpr, div_rd;
@@ -474,7 +477,8 @@ void gemv_reduce4(cf_gemv_args_t a, Tiles t) {
         if (n + e < sg.n) out[e] = from_f<T>(o[e]);
 }
 
-// ---- small projections (a few batch rows, weights of a few MB, e.g. GPT-2-small
+// ---- small projections that gemv_one does not take (K no multiple of 32, or fp16 widths no
+// multiple of 32; a few batch rows, weights of a few MB, e.g. GPT-2-small
 // decode at batch 1): one pass over all of K, so no partials and no second launch; at
 // that size the fixed cost of the extra launch is most of the time.  A workgroup owns
 // kSmallCols = 16 columns and its 4 waves a quarter of K each.  A lane loads 16 bytes of
@@ -483,6 +487,7 @@ void gemv_reduce4(cf_gemv_args_t a, Tiles t) {
 // of W loads is issued before X is staged, so both arrive in one round trip.  Lanes of
 // one column group then sum over their rows with shuffles, the waves through LDS, and
 // M * 4 threads add the bias, rotate RoPE pairs and store 4 columns each.
+constexpr long long kOneMaxBytes = 16ll << 20;    // fp16 weight bytes up to which gemv_one is taken (fp32: twice)
 constexpr int kSmallCols = 16;
 constexpr int kSmallMaxM = 4;
 constexpr int kSmallMaxX = 4096;                  // M * K floats of X staged in LDS
@@ -614,6 +619,171 @@ void gemv_small(cf_gemv_args_t a, Tiles t) {
     }
 }
 
+// ---- up to 16 rows, weights of a few MB: one pass over all of K and no second launch.  A
+// workgroup owns 64 bytes of columns (BN = 32 fp16, 16 fp32); its 8 waves take the 32-k steps
+// in turn, each through a ring of its own as in gemv_f16_dma (NS steps deep: up to K = 256 NS
+// every load is in flight at once), and their sums meet in LDS, where a thread per output
+// adds them, the bias, and RoPE to the pair it shares with its neighbour.
+// What bounds it is the load path's cost per cache line, about 4 clk for each of the K rows a
+// workgroup touches however few columns it has (16 fp16 columns measured 10-15 % slower than
+// 32), so about K / 600 us beside launch and reduction; weights beyond kOneMaxBytes, and with
+// them long K, keep the split-K kernels.  The decode op, fp16, 6 sequences, RoPE: 12 heads of
+// 64, 200 positions 19.3 -> 14.5 us; 16 heads, 777 positions 22.3 -> 19.8; 16 / 4 heads of 128,
+// 251 positions 24.5 -> 23.1; 32 / 8 heads of 128 (50 MB of Q|K|V weights, not taken) would go
+// from 39 to 51.  fp32: 12 heads of 64, 6 sequences 25 -> 17 us, 16 sequences 33 -> 20; 16 / 4
+// heads of 128, 8 sequences 34 -> 28.  It also takes what gemv_small took where both apply (one
+// sequence, 12 heads of 64: fp16 16.0 -> 13.0 us, fp32 18.4 -> 16.3).
+template <typename T>
+__global__ __launch_bounds__(512)
+void gemv_one(cf_gemv_args_t a, Tiles t) {
+    constexpr bool F16 = sizeof(T) == 2;
+    constexpr int BN = 64 / (int)sizeof(T), NS = F16 ? 6 : 4, NWV = 8;
+    constexpr int CPR = 4, RPI = 16, NI = 2;     // chunks per W row, rows and instructions per stage
+    constexpr int XI = F16 ? 1 : 2, NL = NI + XI;   // X: 16 rows of 32 k
+    constexpr int NT = BN / 16;
+    constexpr int W_ST = kDK * BN, STAGE = W_ST + kMTile * kDK;
+    __shared__ __attribute__((aligned(16))) T ring_all[NWV * NS * STAGE];
+
+    const int tile = blockIdx.x, mt = blockIdx.y;
+    const int seg = seg_of(a, t, tile);
+    const cf_gemv_seg_t& sg = a.seg[seg];
+    const int N = (int)sg.n;
+    const int n0 = (tile - t.start[seg]) * BN;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T* const ring = ring_all + wave * (NS * STAGE);
+    const int steps = a.K / kDK, nst = (steps - wave + NWV - 1) / NWV;   // steps wave, wave + 8, ..
+    const T* __restrict__ W = (const T*)sg.w;
+    const T* __restrict__ X = (const T*)a.x;
+
+    // The storing threads' bias and RoPE angle, unconditional through a stand-in as in
+    // gemv_small.  With a host-known position they are issued before the ring's loads and
+    // never waited for there (an older load still in flight only makes the ring's counted
+    // waits stricter); with device positions the angle waits for the position, which is
+    // loaded after the ring's first loads and so arrives in their round trip.
+    const int om = tid / BN, oc = tid % BN, m_out = mt * kMTile + om, n = n0 + oc;
+    const bool storer = om < kMTile && m_out < a.M;
+    const T* const stand_in = W;
+    const T* const bp = sg.bias ? (const T*)sg.bias : stand_in;
+    const T bias_v = bp[n];
+    const int rd = a.rope_table ? a.rope_d : 2, pair = (n - fastdiv(n, t.div_rd) * rd) >> 1;
+    const bool rope_seg = a.rope_table && ((a.rope_segs >> seg) & 1);
+    const float2* const table = a.rope_table ? (const float2*)a.rope_table : (const float2*)stand_in;
+    auto in_table = [&](int64_t p) { return rope_seg && p >= 0 && p < a.rope_rows; };
+    int64_t pos = a.pos_uniform;
+    float2 cs = table[(in_table(pos) ? pos : 0) * (rd >> 1) + pair];
+
+    // fp16 W is read transposed: chunk c of row r sits at c ^ 2 for rows 8-15 and 24-31, so
+    // the 8 rows of a half-wave's read (0-3 and 8-11 of each 16) do not meet in a bank.
+    auto wswz1 = [](int row) { return F16 ? ((row >> 3) & 1) << 1 : 0; };
+    uint32_t woff[NI], xoff[XI];
+#pragma unroll
+    for (int u = 0; u < NI; u++) {
+        const int row = RPI * u + lane / CPR;
+        woff[u] = (uint32_t)row * (uint32_t)N * (uint32_t)sizeof(T) + 16u * (uint32_t)((lane % CPR) ^ wswz1(row));
+    }
+#pragma unroll
+    for (int u = 0; u < XI; u++) {
+        const int row = F16 ? lane >> 2 : 8 * u + (lane >> 3);
+        const int c = F16 ? (lane & 3) ^ xswz(row) : (lane & 7) ^ ((row >> 1) & 7);
+        xoff[u] = (uint32_t)min(mt * kMTile + row, a.M - 1) * (uint32_t)a.K * (uint32_t)sizeof(T) + 16u * (uint32_t)c;
+    }
+    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_offset(ring));
+    auto issue = [&](int st, int stage) {           // stage == st % NS
+        const int k0 = (wave + NWV * st) * kDK;
+        const uint32_t sb = base + (uint32_t)(stage * STAGE * (int)sizeof(T));
+        const T* wb = W + (size_t)k0 * N + n0;
+#pragma unroll
+        for (int u = 0; u < NI; u++) lds_dma16_s(woff[u], wb, sb + u * 1024u);
+#pragma unroll
+        for (int u = 0; u < XI; u++) lds_dma16_s(xoff[u], X + k0, sb + (uint32_t)(W_ST * (int)sizeof(T)) + u * 1024u);
+    };
+    // Per-lane LDS read offsets inside a stage (fp16 W transposed; fp32 as it lies).
+    int x_rd[F16 ? 1 : kDK / 4], w_rd[NT][2];
+#pragma unroll
+    for (int i = 0; i < (F16 ? 1 : kDK / 4); i++)
+        x_rd[i] = W_ST + lr * kDK + (F16 ? 8 * (lq ^ xswz(lr)) : 4 * (i ^ ((lr >> 1) & 7)) + lq);
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int row = 8 * lq + 4 * e + (lr >> 2), col = 16 * j + 4 * (lr & 3);
+            w_rd[j][e] = F16 ? row * BN + 8 * ((col >> 3) ^ wswz1(row)) + (col & 7) : lq * BN + lr;
+        }
+    // fp16: a sum per 16 columns.  fp32: four sums of the 16 columns in turn, so that an MFMA
+    // does not wait for the one before it.
+    constexpr int NA = F16 ? NT : 4;
+    f4_t acc[NA];
+#pragma unroll
+    for (int j = 0; j < NA; j++) acc[j] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < NS - 1; st++)
+        if (st < nst) issue(st, st);
+    if (a.pos_lens) {
+        pos = a.pos_lens[min(m_out, a.M - 1)];
+        cs = table[(in_table(pos) ? pos : 0) * (rd >> 1) + pair];
+    }
+    for_each_stage<NS>(nst, [&](int st, auto stage_c) {
+        constexpr int stage = decltype(stage_c)::value;
+        if (st + NS - 1 < nst) {
+            wait_lds_reads();
+            issue(st + NS - 1, (stage + NS - 1) % NS);
+        }
+        wait_ahead<NL, NS - 1>(min(NS - 1, nst - 1 - st));
+        const T* sp = ring + stage * STAGE;
+        if constexpr (F16) {
+            const h8_t xa = *(const h8_t*)(sp + x_rd[0]);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const h8_t wb = cat8(ds_read_tr4(sp + w_rd[j][0]), ds_read_tr4(sp + w_rd[j][1]));
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, wb, acc[j], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kDK / 4; i++)       // k = 4 i + lq
+                acc[i % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(sp[x_rd[i]], sp[w_rd[0][0] + 4 * i * BN], acc[i % NA], 0, 0, 0);
+        }
+    });
+    if constexpr (!F16) acc[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    // Sums to the start of the wave's own ring (its reads are done), [16 rows][BN].
+    wait_lds_reads();
+    float* const red = (float*)ring;
+    static_assert(kMTile * BN * 4 <= NS * STAGE * (int)sizeof(T), "the sums fit the ring");
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[(4 * lq + i) * BN + 16 * j + lr] = acc[j][i];
+    __syncthreads();
+    advance_lengths(a);
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NWV; w++) v += ((const float*)(ring_all + w * (NS * STAGE)))[min(om, kMTile - 1) * BN + oc];
+    v = sg.bias ? v + to_f(bias_v) : v;
+    // n and n + 1 (n even) are neighbouring lanes and rope_d is even: a pair never splits.
+    const float other = dpp_f<kDppXor1>(v);
+    if (in_table(pos)) {
+        float x0 = (n & 1) ? other : v, x1 = (n & 1) ? v : other;
+        rotate_pair(x0, x1, cs);
+        v = (n & 1) ? x1 : x0;
+    }
+    if (storer) store_val<T>(a, sg, m_out, n, v);
+}
+
+int g_one = 1;      // 0: never take gemv_one; 1: automatic; 2: wherever the shape allows it
+
+// Columns per workgroup of gemv_one for this launch, or 0.
+int one_bn(const cf_gemv_args_t* a) {
+    const int esz = a->elem == CF_ELEM_F16 ? 2 : 4, bn = 64 / esz;
+    if (g_one == 0 || a->K % kDK != 0 || (uintptr_t)a->x % 16 != 0) return 0;
+    long long bytes = 0;
+    for (int s = 0; s < a->nseg; s++) {
+        if ((uintptr_t)a->seg[s].w % 16 != 0 || a->seg[s].n % bn != 0) return 0;
+        bytes += (long long)a->K * a->seg[s].n * esz;
+    }
+    if (g_one == 1 && (bytes > kOneMaxBytes * (esz / 2) || a->M > kMTile)) return 0;
+    return bn;
+}
+
 int g_small = 1;    // 0: never take gemv_small; 1: for small weights; 2: wherever it applies
 
 int small_ok(const cf_gemv_args_t* a) {
@@ -630,13 +800,27 @@ int small_ok(const cf_gemv_args_t* a) {
 
 Tiles make_tiles(const cf_gemv_args_t* a) {
     Tiles t{};
-    if (small_ok(a)) {
+    const int ob = g_small != 1 || g_dma_bn || g_dma_ks ? 0 : one_bn(a);
+    if (!ob && small_ok(a)) {
         t.small = 1;
         t.bn = kSmallCols;
         int acc = 0;
         for (int s = 0; s < a->nseg; s++) {
             t.start[s] = acc;
             acc += (int)(a->seg[s].n / kSmallCols);
+        }
+        for (int s = a->nseg; s <= CF_GEMV_MAX_SEGS; s++) t.start[s] = acc;
+        t.ks = 1;
+        t.k_chunk = a->K;
+        t.vec_ok = 1;
+        return t;
+    }
+    if (ob) {
+        t.one = t.bn = ob;
+        int acc = 0;
+        for (int s = 0; s < a->nseg; s++) {
+            t.start[s] = acc;
+            acc += (int)(a->seg[s].n / ob);
         }
         for (int s = a->nseg; s <= CF_GEMV_MAX_SEGS; s++) t.start[s] = acc;
         t.ks = 1;
@@ -696,10 +880,11 @@ Tiles make_tiles(const cf_gemv_args_t* a) {
 extern "C" int32_t cf_gemv_col_tile(int32_t elem) { (void)elem; return kColTile; }
 extern "C" void cf_gemv_set_dma_tile(int32_t bn) { g_dma_bn = bn; }
 extern "C" void cf_gemv_set_dma_ksplit(int32_t ks) { g_dma_ks = ks; }
+extern "C" void cf_gemv_set_one(int32_t mode) { g_one = mode >= 0 && mode <= 2 ? mode : 1; }
 extern "C" void cf_gemv_set_small(int32_t mode) { g_small = mode >= 0 && mode <= 2 ? mode : 1; }
 extern "C" int32_t cf_gemv_fuses_rope(const cf_gemv_args_t* a) {
     const Tiles t = make_tiles(a);
-    return t.small || t.ks > 1 ? 1 : 0;
+    return t.small || t.one || t.ks > 1 ? 1 : 0;
 }
 extern "C" int32_t cf_gemv_k_step(int32_t elem) {
     return elem == CF_ELEM_F16 ? Cfg<_Float16>::KSTEP : Cfg<float>::KSTEP;
@@ -715,7 +900,7 @@ extern "C" int cf_launch_gemv(const cf_gemv_args_t* a, void* stream) {
     const Tiles t = make_tiles(a);
     if (a->M <= 0 || a->K <= 0 || t.start[a->nseg] <= 0) return (int)hipErrorInvalidValue;
     // RoPE is applied in the K-chunk sum or the one-pass small kernel only.
-    if (a->rope_table && ((t.ks == 1 && !t.small) || a->rope_d <= 0 || (a->rope_d & 1)))
+    if (a->rope_table && ((t.ks == 1 && !t.small && !t.one) || a->rope_d <= 0 || (a->rope_d & 1)))
         return (int)hipErrorInvalidValue;
     cf_gemv_args_t args = *a;
     args.k_split = t.ks;
@@ -730,6 +915,14 @@ extern "C" int cf_launch_gemv(const cf_gemv_args_t* a, void* stream) {
         return (int)hipGetLastError();
     }
     const int m_tiles = (a->M + kMTile - 1) / kMTile;
+    if (t.one) {
+        Tiles to = t;
+        to.div_rd = fastdiv_make(a->rope_table ? (int)a->rope_d : 2);
+        const dim3 g((unsigned)t.start[a->nseg], (unsigned)m_tiles);
+        if (a->elem == CF_ELEM_F16) hipLaunchKernelGGL(gemv_one<_Float16>, g, dim3(512), 0, s, args, to);
+        else hipLaunchKernelGGL(gemv_one<float>, g, dim3(512), 0, s, args, to);
+        return (int)hipGetLastError();
+    }
     dim3 grid((unsigned)t.start[a->nseg], (unsigned)t.ks, (unsigned)m_tiles);
     if (t.dma == 256)
         hipLaunchKernelGGL(gemv_f16_dma<256>, grid, dim3(64), 0, s, args, t);

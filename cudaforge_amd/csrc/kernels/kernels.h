@@ -153,10 +153,14 @@ int     cf_launch_gemv(const cf_gemv_args_t* a, void* stream);
 void    cf_gemv_set_dma_tile(int32_t bn);
 /* Tuning override of the fp16 DMA path's K split (1..32; 0 = automatic). */
 void    cf_gemv_set_dma_ksplit(int32_t ks);
-/* The one-pass kernel for small projections (M <= 4, M * K <= 4096, every segment width
- * a multiple of 16, weights of at most 8 MB): 0 never, 1 automatic (default), 2 wherever
- * the shape allows it whatever the weight size (tests). */
+/* The one-pass kernel for small projections (gemv_small: M <= 4, M * K <= 4096, every segment
+ * width a multiple of 16, weights of at most 8 MB): 1 automatic (default: what gemv_one does
+ * not take), 2 wherever the shape allows it whatever the weight size, 0 no one-pass kernel
+ * at all (tests). */
 void    cf_gemv_set_small(int32_t mode);
+/* The one-pass kernel of up to 16 rows (gemv_one): 0 never, 1 automatic (default), 2 wherever
+ * the shape allows it, whatever the rows and the weight size (tests, measurements). */
+void    cf_gemv_set_one(int32_t mode);
 /* 1 when a launch with these arguments can apply RoPE (rope_table): the K-chunk sum or
  * the one-pass small kernel runs it; a single-chunk split-K launch cannot. */
 int32_t cf_gemv_fuses_rope(const cf_gemv_args_t* a);

@@ -222,6 +222,40 @@ def test_mha_decode_rope_fused_and_separate_rotation(gpu, native, f16, small):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("B,H,H_kv,d,ragged,rope", [
+    (1, 1, 1, 32, False, True), (4, 3, 1, 64, True, True), (16, 12, 12, 64, False, True), (5, 8, 4, 128, True, False),
+    (17, 4, 4, 64, True, True), (3, 25, 5, 64, False, True), (2, 20, 2, 128, True, True)])
+def test_one_pass_projections(gpu, native, f16, B, H, H_kv, d, ragged, rope):
+    """The one-pass projections of a decode step against the oracle and the split-K kernels:
+    from one 32-k step (seven of the eight waves idle) to more than the rings hold, batch
+    rows that fill, cut and exceed the 16-row tile, Q | K | V of different widths, bias,
+    RoPE and the cache rows at host-known and per-sequence positions."""
+    cap = 90
+    lens = [(7 * b + 3) % cap for b in range(B)] if ragged else None
+    c = DecodeCase(B, H, H_kv, d, cap, cache_len=None if ragged else 41, seq_lens=lens, seed=B + H, f16=f16)
+
+    def run():
+        if rope:
+            return _decode_rope_gpu(c, 10000.0)
+        from helpers import run_decode_gpu
+        return run_decode_gpu(c)[:2]
+
+    want = _decode_rope_oracle(c, 10000.0) if rope else c.oracle()
+    try:
+        native.cf_gemv_set_one(2)
+        one = run()
+        native.cf_gemv_set_small(0)
+        split = run()
+    finally:
+        native.cf_gemv_set_one(1)
+        native.cf_gemv_set_small(1)
+    for w, a, b in zip(want, one, split):
+        assert max_abs(w, a) <= (TOL16 if f16 else TOL32)
+        assert max_abs(a, b) <= (1e-2 if f16 else 2e-5)
+
+
+@pytest.mark.gpu
 def test_mha_decode_rope_long_context_gqa_f16(gpu):
     """Llama-3 shape per head (32/8 heads, d = 128, base 500000) at the last position of a
     4096 cache, where the angles are largest."""
