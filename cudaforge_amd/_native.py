@@ -128,6 +128,7 @@ def _proto(lib):
         "cf_gemm_set_ws": (None, [c_int32]),
         "cf_gemm_set_ws_shape": (None, [c_int32, c_int32]),
         "cf_gemm_set_ws_ksplit": (None, [c_int32]),
+        "cf_gemm_set_mix": (None, [c_int32, c_int32]),
         "cf_gemm_set_f32": (None, [c_int32, c_int32, c_int32, c_int32]),
         "cf_gemm_set_x3": (None, [c_int32, c_int32, c_int32, c_int32]),
         "cf_flash_set_mode": (None, [c_int32]),

@@ -1335,7 +1335,9 @@ __device__ __forceinline__ void ws_store(const WsEpi& e, const int (&start)[4], 
 // Sum of gemm_f16_ws's k ranges: KS >= a.ksplit partials of four columns of one row per
 // thread, all loaded before the first add (the range index clamped, the surplus left out),
 // plus bias and residual in fp32 and one rounding.
-template <typename T, int KS>
+// T: the product's type; TB: the bias's and residual's (fp32 for a mixed product, rounded to
+// T first).
+template <typename T, typename TB, int KS>
 __global__ __launch_bounds__(64)
 void gemm_splitk_sum(cf_gemm_args_t a, int ntot, FastDiv div_row) {
     const int id = blockIdx.x * 64 + threadIdx.x;          // four columns: M * ntot / 4 < 2^31
@@ -1349,10 +1351,12 @@ void gemm_splitk_sum(cf_gemm_args_t a, int ntot, FastDiv div_row) {
     const int n1 = a.n[0], n2 = n1 + (a.nseg > 1 ? a.n[1] : 0);
     const int seg = a.nseg > 2 && n >= n2 ? 2 : a.nseg > 1 && n >= n1 ? 1 : 0;
     typedef T v4_t __attribute__((ext_vector_type(4)));
-    const T* bias = (const T*)(seg == 2 ? a.bias[2] : seg == 1 ? a.bias[1] : a.bias[0]);
+    typedef TB b4_t __attribute__((ext_vector_type(4)));
+    const TB* bias = (const TB*)(seg == 2 ? a.bias[2] : seg == 1 ? a.bias[1] : a.bias[0]);
     const int col = n - (seg == 2 ? n2 : seg == 1 ? n1 : 0);
-    const v4_t b = bias ? *(const v4_t*)(bias + col) : v4_t{0, 0, 0, 0};
-    const v4_t r = a.residual ? *(const v4_t*)((const T*)a.residual + (size_t)m * ntot + n) : v4_t{0, 0, 0, 0};
+    const b4_t b4 = bias ? *(const b4_t*)(bias + col) : b4_t{0, 0, 0, 0};
+    const b4_t r4 = a.residual ? *(const b4_t*)((const TB*)a.residual + (size_t)m * ntot + n) : b4_t{0, 0, 0, 0};
+    const v4_t b = __builtin_convertvector(b4, v4_t), r = __builtin_convertvector(r4, v4_t);
     f4_t s = v[0];
 #pragma unroll
     for (int k = 1; k < KS; k++)
@@ -1591,21 +1595,22 @@ extern "C" void cf_gemm_set_bn(int32_t bn) { g_gemm_bn = bn == 96 || bn == 128 |
 
 extern "C" void cf_gemm_set_ws(int32_t mode) { g_gemm_ws = mode == 1 ? 1 : 0; }
 
-template <typename T>
+template <typename T, typename TB>
 static void splitk_sum(const cf_gemm_args_t& a, int ntot, hipStream_t st) {
     const dim3 g((unsigned)(((long long)a.M * (ntot / 4) + 63) / 64));
     const FastDiv dr = fastdiv_make(ntot / 4);
-    if (a.ksplit <= 2) hipLaunchKernelGGL((gemm_splitk_sum<T, 2>), g, dim3(64), 0, st, a, ntot, dr);
-    else if (a.ksplit <= 4) hipLaunchKernelGGL((gemm_splitk_sum<T, 4>), g, dim3(64), 0, st, a, ntot, dr);
-    else if (a.ksplit <= 8) hipLaunchKernelGGL((gemm_splitk_sum<T, 8>), g, dim3(64), 0, st, a, ntot, dr);
-    else hipLaunchKernelGGL((gemm_splitk_sum<T, kWsMaxSplit>), g, dim3(64), 0, st, a, ntot, dr);
+    if (a.ksplit <= 2) hipLaunchKernelGGL((gemm_splitk_sum<T, TB, 2>), g, dim3(64), 0, st, a, ntot, dr);
+    else if (a.ksplit <= 4) hipLaunchKernelGGL((gemm_splitk_sum<T, TB, 4>), g, dim3(64), 0, st, a, ntot, dr);
+    else if (a.ksplit <= 8) hipLaunchKernelGGL((gemm_splitk_sum<T, TB, 8>), g, dim3(64), 0, st, a, ntot, dr);
+    else hipLaunchKernelGGL((gemm_splitk_sum<T, TB, kWsMaxSplit>), g, dim3(64), 0, st, a, ntot, dr);
 }
 
 int gemm_splitk_sum_launch(const cf_gemm_args_t* a, hipStream_t st) {
     int ntot = 0;
     for (int s = 0; s < a->nseg; s++) ntot += a->n[s];
-    if (a->elem == CF_ELEM_F32) splitk_sum<float>(*a, ntot, st);
-    else splitk_sum<_Float16>(*a, ntot, st);
+    if (a->elem == CF_ELEM_F32) splitk_sum<float, float>(*a, ntot, st);
+    else if (a->mix) splitk_sum<_Float16, float>(*a, ntot, st);
+    else splitk_sum<_Float16, _Float16>(*a, ntot, st);
     return (int)hipGetLastError();
 }
 
@@ -1642,6 +1647,8 @@ extern "C" size_t cf_gemm_plan(cf_gemm_args_t* a) {
     return c.ks > 1 ? (size_t)c.ks * (size_t)a->M * ntot : 0;
 }
 
+extern "C" int32_t cf_gemm_mix_ok(const cf_gemm_args_t* a) { return gemm_args_ok(a) && gemm_mix_ok(a); }
+
 extern "C" void cf_gemm_set_ws_ksplit(int32_t ks) { g_gemm_ws_ks = ks > 0 && ks <= kWsMaxSplit ? ks : 0; }
 
 extern "C" void cf_gemm_set_ws_shape(int32_t bm, int32_t bn) {
@@ -1655,6 +1662,7 @@ extern "C" void cf_gemm_set_group_m(int32_t group_m) { g_gemm_group_m = group_m 
 
 extern "C" int cf_launch_gemm(const cf_gemm_args_t* a, void* stream) {
     if (!gemm_args_ok(a)) return (int)hipErrorInvalidValue;
+    if (a->mix) return gemm_mix_launch(a, (hipStream_t)stream);
     if (a->plan >= kPlanF32) return gemm_f32_ws_launch(a, a->plan - kPlanF32, (hipStream_t)stream);
     if (a->plan >= kPlanX3 && a->partials) return gemm_x3_launch(a, a->plan - kPlanX3, (hipStream_t)stream);
     Tiling t = gemm_tiling(a);

@@ -17,6 +17,9 @@ int gemm_x3_launch(const cf_gemm_args_t* a, int pick, hipStream_t st);
 int gemm_f32_ws_pick(const cf_gemm_args_t* a, int* ks, float* clk);
 size_t gemm_f32_ws_floats(const cf_gemm_args_t* a);
 int gemm_f32_ws_launch(const cf_gemm_args_t* a, int pick, hipStream_t st);
+// FP16 products whose operands are FP32 in memory (a->mix), with a->ksplit ranges of k.
+int32_t gemm_mix_ok(const cf_gemm_args_t* a);
+int gemm_mix_launch(const cf_gemm_args_t* a, hipStream_t st);
 // Sums a->ksplit ranges of fp32 partial sums at a->partials into out[0] (gemm.hip).
 int gemm_splitk_sum_launch(const cf_gemm_args_t* a, hipStream_t st);
 

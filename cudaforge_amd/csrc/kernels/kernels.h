@@ -178,6 +178,8 @@ int32_t cf_gemv_fuses_rope(const cf_gemv_args_t* a);
  *                          wave-specialised kernel only (cf_gemm_plan gives plan > 0 for a
  *                          product that can take it; cf_launch_gemm rejects it otherwise).
  * ------------------------------------------------------------------------------- */
+/* a, w, bias and residual are fp32; or all but a, which is fp16. */
+enum { CF_GEMM_MIX_A32 = 1, CF_GEMM_MIX_A16 = 2 };
 enum { CF_GEMM_OUT_ROWMAJOR = 0, CF_GEMM_OUT_QKV = 1, CF_GEMM_OUT_ROWCAT = 2 };
 
 typedef struct {
@@ -194,6 +196,8 @@ typedef struct {
     int32_t     elem;        /* element type of a, w, bias, out, residual */
     int32_t     w_nk;        /* 1: w[0] is (N, K) row-major (one segment; wave-specialised
                                 kernel only) */
+    int32_t     mix;         /* CF_GEMM_MIX_*: fp16 product (row-major, row-concatenated) of fp32
+                                operands, rounded to fp16 as they are used */
     int32_t     out_f32;     /* 1: out[0] takes the fp16 results widened to fp32 (row-major,
                                 wave-specialised kernel only) */
     int32_t     plan;        /* set by cf_gemm_plan: the wave-specialised kernel's tile
@@ -215,6 +219,10 @@ void    cf_gemm_set_x3(int32_t mode, int32_t bm, int32_t bn, int32_t ks);
  * k, or the split operands of an FP32 product.  The pointers may be stand-ins of the same
  * alignment. */
 size_t  cf_gemm_plan(cf_gemm_args_t* a);
+/* Forces a tile of those launches (0, 0 = by size; tests and measurements). */
+void    cf_gemm_set_mix(int32_t bm, int32_t bn);
+/* 1 when a launch with a->mix can take these (real) pointers and sizes. */
+int32_t cf_gemm_mix_ok(const cf_gemm_args_t* a);
 /* Tuning override of the fp16 direct-to-LDS GEMM's ring depth (3 or 4 stages; 0 =
  * automatic: 3, i.e. three workgroups per CU, when there are more than two tiles per CU). */
 void cf_gemm_set_stages(int32_t stages);

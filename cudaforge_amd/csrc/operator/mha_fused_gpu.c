@@ -249,6 +249,35 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
     const size_t off_p = cf_ws_take(&cur, part);
     char* data = (char*)gpu_workspace_get_stream(st, cur);
     if (!data) return -1;
+    /* Few tokens: the two products take the FP32 buffers as they are and round what they
+     * read, with the same bits, instead of a casting launch that reads, writes and reads
+     * again every weight.  Their tiles move twice the bytes per stage, which with many
+     * tokens or a long k loop costs more than the cast.  Cast first against this: hidden 768,
+     * 8 tokens 19.3 and 16.1 us, 384 tokens 24.8 and 22.1; hidden 2048, 16 tokens 30.7 and
+     * 22.2, 256 36.8 and 37.2; hidden 4096, 8 tokens 66 and 47, 128 76.7 and 73.9, 256 85.7
+     * and 98.9. */
+    if (sh.B * sh.S <= 384 && sh.B * sh.S * sh.D <= 1 << 19 && pl.qkv.plan > 0 && pl.wo.plan > 0 && pl.qkv.out_kind == CF_GEMM_OUT_ROWCAT) {
+        fused_plan_t d = pl;
+        fused_rebase(&d, data);
+        d.qkv.a = inputs[0];
+        for (int i = 0; i < 3; i++) {
+            d.qkv.w[i] = inputs[2 + 2 * i];
+            d.qkv.bias[i] = inputs[3 + 2 * i];
+        }
+        d.qkv.mix = CF_GEMM_MIX_A32;
+        d.wo.w[0] = inputs[8];
+        d.wo.bias[0] = inputs[9];
+        d.wo.residual = d.wo.residual ? inputs[1] : NULL;
+        d.wo.out[0] = outputs[0];
+        d.wo.mix = CF_GEMM_MIX_A16;
+        d.wo.out_f32 = 1;
+        if (part > 0) d.qkv.partials = d.wo.partials = (float*)(data + off_p);
+        if (cf_gemm_mix_ok(&d.qkv) && cf_gemm_mix_ok(&d.wo)) {
+            for (int k = 0; k < 3; k++)
+                if (fused_launch(&d, k, st) != 0) return -1;
+            return 0;
+        }
+    }
     cf_cast_many_args_t c;
     for (int i = 0; i < 10; i++) {
         c.in[i] = inputs[i];

@@ -101,6 +101,26 @@ def test_fused_f16_entry_small_and_misaligned(gpu, B, S, H, H_kv, d, skew_in, sk
     assert np.all(got[:n] == 7.0) and np.all(got[n + B * S * H * d:] == 7.0)
 
 
+@pytest.mark.parametrize("bm,bn", [(32, 32), (16, 64), (32, 64), (64, 64), (128, 64)])
+@pytest.mark.parametrize("B,S,H,H_kv,d", [(1, 1, 2, 1, 64), (3, 43, 4, 2, 128), (1, 16, 16, 4, 128)])
+def test_fused_f16_entry_rounds_operands_in_place(gpu, native, bm, bn, B, S, H, H_kv, d):
+    """mha_fused_f16_cuda on few tokens, whose products round the FP32 buffers as they read
+    them: at each tile (rows and columns cut; with ranges of k at 2048) bit for bit the
+    fp16-I/O op on rounded inputs."""
+    import cudaforge_amd as cf
+    c32 = FusedCase(B, S, H, H_kv, d, seed=60 + S, f16=False, residual=True, bias_std=0.02)
+    c16 = FusedCase(B, S, H, H_kv, d, seed=60 + S, f16=True, residual=True, bias_std=0.02)
+    Y = cf.DeviceBuffer.from_numpy(np.full(B * S * H * d + 64, 7.0, np.float32))
+    try:
+        native.cf_gemm_set_mix(bm, bn)
+        assert cf.call_op("mha_fused_f16_cuda", [dev(a) for a in c32.arrays()], [Y], c32.params(cf.MhaFusedParams)) == 0
+        got = Y.download()
+    finally:
+        native.cf_gemm_set_mix(0, 0)
+    assert np.array_equal(got[:-64].reshape(B, S, H * d), run_fused_gpu(c16))
+    assert np.all(got[-64:] == 7.0)
+
+
 @pytest.mark.parametrize("kernel", ["x3", "f32"])
 @pytest.mark.parametrize("B,S,H,H_kv,d,causal", [(2, 131, 6, 2, 64, True), (1, 8, 4, 4, 32, False), (3, 77, 4, 2, 128, False)])
 def test_fused_f32_products(gpu, native, kernel, B, S, H, H_kv, d, causal):
