@@ -112,13 +112,29 @@ static int matmul_op(int elem, const void* inputs[], void* outputs[], const oper
             flip_b = 0;
         }
     }
+    const size_t bytes_a = ta ? (size_t)batch * M * K * esz : 0, bytes_b = (size_t)batch * K * N * esz;
     size_t cur = 0;
-    const size_t off_a = ta ? cf_ws_take(&cur, (size_t)batch * M * K * esz) : 0;
-    const size_t off_b = flip_b ? cf_ws_take(&cur, (size_t)batch * K * N * esz) : 0;
-    const size_t off_p = cf_ws_take(&cur, part * sizeof(float));
+    size_t off_a = cf_ws_take(&cur, bytes_a);
+    size_t off_b = flip_b ? cf_ws_take(&cur, bytes_b) : 0;
     char* ws = NULL;
-    if (cur > 0 && !(ws = (char*)gpu_workspace_get_stream(st, cur))) return -1;
-    if (part > 0) g.partials = (float*)(ws + off_p);
+    if (part > 0) {
+        /* Without room for the partial sums (a recording on a stream with no buffer of that
+         * size, or no memory) the product runs as a launch that needs none. */
+        size_t all = cur;
+        const size_t off_p = cf_ws_take(&all, part * sizeof(float));
+        if ((ws = (char*)gpu_workspace_try_stream(st, all)) != NULL) {
+            g.partials = (float*)(ws + off_p);
+        } else {
+            cur = 0;
+            flip_b = p->transpose_b;
+            off_a = cf_ws_take(&cur, bytes_a);
+            off_b = flip_b ? cf_ws_take(&cur, bytes_b) : 0;
+            g.w_nk = 0;
+            g.plan = 0;
+            g.ksplit = 1;
+        }
+    }
+    if (!ws && cur > 0 && !(ws = (char*)gpu_workspace_get_stream(st, cur))) return -1;
     int rc;
     if (ta) {
         if ((rc = cf_launch_transpose(A, ws + off_a, K, M, batch, sa, M * K, (int32_t)esz, st)) != 0) return rc;

@@ -77,6 +77,17 @@ static void fused_rebase(fused_plan_t* pl, char* data) {
     rebase(&pl->wo.a, data);
 }
 
+/* Workspace of `bytes` with `part` more for partial sums behind it; without room for those (a
+ * recording on a stream whose buffer is smaller, or no memory) *sums is NULL and the products
+ * run as launches that need none. */
+static char* fused_workspace(void* st, size_t bytes, size_t part, float** sums) {
+    size_t all = bytes;
+    const size_t off = cf_ws_take(&all, part);
+    char* ws = part > 0 ? (char*)gpu_workspace_try_stream(st, all) : NULL;
+    *sums = ws ? (float*)(ws + off) : NULL;
+    return ws ? ws : (char*)gpu_workspace_get_stream(st, bytes);
+}
+
 static int fused_plan(int elem, const void* inputs[], void* outputs[], const operator_params_t* params,
                       void* st, fused_plan_t* pl) {
     if (!inputs || !inputs[0] || !outputs || !outputs[0] || !params) return -1;
@@ -86,11 +97,11 @@ static int fused_plan(int elem, const void* inputs[], void* outputs[], const ope
     size_t cur = 0, off[4];
     fused_carve(&sh, elem == CF_ELEM_F16 ? 2 : 4, &cur, off);
     const size_t part = fused_fill(elem, inputs, outputs, params, &sh, off, pl);
-    const size_t off_p = cf_ws_take(&cur, part);
-    char* data = (char*)gpu_workspace_get_stream(st, cur);
+    float* sums;
+    char* data = fused_workspace(st, cur, part, &sums);
     if (!data) return -1;
     fused_rebase(pl, data);
-    if (part > 0) pl->qkv.partials = pl->wo.partials = (float*)(data + off_p);
+    pl->qkv.partials = pl->wo.partials = sums;
     return 0;
 }
 
@@ -246,8 +257,8 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
     void* out16[1] = {FUSED_BASE + off_y};
     fused_plan_t pl;
     const size_t part = fused_fill(CF_ELEM_F16, in16, out16, params, &sh, off, &pl);
-    const size_t off_p = cf_ws_take(&cur, part);
-    char* data = (char*)gpu_workspace_get_stream(st, cur);
+    float* sums;
+    char* data = fused_workspace(st, cur, part, &sums);
     if (!data) return -1;
     /* Few tokens: the two products take the FP32 buffers as they are and round what they
      * read, with the same bits, instead of a casting launch that reads, writes and reads
@@ -271,7 +282,7 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
         d.wo.out[0] = outputs[0];
         d.wo.mix = CF_GEMM_MIX_A16;
         d.wo.out_f32 = 1;
-        if (part > 0) d.qkv.partials = d.wo.partials = (float*)(data + off_p);
+        d.qkv.partials = d.wo.partials = sums;
         if (cf_gemm_mix_ok(&d.qkv) && cf_gemm_mix_ok(&d.wo)) {
             for (int k = 0; k < 3; k++)
                 if (fused_launch(&d, k, st) != 0) return -1;
@@ -296,7 +307,7 @@ int mha_fused_f16_cuda(const void* inputs[], void* outputs[],
     rebase(&pl.wo.bias[0], data);
     rebase(&pl.wo.residual, data);
     rebase((const void**)&pl.wo.out[0], data);
-    if (part > 0) pl.qkv.partials = pl.wo.partials = (float*)(data + off_p);
+    pl.qkv.partials = pl.wo.partials = sums;
     /* The output product widens Y as it stores it, where its kernel can (aligned Y). */
     const int wide = pl.wo.plan > 0 && (uintptr_t)outputs[0] % 16 == 0;
     if (wide) {

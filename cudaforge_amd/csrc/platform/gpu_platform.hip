@@ -279,6 +279,28 @@ void* gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes) {
     return p;
 }
 
+void* gpu_workspace_try_stream(gpu_stream_t stream, size_t bytes) {
+    const int dev = current_device();
+    if (dev < 0 || dev >= kMaxDevices) return nullptr;
+    bool room = false;
+    for (int i = 0; i < kWsSlots; i++) {
+        const Workspace& w = g_ws[dev][i];
+        if (w.used && w.stream == (hipStream_t)stream) {
+            if (w.base && w.bytes >= bytes) return gpu_workspace_get_stream(stream, bytes);
+            room = true;
+        }
+        room = room || !w.used;
+    }
+    if (!room) return nullptr;
+    // A recording can neither wait for the device nor allocate.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return cap == hipStreamCaptureStatusNone ? gpu_workspace_get_stream(stream, bytes) : nullptr;
+}
+
 void* gpu_workspace_get(size_t bytes) { return gpu_workspace_get_stream(nullptr, bytes); }
 
 size_t gpu_workspace_size(void) {

@@ -364,3 +364,48 @@ def test_fp16_layer_chain_through_the_graph(gpu, native):
         assert max_abs(want, got) <= TOL16
     finally:
         gr.destroy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f16,nk,M,N,K", [(True, False, 16, 768, 3072), (True, True, 16, 768, 3072),
+                                          (False, False, 16, 768, 4096), (False, False, 512, 2304, 768),
+                                          (False, True, 512, 2304, 768)])
+@pytest.mark.parametrize("how", ["capture", "memory"])
+def test_matmul_without_room_for_partial_sums(gpu, native, f16, nk, M, N, K, how):
+    """Products whose plan wants a workspace, where there is none to have: first called while
+    a stream is captured, or with the allocation failing.  They still run (where a transposed B
+    has to be copied first, a failed allocation gives -1), and the recording gives the result
+    on every replay."""
+    import cudaforge_amd as cf
+    r = O.round_f16 if f16 else (lambda a: a)
+    A, B = r(O.normal((M, K), M + N)), r(O.normal((K, N), K + 1, 0.0, 1.0 / np.sqrt(K)))
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    ins = [dev(A, f16), dev(B.T if nk else B, f16), None]
+    C = cf.DeviceBuffer.from_numpy(np.full((M, N), 7.0, np.float16 if f16 else np.float32))
+    p = cf.MatmulParams(M, N, K, False, nk, 1, 0, 0, 0, 0)
+    name = "matmul_f16_cuda" if f16 else "matmul_f32_cuda"
+    st = cf.Stream()
+    native.gpu_device_synchronize()
+    native.gpu_workspace_release()
+    if how == "memory":
+        native.gpu_inject_alloc_failures(2)
+        try:
+            rc = cf.call_op(name, ins, [C], p, st)
+        finally:
+            native.gpu_inject_alloc_failures(0)
+        assert rc == 0 or (nk and rc == -1)
+        if rc != 0:
+            assert cf.call_op(name, ins, [C], p, st) == 0
+        assert max_abs(want, C.download(st).astype(np.float64)) <= TOL16
+    elif not nk:
+        ex = ctypes.c_void_p()
+        assert native.gpu_capture_begin(st.handle) == 0
+        rc = cf.call_op(name, ins, [C], p, st)
+        assert native.gpu_capture_end(st.handle, ctypes.byref(ex)) == 0 and rc == 0
+        for _ in range(3):
+            C.fill_zero()
+            native.gpu_device_synchronize()
+            assert native.gpu_graph_launch(ex, st.handle) == 0
+            assert max_abs(want, C.download(st).astype(np.float64)) <= TOL16
+        native.gpu_graph_exec_destroy(ex)
+    st.synchronize()
