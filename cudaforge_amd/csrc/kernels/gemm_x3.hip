@@ -6,13 +6,17 @@
 // left, every subtraction exact), and
 //   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh) + O(2^-24 a b),
 // six bf16 MFMAs with fp32 accumulation for one fp32 product at 1/6 of 2500 TFLOP/s.  The
-// three dropped terms are below 2^-23.4 |a b| together; what an fp32 sum over K of a few
-// hundred loses to rounding is larger, and a 32-k MFMA rounds its running sum an eighth as
-// often as the 4-k fp32 one.  Relative 2-norm error against float64, N(0, 1) x N(0, 0.02),
-// fp32 MFMA kernel -> this one: K = 768 5.0e-7 -> 4.2e-7, 3072 9.9e-7 -> 8.7e-7, 14336 2.1e-6 ->
-// 2.1e-6 (1.0e-6 with ranges of k); all-positive operands 4.2e-7 -> 3.7e-7.
+// three dropped terms are below 2^-23.4 |a b| together.  The bf16 MFMA truncates (towards minus
+// infinity) as it adds to a large C, six times per 32 k, which biases the result: with one
+// running sum all-positive operands of K = 4096 were off by 3.0e-6 and 14336 by 8.2e-6, against
+// 0.9e-6 and 1.8e-6 of the fp32 kernel.  So the six MFMAs of a 32-k stage start from zero and
+// their sum is added to the running one by a rounded fp32 add (4096 x 2304 x 768 76 -> 81 us;
+// placing the adds among the next column tile's MFMAs, or reading its operands ahead, gave
+// nothing: 83-85 us).  Relative 2-norm error against float64, N(0, 1) x
+// N(0, 0.02), fp32 MFMA kernel -> this one: K = 768 5.0e-7 -> 1.2e-7, 4096 1.1e-6 -> 1.8e-7, 14336
+// 2.1e-6 -> 2.5e-7; all-positive operands 4.3e-7 -> 0.9e-7, 9.3e-7 -> 1.0e-7, 1.8e-6 -> 1.0e-7.
 // Times, the 128 x 128 fp32 MFMA kernel (gemm.hip) -> this one with the splitting launch:
-// 4096 x 2304 x 768 170 -> 76 us, 4096 x 768 x 3072 240 -> 105, 2048 x 1024 x 4096 381 -> 100.
+// 4096 x 2304 x 768 170 -> 81 us, 4096 x 768 x 768 68 -> 37, 2048 x 1024 x 4096 383 -> 111.
 // What bounds it: six MFMAs per product at the rate the chip holds with every CU busy (1.4
 // PFLOP/s of bf16 on 256 x 144 tiles, against 2.5 nominal; one tile on an idle chip runs its
 // stages within 20 % of the MFMA time), plus about 11 us of splitting at that shape.
@@ -206,11 +210,16 @@ void gemm_x3(X3Args x) {
 #pragma unroll
                 for (int p = 0; p < 3; p++) bf[p] = *(const b8_t*)(w_rd + stage * ST + (3 * j + p) * kUnit);
                 constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+                f4_t sum[MI];              // from zero: see the top
+#pragma unroll
+                for (int i = 0; i < MI; i++) sum[i] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int q = 0; q < 6; q++)
 #pragma unroll
                     for (int i = 0; i < MI; i++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[PB[q]], af[i][PA[q]], acc[i][j], 0, 0, 0);
+                        sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[PB[q]], af[i][PA[q]], sum[i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < MI; i++) acc[i][j] += sum[i];
             }
             ring_barrier();
         });

@@ -281,9 +281,12 @@ def test_matmul_f32_split_operands_keep_precision_and_range(gpu, native):
 
     M, N, K = 320, 192, 768
     a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    # A running sum of one sign, long enough for a bias of the accumulation to show.
+    long_a, long_b = rng.standard_normal((M, 4096)).astype(np.float32), rng.standard_normal((4096, N)).astype(np.float32)
     spread = np.exp2(rng.integers(-20, 20, (M, K))).astype(np.float32)
     for A, B in ((a, b), (np.abs(a), np.abs(b)), (a * spread, b), (a * np.float32(2.0 ** 100), b * np.float32(2.0 ** -90)),
-                 (a * np.float32(1e-30), b * np.float32(1e-4)), (np.concatenate([a, -a], 1), np.concatenate([b, b], 0))):
+                 (a * np.float32(1e-30), b * np.float32(1e-4)), (np.concatenate([a, -a], 1), np.concatenate([b, b], 0)),
+                 (np.abs(long_a), np.abs(long_b))):
         want = A.astype(np.float64) @ B.astype(np.float64)
         x3 = _mm_f32_run(native, A, B, None, False, "x3", 0, 0, 0)
         if not want.any():
