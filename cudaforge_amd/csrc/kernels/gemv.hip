@@ -710,9 +710,11 @@ void gemv_one(cf_gemv_args_t a, Tiles t) {
             const int row = 8 * lq + 4 * e + (lr >> 2), col = 16 * j + 4 * (lr & 3);
             w_rd[j][e] = F16 ? row * BN + 8 * ((col >> 3) ^ wswz1(row)) + (col & 7) : lq * BN + lr;
         }
-    // fp16: a sum per 16 columns.  fp32: four sums of the 16 columns in turn, so that an MFMA
-    // does not wait for the one before it.
-    constexpr int NA = F16 ? NT : 4;
+    // fp16: a sum per 16 columns.  fp32: eight sums of the 16 columns in turn, so that an MFMA
+    // does not wait for the one before it and, added pairwise like the waves' sums, each
+    // product meets no more roundings than in gemv_small's lanes, shuffles and waves (K = 768:
+    // 12 in a chain, 3 + 3 above it).
+    constexpr int NA = F16 ? NT : 8;
     f4_t acc[NA];
 #pragma unroll
     for (int j = 0; j < NA; j++) acc[j] = f4_t{0.f, 0.f, 0.f, 0.f};
@@ -744,7 +746,7 @@ void gemv_one(cf_gemv_args_t a, Tiles t) {
                 acc[i % NA] = __builtin_amdgcn_mfma_f32_16x16x4f32(sp[x_rd[i]], sp[w_rd[0][0] + 4 * i * BN], acc[i % NA], 0, 0, 0);
         }
     });
-    if constexpr (!F16) acc[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    if constexpr (!F16) acc[0] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
     // Sums to the start of the wave's own ring (its reads are done), [16 rows][BN].
     wait_lds_reads();
     float* const red = (float*)ring;
@@ -755,9 +757,10 @@ void gemv_one(cf_gemv_args_t a, Tiles t) {
         for (int i = 0; i < 4; i++) red[(4 * lq + i) * BN + 16 * j + lr] = acc[j][i];
     __syncthreads();
     advance_lengths(a);
-    float v = 0.0f;
+    float ws[NWV];
 #pragma unroll
-    for (int w = 0; w < NWV; w++) v += ((const float*)(ring_all + w * (NS * STAGE)))[min(om, kMTile - 1) * BN + oc];
+    for (int w = 0; w < NWV; w++) ws[w] = ((const float*)(ring_all + w * (NS * STAGE)))[min(om, kMTile - 1) * BN + oc];
+    float v = ((ws[0] + ws[1]) + (ws[2] + ws[3])) + ((ws[4] + ws[5]) + (ws[6] + ws[7]));
     v = sg.bias ? v + to_f(bias_v) : v;
     // n and n + 1 (n even) are neighbouring lanes and rope_d is even: a pair never splits.
     const float other = dpp_f<kDppXor1>(v);
