@@ -247,13 +247,13 @@ void flash_f16(cf_flash_args_t a) {
 // them as separate ds_read_b64 instead of pairing them into ds_read2st64_b64, which
 // measured four times the LDS cycles (SQ_LDS_BANK_CONFLICT) on gfx950.  Rows and chunks
 // past the sequence end are clamped to the last valid ones (head-major: S % 8 == 0 keeps
-// every 8-key chunk whole) and get p = 0.  The row max is reduced with the gfx950 row swaps, and the
-// running max only moves when a block exceeds it by more than kLazy (log2 units), so the
+// every 8-key chunk whole) and get p = 0.  The row max is reduced with the gfx950 row swaps, and
+// (not EXACT) the running max only moves when a block exceeds it by more than kLazy (log2 units), so the
 // accumulators are rarely rescaled.
 // The kernel is bound by its VALU work per score (the exponential and its neighbours),
 // so everything else is kept off the VALU: the loop is unrolled by ring stage (LDS
 // addresses become immediates), full blocks are loaded as a uniform base plus per-lane
-// offsets fixed for the whole loop, and the row sum of p comes out of the matrix core:
+// offsets fixed for the whole loop, and (not EXACT) the row sum of p comes out of the matrix core:
 // one more MFMA per 32 keys with an all-ones A operand gives every lane the full sum
 // over the block's keys for its query, from the same fp16 p that weights V.
 constexpr float kLazy = 8.0f;
@@ -273,7 +273,12 @@ __device__ __forceinline__ int trswz(int row) { return D == 64 ? 2 * ((row >> 1)
 // they are; V read transposed from LDS), else from q / k / vt laid out head-major.
 // Waves per SIMD the build must allow: three 16-query workgroups per CU; the 32-query
 // build (taken with at least two workgroups per CU) at three would spill registers.
-template <int D, int NJ, bool RC = false>
+// EXACT: the running maximum is moved by every block that exceeds it and the row sum adds
+// the fp32 probabilities in flash_f16's order, so the results are that kernel's bit for bit.
+// Dividing by the sum of the fp16-rounded probabilities instead is off by 5.6e-4 against
+// 5.5e-4 (64 bits; one sequence of 2048, 32 / 8 heads of 128, causal) and would save about
+// 2 us of that prefill's 208.
+template <int D, int NJ, bool RC, bool EXACT>
 __global__ __launch_bounds__(kThreads, D == 64 && NJ == 1 ? 3 : 2)
 void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot, FastDiv div_hq, FastDiv div_g) {
     constexpr int QW = 16 * NJ;                   // queries per wave
@@ -414,9 +419,10 @@ void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot,
     h8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
     // Held in VGPRs for the whole loop: kept as a scalar constant, it was moved into
     // VGPRs before the row-sum MFMAs of every block (two VALU moves per block).
-    asm volatile("" : "+v"(ones));
+    if constexpr (!EXACT) asm volatile("" : "+v"(ones));
     float m_run[NJ];
-    f4_t acc[NJ][UT], lsum[NJ];                    // lsum: every element is the query's sum of p
+    f4_t acc[NJ][UT], lsum[NJ];                    // lsum: every element is the query's sum of p; EXACT: [0], of
+                                                   // the lane's own keys
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         m_run[j] = -INFINITY;
@@ -506,21 +512,29 @@ void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot,
                 mloc = fmaxf(fmaxf(mloc, sc[j][e >> 2][e & 3]), sc[j][(e + 1) >> 2][(e + 1) & 3]);
             mloc = fmaxf(mloc, sc[j][3][3]);
             mloc = max_xor32(max_xor16(mloc)) * c;     // -inf if the whole row is masked
-            if (__builtin_amdgcn_ballot_w64(mloc > m_run[j] + kLazy)) {
-                const float m_new = mloc > m_run[j] + kLazy ? mloc : m_run[j];
-                const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_new);   // 0 on the first move
+            constexpr float kMove = EXACT ? 0.0f : kLazy;
+            float alpha = 1.0f;
+            if (__builtin_amdgcn_ballot_w64(mloc > m_run[j] + kMove)) {
+                const float m_new = mloc > m_run[j] + kMove ? mloc : m_run[j];
+                // 0 on the first move, also in lanes that have seen -inf only.
+                alpha = __builtin_amdgcn_exp2f(m_run[j] - (m_new == -INFINITY ? 0.0f : m_new));
                 m_run[j] = m_new;
-                lsum[j] *= alpha;
+                if constexpr (!EXACT) lsum[j] *= alpha;
 #pragma unroll
                 for (int u = 0; u < UT; u++) acc[j][u] *= alpha;
             }
             // Rows with nothing visible yet keep m = -inf: use 0 so p = 2^-inf = 0.
             const float m_use = m_run[j] == -INFINITY ? 0.0f : m_run[j];
+            float psum = 0.0f;
 #pragma unroll
             for (int t = 0; t < 4; t++)
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    pf[j][t >> 1][(t & 1) * 4 + i] = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][t][i], c, -m_use));
+                for (int i = 0; i < 4; i++) {
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][t][i], c, -m_use));
+                    if constexpr (EXACT) psum += p;
+                    pf[j][t >> 1][(t & 1) * 4 + i] = (_Float16)p;
+                }
+            if constexpr (EXACT) lsum[j][0] = __builtin_fmaf(lsum[j][0], alpha, psum);
         }
         // O^T[16u + 4*lq + i][query] += V^T . P^T; in 32-key step s, k-slot e of lane group
         // lq is key 32s + 16*(e/4) + 4*lq + (e%4).
@@ -535,11 +549,13 @@ void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot,
                 for (int j = 0; j < NJ; j++)
                     acc[j][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[j][s2], acc[j][u], 0, 0, 0);
             }
+        if constexpr (!EXACT) {
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int s2 = 0; s2 < 2; s2++)
-                lsum[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pf[j][s2], lsum[j], 0, 0, 0);
+                for (int s2 = 0; s2 < 2; s2++)
+                    lsum[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pf[j][s2], lsum[j], 0, 0, 0);
+        }
     };
     for_each_stage<NS>(nblk, step);
 
@@ -549,7 +565,7 @@ void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot,
     // swaps run on every lane; only the store is predicated.
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const float inv = 1.0f / lsum[j][0];
+        const float inv = 1.0f / (EXACT ? add_xor32(add_xor16(lsum[j][0])) : lsum[j][0]);
         _Float16* op = (_Float16*)a.o + (((size_t)b * S + min(query[j], S - 1)) * a.H_q + h) * D;
 #pragma unroll
         for (int p = 0; p < UT / 2; p++) {
@@ -895,14 +911,19 @@ extern "C" int cf_launch_flash_attn(const cf_flash_args_t* a, void* stream) {
             auto go = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, grid2, dim3(kThreads), 0, s, *a, pairs, kv_order, dslot, dhq, dg);
             };
+            // EXACT where the matrix core's row sum and the lazy maximum would be less exact
+            // than what else takes the shape (flash_f16): d = 128 and S % 8 != 0.
             if (a->d == 128) {
-                if (nj == 1) go(flash_f16_dma<128, 1, true>);
-                else go(flash_f16_dma<128, 2, true>);
+                if (nj == 1) go(flash_f16_dma<128, 1, true, true>);
+                else go(flash_f16_dma<128, 2, true, true>);
+            } else if (a->S % 8 != 0) {
+                if (nj == 1) go(flash_f16_dma<64, 1, true, true>);
+                else go(flash_f16_dma<64, 2, true, true>);
             } else if (a->qkv_ld) {
-                if (nj == 1) go(flash_f16_dma<64, 1, true>);
-                else go(flash_f16_dma<64, 2, true>);
-            } else if (nj == 1) go(flash_f16_dma<64, 1>);
-            else go(flash_f16_dma<64, 2>);
+                if (nj == 1) go(flash_f16_dma<64, 1, true, false>);
+                else go(flash_f16_dma<64, 2, true, false>);
+            } else if (nj == 1) go(flash_f16_dma<64, 1, false, false>);
+            else go(flash_f16_dma<64, 2, false, false>);
         } else if (a->d == 64) hipLaunchKernelGGL(flash_f16<64>, grid, dim3(kThreads), 0, s, *a);
         else hipLaunchKernelGGL(flash_f16<128>, grid, dim3(kThreads), 0, s, *a);
         return (int)hipGetLastError();

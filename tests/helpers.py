@@ -111,6 +111,33 @@ def run_decode_attn_gpu(Q, K, V, cache_len, H_kv, f16, seq_lens=None, scale=None
     return out.download(stream).astype(np.float32)
 
 
+class FlashArgs(ctypes.Structure):
+    """cf_flash_args_t (kernels.h)."""
+    _fields_ = [(n, c_void_p) for n in ("q", "k", "vt", "o")] + [
+        (n, ctypes.c_int32) for n in ("B", "S", "H_q", "H_kv", "d")] + [
+        ("scale", ctypes.c_float)] + [(n, ctypes.c_int32) for n in ("causal", "elem", "qkv_ld")]
+
+
+def run_flash_gpu(lib, q, k, v, causal, rowcat, scale=None):
+    """The fp16 prefill attention launch on q (B, S, H, d), k and v (B, S, H_kv, d): from one
+    row-concatenated matrix, or from head-major q, k and v^T."""
+    from cudaforge_amd import DeviceBuffer
+    B, S, H, d = q.shape
+    H_kv = k.shape[2]
+    if rowcat:
+        bufs = [dev(np.concatenate([x.reshape(B * S, -1) for x in (q, k, v)], axis=1))]
+        ptrs = [bufs[0].ptr, None, None]
+    else:
+        bufs = [dev(q.transpose(0, 2, 1, 3)), dev(k.transpose(0, 2, 1, 3)), dev(v.transpose(0, 2, 3, 1))]
+        ptrs = [b.ptr for b in bufs]
+    o = DeviceBuffer.empty((B, S, H, d), np.float16)
+    a = FlashArgs(*ptrs, o.ptr, B, S, H, H_kv, d, scale or 1.0 / np.sqrt(d), int(causal), 1,
+                  (H + 2 * H_kv) * d if rowcat else 0)
+    lib.cf_launch_flash_attn.argtypes = [c_void_p, c_void_p]
+    assert lib.cf_launch_flash_attn(ctypes.byref(a), None) == 0
+    return o.download()
+
+
 class FusedCase:
     def __init__(self, B, S, H, H_kv, d, seed=1, f16=False, residual=False, causal=False, wstd=0.02,
                  bias_std=0.0, fill="normal", x_scale=1.0):

@@ -13,7 +13,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from helpers import FusedCase, dev, max_abs, run_fused_gpu
+from helpers import FusedCase, dev, max_abs, run_flash_gpu, run_fused_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -308,6 +308,25 @@ def test_prefill_any_length(gpu, native, B, S, H, H_kv, d, causal):
     for o in outs:
         assert max_abs(want, o) <= TOL16
         assert max_abs(outs[0], o) <= 1e-2
+
+
+@pytest.mark.parametrize("B,S,H,H_kv,d,causal", [
+    (1, 63, 4, 4, 128, False), (2, 200, 8, 2, 128, True), (1, 1024, 16, 4, 128, True), (3, 197, 6, 2, 64, True),
+    (1, 333, 4, 4, 64, False), (1, 7, 1, 1, 64, True)])
+def test_prefill_attention_keeps_fp32_row_sums(gpu, native, B, S, H, H_kv, d, causal):
+    """Attention over row-concatenated Q | K | V at d = 128 and at lengths that are no multiple
+    of 8: bit for bit the head-major kernel's result, which sums the FP32 probabilities under
+    the exact running maximum, at both query widths and with scores far enough apart that the
+    maximum moves often."""
+    rng = np.random.default_rng(S + d)
+    q, k, v = ((rng.standard_normal((B, S, h, d)) * s).astype(np.float16) for h, s in ((H, 3.0), (H_kv, 1.0), (H_kv, 1.0)))
+    want = run_flash_gpu(native, q, k, v, causal, rowcat=False)
+    try:
+        for mode in (1, 2):
+            native.cf_flash_set_mode(mode)
+            assert np.array_equal(run_flash_gpu(native, q, k, v, causal, rowcat=True), want)
+    finally:
+        native.cf_flash_set_mode(3)
 
 
 WS_SHAPES = [(256, 192), (256, 144), (256, 128), (256, 96), (256, 64), (256, 48), (128, 192), (128, 128),
