@@ -1508,7 +1508,7 @@ constexpr int kWsCount = (int)(sizeof(kWsShapes) / sizeof(kWsShapes[0]));
 
 // The wave-specialised shape for this product, or nullptr where the kernel does not apply
 // (fp16 only; 16-byte aligned rows and stores; K a multiple of 64; every segment width a
-// multiple of 8; 32-bit A offsets; whole tiles for the Q|K|V scatter).
+// multiple of 8; 32-bit A offsets and W steps; whole tiles for the Q|K|V scatter).
 struct WsChoice {
     int i;      // index into kWsShapes, -1 where the kernel does not apply
     int ks;     // k ranges
@@ -1524,7 +1524,7 @@ WsChoice ws_pick(const cf_gemm_args_t* a, const Tiling& t) {
     // 13.3 us).  A tile override (cf_gemm_set_ws_shape) still routes the scatter here.
     if (a->out_kind == CF_GEMM_OUT_QKV && g_gemm_ws_bm == 0) return none;
     if (a->out_kind == CF_GEMM_OUT_ROWCAT && a->residual) return none;
-    if (a->K % WS_BK != 0 || (long long)a->M * a->K * 2 >= (1LL << 32)) return none;
+    if (a->K % WS_BK != 0 || (long long)a->M * a->K * 2 >= (1LL << 32) || !gemm_w_steps_fit(a)) return none;
     long long ntot = 0;
     for (int s = 0; s < a->nseg; s++) {
         if (!t.w_vec[s] || a->n[s] % 8 != 0 || (uintptr_t)a->bias[s] % 16 != 0) return none;

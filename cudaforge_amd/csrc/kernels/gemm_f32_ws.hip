@@ -299,7 +299,7 @@ extern "C" void cf_gemm_set_f32(int32_t mode, int32_t bm, int32_t bn, int32_t ks
 
 int gemm_f32_ws_pick(const cf_gemm_args_t* a, int* ks_out, float* clk) {
     if (g_f32_mode == 1 || a->elem != CF_ELEM_F32 || a->out_f32) return -1;
-    if (a->K % BK != 0 || (uintptr_t)a->a % 16 != 0) return -1;
+    if (a->K % BK != 0 || (uintptr_t)a->a % 16 != 0 || !gemm_w_steps_fit(a)) return -1;
     if (a->w_nk && (a->nseg != 1 || a->out_kind != CF_GEMM_OUT_ROWMAJOR)) return -1;
     if (a->out_kind == CF_GEMM_OUT_QKV && a->d % 4 != 0) return -1;
     uintptr_t al = (uintptr_t)a->residual;
@@ -379,7 +379,7 @@ int32_t gemm_mix_ok(const cf_gemm_args_t* a) {
         if (a->n[s] % 4 != 0) return 0;
         al |= (uintptr_t)a->bias[s] | (uintptr_t)a->w[s];
     }
-    return a->K % 64 == 0 && a->out_kind != CF_GEMM_OUT_QKV && al % 16 == 0;
+    return a->K % 64 == 0 && gemm_w_steps_fit(a) && a->out_kind != CF_GEMM_OUT_QKV && al % 16 == 0;
 }
 
 int gemm_mix_launch(const cf_gemm_args_t* a, hipStream_t st) {

@@ -7,6 +7,15 @@
 
 #include "kernels.h"
 
+// The DMA kernels step their W (K, N) addresses by a stage of rows in 32 bits (64 fp16 rows,
+// 32 fp32 ones): every segment narrower than 2^25 columns.  Wider ones take the
+// register-staged kernels, which index in 64 bits.
+inline bool gemm_w_steps_fit(const cf_gemm_args_t* a) {
+    for (int s = 0; s < a->nseg; s++)
+        if (!a->w_nk && a->n[s] >= 1 << 25) return false;
+    return true;
+}
+
 // The tile for this product (an index for gemm_x3_launch), or -1 where it does not apply.
 // *ks: the ranges of k its workgroups sum; *clk: its estimated time in CU clocks.
 int gemm_x3_pick(const cf_gemm_args_t* a, int* ks, float* clk);

@@ -111,6 +111,29 @@ def run_decode_attn_gpu(Q, K, V, cache_len, H_kv, f16, seq_lens=None, scale=None
     return out.download(stream).astype(np.float32)
 
 
+class GemmArgs(ctypes.Structure):
+    """cf_gemm_args_t (kernels.h)."""
+    _fields_ = [("a", c_void_p), ("M", ctypes.c_int32), ("K", ctypes.c_int32), ("nseg", ctypes.c_int32),
+                ("w", c_void_p * 3), ("bias", c_void_p * 3), ("n", ctypes.c_int32 * 3), ("out_kind", ctypes.c_int32),
+                ("out", c_void_p * 3), ("residual", c_void_p)] + [(n, ctypes.c_int32) for n in (
+                    "B", "S", "H_q", "H_kv", "d", "elem", "w_nk", "mix", "out_f32", "plan", "ksplit")] + [
+                ("partials", c_void_p)]
+
+
+def gemm_plan(lib, M, n, K, f16, nk=False):
+    """The plan of a row-major product with one segment per width in n (side by side), with
+    stand-ins for its operands, and whether it could round FP32 operands as it reads them:
+    (plan, ksplit, mix_ok)."""
+    n = [n] if isinstance(n, int) else n
+    a = GemmArgs(a=256, M=M, K=K, nseg=len(n), out_kind=0 if len(n) == 1 else 2, elem=int(f16), w_nk=int(nk))
+    for i, w in enumerate(n):
+        a.w[i], a.out[i], a.n[i] = 256, 256, w
+    lib.cf_gemm_plan.argtypes, lib.cf_gemm_plan.restype = [c_void_p], ctypes.c_size_t
+    lib.cf_gemm_mix_ok.argtypes, lib.cf_gemm_mix_ok.restype = [c_void_p], ctypes.c_int32
+    lib.cf_gemm_plan(ctypes.byref(a))
+    return a.plan, a.ksplit, lib.cf_gemm_mix_ok(ctypes.byref(a))
+
+
 class FlashArgs(ctypes.Structure):
     """cf_flash_args_t (kernels.h)."""
     _fields_ = [(n, c_void_p) for n in ("q", "k", "vt", "o")] + [

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from helpers import dev, max_abs
+from helpers import dev, gemm_plan, max_abs
 
 TOL32, TOL16 = 1e-4, 2e-2
 needs_ref = pytest.mark.skipif(not O.ref_available(), reason="reference build not available")
@@ -23,6 +23,24 @@ def _ln_inputs(N, D, seed):
     g = O.normal((D,), seed + 1, 1.0, 0.1)
     b = O.normal((D,), seed + 2, 0.0, 0.1)
     return x, g, b
+
+
+# --------------------------------------------------------------------- plans (CPU) ---
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M", [1, 16, 300])
+def test_very_wide_products_keep_64_bit_indexing(native, M, f16):
+    """The DMA products step over W (K, N) by 32 or 64 rows in 32 bits, which wraps from 2^25
+    columns on (a step of 0 there in FP32): such a product, alone or as one of the three side
+    by side, keeps the kernels that index in 64 bits.  W (N, K) steps along k and is not meant."""
+    wide = 1 << 25
+    assert gemm_plan(native, M, wide - 64, 64, f16)[0] > 0
+    for n in (wide, wide + 64, 1 << 26, (1 << 31) - 64):
+        plan, _, mix_ok = gemm_plan(native, M, n, 64, f16)
+        assert plan == -1 and not mix_ok
+    if f16:
+        assert gemm_plan(native, M, [64, wide, 64], 64, f16)[0] == -1
+    assert gemm_plan(native, M, wide, 64, f16, nk=True)[0] > 0
 
 
 # ------------------------------------------------------------------ oracle (CPU) ---
