@@ -27,9 +27,9 @@
 //    one conflict-free ds_read_b128, whatever the layout of the operand was.
 // 2. gemm_x3: 4 loader and 4 compute waves as in gemm_f16_ws, 32-k stages of (BM + BN) / 16
 //    x 3 units.
-// Infinities and NaN cannot be split (inf - inf); split_kernel reports any by writing the
-// call's number to a flag word, and gemm_x3 then computes its tile from the original
-// operands on the fp32 MFMA, with the results the fp32 kernel would have.
+// Infinities and NaN cannot be split (inf - inf is NaN, and so is every sum it enters): a
+// compute wave whose sums are not all finite computes its part of the tile again from the
+// original operands on the fp32 MFMA, with the results the fp32 kernel would have.  Nothing is kept for another tile, launch or replay of a recording.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -52,8 +52,6 @@ struct X3Args {
     cf_gemm_args_t g;
     uint16_t* ap;                          // A's parts, [row tile][k tile][3] units
     uint16_t* wp;                          // W's, [column tile][k tile][3], segments side by side
-    uint32_t* flag;                        // == call: an operand is not finite
-    uint32_t  call;
     int       mt, nt, kt;                  // tiles of 16 rows, 16 columns, 32 k
     int       tiles_m, tiles_n;
     int       ks, per;                     // ranges of k (blockIdx.y) and their 32-k stages
@@ -102,13 +100,8 @@ void split_kernel(X3Args x, int a_wgs) {
         dst = x.wp;
     }
     uint32_t h[8], m[8], l[8];
-    bool bad = false;
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        bad = bad || (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
-        split3(v[e], h[e], m[e], l[e]);
-    }
-    if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) *x.flag = x.call;
+    for (int e = 0; e < 8; e++) split3(v[e], h[e], m[e], l[e]);
     uint4* const o = (uint4*)(dst + (size_t)(t * x.kt + kt) * (3 * kUnit)) + lane;
     o[0] = uint4{pack_hi(h[0], h[1]), pack_hi(h[2], h[3]), pack_hi(h[4], h[5]), pack_hi(h[6], h[7])};
     o[64] = uint4{pack_hi(m[0], m[1]), pack_hi(m[2], m[3]), pack_hi(m[4], m[5]), pack_hi(m[6], m[7])};
@@ -147,10 +140,8 @@ void gemm_x3(X3Args x) {
     const int ntot = sg.total;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool slow = (uint32_t)__builtin_amdgcn_readfirstlane((int)*(const volatile uint32_t*)x.flag) == x.call;
 
     if (wave >= NCW) {
-        if (slow) return;                                  // the compute waves use no barrier then
         const int cw = wave & 3;
         uint32_t off[PW];
         int nu = 0;
@@ -193,7 +184,7 @@ void gemm_x3(X3Args x) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
 
-    if (!slow) {
+    {
         const uint16_t* const a_rd = smem_x3 + (wm / 16) * (3 * kUnit) + lane * 8;
         const uint16_t* const w_rd = smem_x3 + (AU + (wn / 16) * 3) * kUnit + lane * 8;
         ring_barrier();
@@ -223,8 +214,22 @@ void gemm_x3(X3Args x) {
             }
             ring_barrier();
         });
-    } else {
+    }
+    // 0 x sum: NaN where the sum is not finite.  A row (column) with a non-finite operand has no
+    // finite sum at all, so one column of every row and one row of every column tell.
+    float test[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) test[e] = __builtin_fmaf(acc[0][j][e], 0.0f, test[e]);
+#pragma unroll
+    for (int i = 1; i < MI; i++) test[i & 3] = __builtin_fmaf(acc[i][0][0], 0.0f, test[i & 3]);
+    if (__builtin_amdgcn_ballot_w64(__float_as_uint((test[0] + test[1]) + (test[2] + test[3])) << 1)) {
         // From the original operands: lane (lr, lq) loads row (column) lr's k0 + lq.
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
         const float* ar[MI];
         const CF_GLOBAL float* wr[NJ];
         size_t wst[NJ];
@@ -350,12 +355,11 @@ size_t gemm_x3_floats(const cf_gemm_args_t* a) {
     size_t ntot = 0;
     for (int s = 0; s < a->nseg; s++) ntot += (size_t)a->n[s];
     const size_t units = ((size_t)(a->M + 15) / 16 + ntot / 16) * (size_t)(a->K / 32) * 3;
-    // The flag's 256 bytes, then 1 KB per unit, then the ranges' sums.
-    return 64 + units * 256 + (a->ksplit > 1 ? (size_t)a->ksplit * (size_t)a->M * ntot : 0);
+    // 1 KB per unit, then the ranges' sums.
+    return units * 256 + (a->ksplit > 1 ? (size_t)a->ksplit * (size_t)a->M * ntot : 0);
 }
 
 int gemm_x3_launch(const cf_gemm_args_t* a, int pick, hipStream_t st) {
-    static std::atomic<uint32_t> calls{0};
     X3Args x;
     x.g = *a;
     int ntot = 0;
@@ -363,9 +367,7 @@ int gemm_x3_launch(const cf_gemm_args_t* a, int pick, hipStream_t st) {
     x.mt = (a->M + 15) / 16;
     x.nt = ntot / 16;
     x.kt = a->K / 32;
-    x.flag = (uint32_t*)a->partials;
-    x.call = calls.fetch_add(1, std::memory_order_relaxed) + 1;
-    x.ap = (uint16_t*)(a->partials + 64);
+    x.ap = (uint16_t*)a->partials;
     x.wp = x.ap + (size_t)x.mt * x.kt * (3 * kUnit);
     const X3Candidate& c = kX3Shapes[pick];
     x.tiles_m = (a->M + c.bm - 1) / c.bm;

@@ -324,6 +324,44 @@ def test_matmul_f32_split_operands_keep_precision_and_range(gpu, native):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn,ks", [(64, 64, 1), (256, 144, 1), (128, 64, 3)])
+def test_matmul_f32_non_finite_operands_stay_where_they_are(gpu, native, bm, bn, ks):
+    """FP32 products on split operands: an infinity in one row changes the results' path in
+    the tiles of that row only (rows of other tiles keep the bits of the finite product), and
+    leaves nothing behind in a recording, whose next replay with finite operands has the bits
+    it had before."""
+    import cudaforge_amd as cf
+    M, N, K = 512, 288, 768
+    A, B = O.normal((M, K), 11), O.normal((K, N), 12, 0.0, 1.0 / np.sqrt(K))
+    bad = A.copy()
+    bad[3, 5], bad[3, 6], bad[7, 40] = np.inf, -np.inf, np.nan
+    clean = _mm_f32_run(native, A, B, None, False, "x3", bm, bn, ks)
+    got = _mm_f32_run(native, bad, B, None, False, "x3", bm, bn, ks)
+    assert np.array_equal(got[256:], clean[256:])
+    assert not np.isfinite(got[3]).any() and np.isnan(got[7]).all()
+    rest = np.setdiff1d(np.arange(256), [3, 7])
+    assert max_abs(got[rest], clean[rest]) <= 1e-5
+    dA, dB, C = dev(A), dev(B), cf.DeviceBuffer.empty((M, N), np.float32)
+    p, st, ex = cf.MatmulParams(M, N, K, False, False, 1, 0, 0, 0, 0), cf.Stream(), ctypes.c_void_p()
+    try:
+        native.cf_gemm_set_x3(2, bm, bn, ks)
+        assert cf.call_op("matmul_f32_cuda", [dA, dB, None], [C], p, st) == 0        # the workspace
+        st.synchronize()
+        assert native.gpu_capture_begin(st.handle) == 0
+        rc = cf.call_op("matmul_f32_cuda", [dA, dB, None], [C], p, st)
+        assert native.gpu_capture_end(st.handle, ctypes.byref(ex)) == 0 and rc == 0
+        for a, want in ((A, clean), (bad, got), (A, clean), (A, clean)):
+            dA.upload(a, st)
+            assert native.gpu_graph_launch(ex, st.handle) == 0
+            assert np.array_equal(C.download(st), want, equal_nan=True)
+    finally:
+        native.cf_gemm_set_x3(0, 0, 0, 0)
+        st.synchronize()
+        if ex:
+            native.gpu_graph_exec_destroy(ex)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])
 def test_matmul_cuda_transposed_batched(gpu, f16, ta, tb):
