@@ -1,20 +1,26 @@
 // gemm_x3.hip — FP32 products on the bf16 matrix cores (gfx950).
 //
 // The fp32 MFMA runs at 1/16 of the bf16 one's rate (157 against 2500 TFLOP/s), so large
-// FP32 products are computed from an exact three-way split: x = h + m + l, each a bf16
-// holding 8 of x's 24 significant bits (h the top ones by truncation, m and l what is
-// left, every subtraction exact), and
-//   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh) + O(2^-24 a b),
-// six bf16 MFMAs with fp32 accumulation for one fp32 product at 1/6 of 2500 TFLOP/s.  The
-// three dropped terms are below 2^-23.4 |a b| together.  The bf16 MFMA truncates (towards minus
-// infinity) as it adds to a large C, six times per 32 k, which biases the result: with one
-// running sum all-positive operands of K = 4096 were off by 3.0e-6 and 14336 by 8.2e-6, against
-// 0.9e-6 and 1.8e-6 of the fp32 kernel.  So the six MFMAs of a 32-k stage start from zero and
-// their sum is added to the running one by a rounded fp32 add (4096 x 2304 x 768 76 -> 81 us;
-// placing the adds among the next column tile's MFMAs, or reading its operands ahead, gave
-// nothing: 83-85 us).  Relative 2-norm error against float64, N(0, 1) x
-// N(0, 0.02), fp32 MFMA kernel -> this one: K = 768 5.0e-7 -> 1.2e-7, 4096 1.1e-6 -> 1.8e-7, 14336
-// 2.1e-6 -> 2.5e-7; all-positive operands 4.3e-7 -> 0.9e-7, 9.3e-7 -> 1.0e-7, 1.8e-6 -> 1.0e-7.
+// FP32 products are computed from a three-way split (Henry, Tang and Heinecke, "Leveraging the
+// bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019):
+// x = h + m + l exactly, h the nearest bf16 to x, m the nearest to the rest, l what is left, and
+//   a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh) + dropped,
+// six bf16 MFMAs with fp32 accumulation for one fp32 product at 1/6 of 2500 TFLOP/s.  With
+// |m| <= 2^-8 |x| and |l| <= 2^-17 |x| the three dropped terms are below 2^-24 |a b| together, of
+// either sign.  (Cut instead of rounded parts drop up to 2^-21 |a b|, always towards zero: sums of
+// one sign were 4.2e-8 too small on average, now 2e-10.)
+// The bf16 MFMA cuts (towards minus infinity) what its products and C have below the last
+// place of the largest.  With one running sum, six times per 32 k, all-positive operands of
+// K = 4096 were off by 3.0e-6 and 14336 by 8.2e-6, against 0.9e-6 and 1.8e-6 of the fp32 kernel.
+// So the six MFMAs of a 32-k stage start from zero and their sum is added to the running one by
+// a rounded fp32 add (4096 x 2304 x 768 76 -> 81 us; placing the adds among the next column
+// tile's MFMAs, or reading its operands ahead, gave nothing: 83-85 us).  What they still cut
+// has one sign too (columns' means of 4096 rows were off by 1.9e-6, the fp32 kernel's by 5.1e-7),
+// so the parts of A are stored negated for every second stage and that stage's sum is
+// subtracted: 1.3e-7, at no cost.
+// Relative 2-norm error against float64, N(0, 1) x N(0, 0.02), fp32 MFMA kernel -> this one:
+// K = 768 5.0e-7 -> 1.0e-7, 4096 1.1e-6 -> 1.6e-7, 14336 2.1e-6 -> 2.0e-7; all-positive operands
+// 4.3e-7 -> 0.8e-7, 9.3e-7 -> 0.9e-7, 1.8e-6 -> 0.9e-7.
 // Times, the 128 x 128 fp32 MFMA kernel (gemm.hip) -> this one with the splitting launch:
 // 4096 x 2304 x 768 170 -> 81 us, 4096 x 768 x 768 68 -> 37, 2048 x 1024 x 4096 383 -> 111.
 // What bounds it: six MFMAs per product at the rate the chip holds with every CU busy (1.4
@@ -29,7 +35,8 @@
 //    x 3 units.
 // Infinities and NaN cannot be split (inf - inf is NaN, and so is every sum it enters): a
 // compute wave whose sums are not all finite computes its part of the tile again from the
-// original operands on the fp32 MFMA, with the results the fp32 kernel would have.  Nothing is kept for another tile, launch or replay of a recording.
+// original operands on the fp32 MFMA, with the results the fp32 kernel would have.  Nothing is
+// kept for another tile, launch or replay of a recording.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -58,12 +65,19 @@ struct X3Args {
     float*    part;                        // ks > 1: sums [range][M][columns]
 };
 
-// The three parts of x, as the upper halves of three floats.
+// x to the nearest bf16 (ties to even), as the upper half of a float.
+__device__ __forceinline__ uint32_t nearest_bf16(float x) {
+    const uint32_t u = __float_as_uint(x);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
+}
+// The three parts of x, as the upper halves of three floats.  Where rounding up would leave the
+// finite numbers h is cut instead (and an infinity's or NaN's m is NaN).
 __device__ __forceinline__ void split3(float x, uint32_t& h, uint32_t& m, uint32_t& l) {
-    h = __float_as_uint(x) & 0xffff0000u;
+    h = nearest_bf16(x);
+    h = (h & 0x7f800000u) == 0x7f800000u ? __float_as_uint(x) & 0xffff0000u : h;
     const float r = x - __uint_as_float(h);
-    m = __float_as_uint(r) & 0xffff0000u;
-    l = __float_as_uint(r - __uint_as_float(m));          // at most 8 bits: its lower half is zero
+    m = (__float_as_uint(r) & 0x7f800000u) == 0x7f800000u ? 0x7fc00000u : nearest_bf16(r);
+    l = __float_as_uint(r - __uint_as_float(m));          // at most 7 bits: its lower half is zero
 }
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
 
@@ -102,10 +116,15 @@ void split_kernel(X3Args x, int a_wgs) {
     uint32_t h[8], m[8], l[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) split3(v[e], h[e], m[e], l[e]);
+    const uint32_t neg = !is_w && (kt & 1) ? 0x80008000u : 0u;       // every second stage of A: see the top
     uint4* const o = (uint4*)(dst + (size_t)(t * x.kt + kt) * (3 * kUnit)) + lane;
-    o[0] = uint4{pack_hi(h[0], h[1]), pack_hi(h[2], h[3]), pack_hi(h[4], h[5]), pack_hi(h[6], h[7])};
-    o[64] = uint4{pack_hi(m[0], m[1]), pack_hi(m[2], m[3]), pack_hi(m[4], m[5]), pack_hi(m[6], m[7])};
-    o[128] = uint4{pack_hi(l[0], l[1]), pack_hi(l[2], l[3]), pack_hi(l[4], l[5]), pack_hi(l[6], l[7])};
+    auto put = [&](int part, const uint32_t (&v)[8]) {
+        o[64 * part] = uint4{pack_hi(v[0], v[1]) ^ neg, pack_hi(v[2], v[3]) ^ neg, pack_hi(v[4], v[5]) ^ neg,
+                             pack_hi(v[6], v[7]) ^ neg};
+    };
+    put(0, h);
+    put(1, m);
+    put(2, l);
 }
 
 // NCW compute waves, WMC of them along M.  Two per SIMD (8) where the tile divides among
@@ -188,8 +207,9 @@ void gemm_x3(X3Args x) {
         const uint16_t* const a_rd = smem_x3 + (wm / 16) * (3 * kUnit) + lane * 8;
         const uint16_t* const w_rd = smem_x3 + (AU + (wn / 16) * 3) * kUnit + lane * 8;
         ring_barrier();
-        for_each_stage<S>(nk, [&](int, auto stage_c) {
-            constexpr int stage = decltype(stage_c)::value;
+        for_each_stage<S % 2 ? 2 * S : S>(nk, [&](int, auto stage_c) {
+            constexpr int stage = decltype(stage_c)::value % S;
+            constexpr bool odd = decltype(stage_c)::value % 2;     // kt0 is even
             b8_t af[MI][3];
 #pragma unroll
             for (int i = 0; i < MI; i++)
@@ -210,7 +230,10 @@ void gemm_x3(X3Args x) {
                     for (int i = 0; i < MI; i++)
                         sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[PB[q]], af[i][PA[q]], sum[i], 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < MI; i++) acc[i][j] += sum[i];
+                for (int i = 0; i < MI; i++) {
+                    if constexpr (odd) acc[i][j] -= sum[i];
+                    else acc[i][j] += sum[i];
+                }
             }
             ring_barrier();
         });
@@ -289,6 +312,8 @@ const X3Candidate kX3Shapes[] = {
 };
 constexpr int kX3Count = (int)(sizeof(kX3Shapes) / sizeof(kX3Shapes[0]));
 constexpr int kX3MaxSplit = 16;
+// Stages of each of ks ranges: even, so that every range starts with a stage of A as it is.
+inline int x3_per(int kt, int ks) { return ks == 1 ? kt : (kt + 2 * ks - 1) / (2 * ks) * 2; }
 int g_x3_mode = 0, g_x3_bm = 0, g_x3_bn = 0, g_x3_ks = 0;
 
 }  // namespace
@@ -332,7 +357,7 @@ int gemm_x3_pick(const cf_gemm_args_t* a, int* ks_out, float* clk) {
         // Ranges of k add a second launch (8900 clk) and the sums' way through memory.
         const float stage = 450.0f + (float)(c.bm * c.bn) * (32.0f * 2.0f * 6.0f / 2900.0f);
         for (int ks = 1; ks <= kX3MaxSplit; ks++) {
-            const int per = (int)((kt + ks - 1) / ks);
+            const int per = x3_per((int)kt, ks);
             if (ks > 1 && (!may_split || tiles * ks > 2LL * cus || per < 4)) break;
             if (ks > 1 && (long long)(ks - 1) * per >= kt) continue;
             float cost = (float)((tiles * ks + cus - 1) / cus) * (stage * (float)per + 4000.0f);
@@ -379,7 +404,7 @@ int gemm_x3_launch(const cf_gemm_args_t* a, int pick, hipStream_t st) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     x.ks = a->ksplit;
-    x.per = (x.kt + x.ks - 1) / x.ks;
+    x.per = x3_per(x.kt, x.ks);
     x.part = (float*)(x.wp + (size_t)x.nt * x.kt * (3 * kUnit));
     e = c.launch(dim3((unsigned)(x.tiles_m * x.tiles_n), (unsigned)x.ks), st, x);
     if (e == hipSuccess) e = hipGetLastError();

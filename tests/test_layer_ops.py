@@ -324,6 +324,47 @@ def test_matmul_f32_split_operands_keep_precision_and_range(gpu, native):
 
 
 @pytest.mark.gpu
+def test_matmul_f32_split_operands_single_products(gpu, native):
+    """FP32 products on split operands, element by element against float64, with one term per
+    sum (a diagonal A): random ones, the mantissas whose dropped terms are largest, and results
+    at the end of the finite numbers whose rounded first parts multiply to more than that.
+    Bound: h and m are the nearest of 8 bits, so |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, and the three
+    dropped terms are below 2 * 2^-25 + 2^-34 of |a b|; the MFMAs cut their sums at 2^-23, of |a b|
+    the last, of 2^-8 |a b| and less the others."""
+    rng = np.random.default_rng(8)
+    n = 512
+    one = 1 + 2.0 ** -7 - 2.0 ** -23                           # all bits after the first seven zeros
+    tie = 1 + 2.0 ** -8 + 2.0 ** -17 + 2.0 ** -23                # h and m next to ties
+    for d, B in ((rng.standard_normal(n), rng.standard_normal((n, 64)) * 0.02), (np.full(n, one), np.full((n, 64), one)),
+                 (np.full(n, tie), np.full((n, 64), tie)), (np.full(n, 3.4e38), rng.uniform(-1, 1, (n, 64))),
+                 (np.full(n, 2.0 ** 65 * (1 - 2.0 ** -24)), np.full((n, 64), 2.0 ** 63 * (1 - 2.0 ** -10)))):
+        A, B = np.diag(d.astype(np.float32)), B.astype(np.float32)
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        got = _mm_f32_run(native, A, B, None, False, "x3", 64, 64, 0)
+        assert np.all(np.abs(got - want) <= np.abs(want) * (2.0 ** -24 + 2.0 ** -34 + 1.01 * 2.0 ** -23))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ks", [1, 3])
+def test_matmul_f32_split_operands_have_no_bias(gpu, native, ks):
+    """The mean error of the FP32 product on split operands: sums of one sign are off by no
+    more than 2^-26 on average (cut instead of rounded parts lose 2^-24.6, all the same way), and
+    the columns' means of sums of both signs, where a bias of the matrix core's sums would
+    stay while the elements' own errors average out, by no more than the fp32 kernel's.  An even
+    and an odd number of stages, and ranges of k of which the last is shorter."""
+    rng = np.random.default_rng(9)
+    for K in (768, 800):
+        A, B = rng.uniform(1, 2, (256, K)).astype(np.float32), rng.uniform(1, 2, (K, 64)).astype(np.float32)
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        assert abs(((_mm_f32_run(native, A, B, None, False, "x3", 64, 64, ks) - want) / want).mean()) <= 2.0 ** -26
+        A, B = rng.standard_normal((4096, K)).astype(np.float32), rng.standard_normal((K, 64)).astype(np.float32)
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        x3, general = (np.linalg.norm((_mm_f32_run(native, A, B, None, False, k, 64, 64, ks) - want).mean(0))
+                       for k in ("x3", "general"))
+        assert x3 <= general
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bm,bn,ks", [(64, 64, 1), (256, 144, 1), (128, 64, 3)])
 def test_matmul_f32_non_finite_operands_stay_where_they_are(gpu, native, bm, bn, ks):
     """FP32 products on split operands: an infinity in one row changes the results' path in
