@@ -37,6 +37,10 @@
 // compute wave whose sums are not all finite computes its part of the tile again from the
 // original operands on the fp32 MFMA, with the results the fp32 kernel would have.  Nothing is
 // kept for another tile, launch or replay of a recording.
+// Very small numbers cannot be split either: the bf16 MFMA takes subnormal operands as zero, so
+// below 2^-103 the last part is lost, below 2^-118 the second (1e-37 x 1e5 was off by 1e-3).  Where a
+// row's 32 k hold such a number and nothing from 2^-80 on, its parts are stored as NaN, with the
+// same consequence; beside a larger number what is lost is below 2^-46 of that.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -81,6 +85,8 @@ __device__ __forceinline__ void split3(float x, uint32_t& h, uint32_t& m, uint32
 }
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
 
+constexpr uint32_t kTiny = (127u - 103u) << 23, kSmall = (127u - 80u) << 23;     // 2^-103, 2^-80
+
 // One unit per wave: lane (lr, lq) takes row lr's k 8 lq .. +7.  Workgroups 0 .. (A's row
 // tiles x k tile groups) - 1 split A, the rest W.  Bound by memory (4 bytes in, 6 out).
 __global__ __launch_bounds__(256)
@@ -116,6 +122,20 @@ void split_kernel(X3Args x, int a_wgs) {
     uint32_t h[8], m[8], l[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) split3(v[e], h[e], m[e], l[e]);
+    // The bf16 MFMA takes subnormal operands as zero, and parts go down to 2^-23 of x: see the top.
+    uint32_t least = 0xffffffffu, most = 0;                // of 2 |x| - 1 (0: the largest), and |x|, as bits
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        least = min(least, (__float_as_uint(v[e]) << 1) - 1u);
+        most = max(most, __float_as_uint(v[e]) & 0x7fffffffu);
+    }
+    if (__builtin_amdgcn_ballot_w64(least < 2u * kTiny)) {
+        most = max(most, (uint32_t)__shfl_xor((int)most, 16));
+        most = max(most, (uint32_t)__shfl_xor((int)most, 32));     // of the row's 32 k
+        if (most > 0 && most < kSmall)
+#pragma unroll
+            for (int e = 0; e < 8; e++) m[e] = 0x7fc00000u;
+    }
     const uint32_t neg = !is_w && (kt & 1) ? 0x80008000u : 0u;       // every second stage of A: see the top
     uint4* const o = (uint4*)(dst + (size_t)(t * x.kt + kt) * (3 * kUnit)) + lane;
     auto put = [&](int part, const uint32_t (&v)[8]) {

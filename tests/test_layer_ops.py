@@ -365,6 +365,33 @@ def test_matmul_f32_split_operands_have_no_bias(gpu, native, ks):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nk", [False, True])
+def test_matmul_f32_split_operands_very_small_numbers(gpu, native, nk):
+    """FP32 products on split operands whose parts would be subnormal (the bf16 MFMA takes those
+    as zero): operands down to the smallest normal numbers, on either side, in some rows only
+    and beside zeros and ordinary numbers.  Bound per element: each of the K products rounded
+    once per step (test_matmul_f32_tiles), and beside a number of 2^-80 or more what is lost is
+    below 2^-126 per element; subnormal operands give what the general kernel gives."""
+    rng = np.random.default_rng(10)
+    M, N, K = 80, 64, 96
+    a, b = rng.standard_normal((M, K)), rng.standard_normal((K, N))
+    tiny, some = np.ones((M, 1)), a.copy()
+    tiny[10:30] = 1e-37
+    some[:, 1:] *= 1e-37
+    sparse = np.where(rng.random((M, K)) < 0.1, a * 1e-36, 0.0)
+    for A, B in ((a * 1e-37, b * 1e5), (a * 1e5, b * 1e-37), (a * tiny, b * 1e5), (a * 1e-32, b * 1e-3),
+                 (sparse, b * 1e5), (some, b), (a * 2.0 ** -90, b)):
+        A, B = A.astype(np.float32), B.astype(np.float32)
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        bound = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64) * (K ** 0.5 * 2.0 ** -24) + 2.0 ** -126 * K
+        got = _mm_f32_run(native, A, B, None, nk, "x3", 64, 64, 1)
+        assert np.all(np.abs(got - want) <= np.where(np.abs(want) < 1e-20, bound - 2.0 ** -126 * K, bound))
+    A = (a * 1e-40).astype(np.float32)
+    x3, general = (_mm_f32_run(native, A, (b * 1e8).astype(np.float32), None, nk, k, 64, 64, 1) for k in ("x3", "general"))
+    assert np.array_equal(x3, general)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bm,bn,ks", [(64, 64, 1), (256, 144, 1), (128, 64, 3)])
 def test_matmul_f32_non_finite_operands_stay_where_they_are(gpu, native, bm, bn, ks):
     """FP32 products on split operands: an infinity in one row changes the results' path in
