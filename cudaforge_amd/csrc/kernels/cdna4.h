@@ -71,7 +71,8 @@ __device__ __forceinline__ void for_each_stage(int n, F&& step) {
     for (int i0 = 0; i0 < n; i0 += NS) stage_group(i0, n, step, std::make_integer_sequence<int, NS>{});
 }
 
-// s_waitcnt lgkmcnt(0): every LDS read issued so far has returned its data, so a DMA
+// s_waitcnt lgkmcnt(0): every LDS read issued so far has returned its data (and every LDS
+// write is done), so a DMA
 // may refill the stage it read.
 __device__ __forceinline__ void wait_lds_reads() {
     asm volatile("" ::: "memory");

@@ -247,7 +247,7 @@ void flash_f16(cf_flash_args_t a) {
 // them as separate ds_read_b64 instead of pairing them into ds_read2st64_b64, which
 // measured four times the LDS cycles (SQ_LDS_BANK_CONFLICT) on gfx950.  Rows and chunks
 // past the sequence end are clamped to the last valid ones (head-major: S % 8 == 0 keeps
-// every 8-key chunk whole) and get p = 0.  The row max is reduced with the gfx950 row swaps, and
+// every 8-key chunk whole), get p = 0, and their V is cleared.  The row max is reduced with the gfx950 row swaps, and
 // (not EXACT) the running max only moves when a block exceeds it by more than kLazy (log2 units), so the
 // accumulators are rarely rescaled.
 // The kernel is bound by its VALU work per score (the exponential and its neighbours),
@@ -472,10 +472,20 @@ void flash_f16_dma(cf_flash_args_t a, int pairs, int kv_order, FastDiv div_slot,
         constexpr int stage = decltype(stage_c)::value;
         // Blocks issued after this one that may still be in flight (2 NI loads each).
         wait_ahead<2 * NI, NS - 2>(nblk - 1 - bi);
+        const int k0 = bi * kKB;
+        if (k0 + kKB > S) {
+            // The wave's V past the sequence end: 0, as p = 0 times a clamped row's infinity is not.
+            _Float16* const vz = ring + stage * 2 * TILE + TILE;
+#pragma unroll
+            for (int u = 0; u < NI; u++) {
+                const int row = drow0 + RPI * u;
+                if (k0 + (RC ? row : 8 * (dch ^ vswz(row))) >= S) *(h8_t*)(vz + row * D + 8 * dch) = h8_t{};
+            }
+            wait_lds_reads();
+        }
         ring_barrier();                            // every wave's part of block bi landed;
                                                    // block bi-1's stage is free again
         if (bi + NS - 1 < nblk) issue(bi + NS - 1, std::integral_constant<int, (stage + NS - 1) % NS>{});
-        const int k0 = bi * kKB;
         const _Float16* st = ring + stage * 2 * TILE;
 
         // S^T tiles: sc[j][t][i] = score(key k0 + 16t + 4*lq + i, query[j]).

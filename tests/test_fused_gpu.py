@@ -329,6 +329,28 @@ def test_prefill_attention_keeps_fp32_row_sums(gpu, native, B, S, H, H_kv, d, ca
         native.cf_flash_set_mode(3)
 
 
+@pytest.mark.parametrize("rowcat,S,d", [(True, 63, 128), (True, 197, 64), (True, 130, 128), (True, 200, 64), (False, 200, 64)])
+def test_prefill_attention_infinity_in_the_last_value(gpu, native, rowcat, S, d):
+    """An infinity in the last token's V, with a length inside a key block: the DMA kernels load
+    that row again for the keys past the end, whose probability is 0, and 0 times infinity must
+    not meet the sums.  Every query attends to it (causal: the last one), so that dim is infinite
+    and the others finite, as in the register-staged kernel."""
+    rng = np.random.default_rng(S)
+    q, k, v = (rng.standard_normal((2, S, h, d)).astype(np.float16) for h in (4, 2, 2))
+    v[:, -1, 0, 5], v[:, -1, 1, 17] = np.inf, -np.inf
+    want = np.zeros((2, S, 4, d), np.float32)
+    want[:, :, :2, 5], want[:, :, 2:, 17] = np.inf, -np.inf
+    try:
+        for mode in (1, 2):
+            native.cf_flash_set_mode(mode)
+            got = run_flash_gpu(native, q, k, v, False, rowcat)
+            assert np.array_equal(np.where(np.isfinite(got), 0, got), want)
+            got = run_flash_gpu(native, q, k, v, True, rowcat)
+            assert np.array_equal(np.where(np.isfinite(got), 0, got)[:, -1], want[:, -1])
+    finally:
+        native.cf_flash_set_mode(3)
+
+
 WS_SHAPES = [(256, 192), (256, 144), (256, 128), (256, 96), (256, 64), (256, 48), (128, 192), (128, 128),
              (128, 96), (128, 64)]
 
