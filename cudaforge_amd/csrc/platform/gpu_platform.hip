@@ -42,6 +42,11 @@ int current_device() {
     return dev;
 }
 
+// Workspace sizes are multiples of 256 bytes: what a request needs, and what is allocated for it
+// (a quarter more, so that slowly growing requests do not reallocate each time).
+size_t ws_need(size_t bytes) { return (bytes + 255) / 256 * 256; }
+size_t ws_grown(size_t need) { return need < (size_t)64 << 20 ? (size_t)64 << 20 : ws_need(need + need / 4); }
+
 int rc(hipError_t e) { return e == hipSuccess ? 0 : (int)e; }
 
 }  // namespace
@@ -261,7 +266,7 @@ void* gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes) {
     slot->used = true;
     slot->stream = st;
     slot->last = ++g_ws_clock;
-    const size_t need = ((bytes + 255) / 256) * 256;
+    const size_t need = ws_need(bytes);
     if (slot->base && slot->bytes >= need) return slot->base;
     // Grow: in-flight kernels may still use the old buffer.
     if (slot->base) {
@@ -271,7 +276,7 @@ void* gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes) {
         slot->bytes = 0;
         g_buffer_generation++;
     }
-    size_t grow = need < (size_t)64 << 20 ? (size_t)64 << 20 : need + need / 4;
+    const size_t grow = ws_grown(need);
     void* p = gpu_device_alloc(grow);
     if (!p) return nullptr;
     slot->base = p;
@@ -286,7 +291,7 @@ void* gpu_workspace_try_stream(gpu_stream_t stream, size_t bytes) {
     for (int i = 0; i < kWsSlots; i++) {
         const Workspace& w = g_ws[dev][i];
         if (w.used && w.stream == (hipStream_t)stream) {
-            if (w.base && w.bytes >= bytes) return gpu_workspace_get_stream(stream, bytes);
+            if (w.base && w.bytes >= ws_need(bytes)) return gpu_workspace_get_stream(stream, bytes);
             room = true;
         }
         room = room || !w.used;

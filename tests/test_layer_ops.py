@@ -494,6 +494,27 @@ def test_fp16_layer_chain_through_the_graph(gpu, native):
 
 
 @pytest.mark.gpu
+def test_workspace_request_of_all_it_holds_inside_a_recording(gpu, native):
+    """A buffer grown by a quarter, asked for down to its last byte and for one byte more while
+    its stream is captured: the first is given as it is, the second refused, and neither frees
+    anything (the buffer generation stays) or breaks the recording."""
+    import cudaforge_amd as cf
+    native.gpu_buffer_generation.restype = ctypes.c_uint64
+    st, ex = cf.Stream(), ctypes.c_void_p()
+    native.gpu_device_synchronize()
+    native.gpu_workspace_release()
+    base = native.gpu_workspace_get_stream(st.handle, (64 << 20) + 257)
+    held, gen = native.gpu_workspace_size(), native.gpu_buffer_generation()
+    assert base and held > 64 << 20
+    assert native.gpu_capture_begin(st.handle) == 0
+    got = [native.gpu_workspace_try_stream(st.handle, held + more) for more in (-1, 0, 1)]
+    assert native.gpu_capture_end(st.handle, ctypes.byref(ex)) == 0
+    native.gpu_graph_exec_destroy(ex)
+    assert got == [base, base, None]
+    assert (native.gpu_workspace_size(), native.gpu_buffer_generation()) == (held, gen)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("f16,nk,M,N,K", [(True, False, 16, 768, 3072), (True, True, 16, 768, 3072),
                                           (False, False, 16, 768, 4096), (False, False, 512, 2304, 768),
                                           (False, True, 512, 2304, 768)])
