@@ -287,23 +287,41 @@ void* gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes) {
 void* gpu_workspace_try_stream(gpu_stream_t stream, size_t bytes) {
     const int dev = current_device();
     if (dev < 0 || dev >= kMaxDevices) return nullptr;
-    bool room = false;
+    const size_t need = ws_need(bytes);
+    Workspace* slot = nullptr;             // the stream's own, else a free one
     for (int i = 0; i < kWsSlots; i++) {
-        const Workspace& w = g_ws[dev][i];
+        Workspace& w = g_ws[dev][i];
         if (w.used && w.stream == (hipStream_t)stream) {
-            if (w.base && w.bytes >= ws_need(bytes)) return gpu_workspace_get_stream(stream, bytes);
-            room = true;
+            if (w.base && w.bytes >= need) return gpu_workspace_get_stream(stream, bytes);
+            slot = &w;
+            break;
         }
-        room = room || !w.used;
+        if (!w.used && !slot) slot = &w;
     }
-    if (!room) return nullptr;
+    if (!slot) return nullptr;
     // A recording can neither wait for the device nor allocate.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    return cap == hipStreamCaptureStatusNone ? gpu_workspace_get_stream(stream, bytes) : nullptr;
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    // The larger buffer first: with no memory for it the old one stays, and with it the
+    // recordings that point at it and what the next operator finds.
+    const size_t grown = ws_grown(need);
+    void* p = gpu_device_alloc(grown);
+    if (!p) return nullptr;
+    if (slot->base) {
+        (void)hipDeviceSynchronize();      // in-flight kernels may still use it
+        (void)hipFree(slot->base);
+        g_buffer_generation++;
+    }
+    slot->used = true;
+    slot->stream = (hipStream_t)stream;
+    slot->last = ++g_ws_clock;
+    slot->base = p;
+    slot->bytes = grown;
+    return p;
 }
 
 void* gpu_workspace_get(size_t bytes) { return gpu_workspace_get_stream(nullptr, bytes); }

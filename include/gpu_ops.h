@@ -120,8 +120,8 @@ int   gpu_event_elapsed_ms(float* ms, gpu_event_t start, gpu_event_t stop);
 void*  gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes);
 void*  gpu_workspace_get(size_t bytes);
 /* The same for scratch an operator can do without: NULL, with nothing changed, where that
- * would take over another stream's buffer or grow one while the stream is being captured;
- * NULL too when memory runs out. */
+ * would take over another stream's buffer, grow one while the stream is being captured, or
+ * find no memory for the larger buffer beside the old one. */
 void*  gpu_workspace_try_stream(gpu_stream_t stream, size_t bytes);
 size_t gpu_workspace_size(void);     /* bytes held on the current device, all streams */
 void   gpu_workspace_release(void);

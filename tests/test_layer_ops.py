@@ -515,6 +515,45 @@ def test_workspace_request_of_all_it_holds_inside_a_recording(gpu, native):
 
 
 @pytest.mark.gpu
+def test_workspace_stays_where_optional_scratch_finds_no_memory(gpu, native):
+    """An operator with a buffer of its own (the FP32 prefill) whose products could use more
+    than memory allows, call after call: the buffer it has stays, so nothing is freed and
+    recordings stay valid (the buffer generation), and the result is that of the products that
+    need no scratch."""
+    import cudaforge_amd as cf
+    from helpers import FusedCase
+    native.gpu_buffer_generation.restype = ctypes.c_uint64
+    B, S, D = 8, 512, 768
+    c = FusedCase(B, S, 12, 12, 64, seed=5, residual=True, bias_std=0.02)
+    ins, p = [dev(x) for x in c.arrays()], c.params(cf.MhaFusedParams)
+    Y = cf.DeviceBuffer.empty((B, S, D), np.float32)
+
+    def run():
+        assert cf.call_op("mha_fused_f32_cuda", ins, [Y], p) == 0
+        return Y.download()
+
+    own = 4 * B * S * D * 4                                    # q, k, v and the attention output
+    native.gpu_device_synchronize()
+    native.gpu_workspace_release()
+    want = run()
+    assert native.gpu_workspace_size() > 64 << 20              # with all the scratch
+    native.gpu_workspace_release()
+    base = native.gpu_workspace_get(own)                       # the least it allocates, 64 MiB
+    before = native.gpu_workspace_size(), native.gpu_buffer_generation()
+    for _ in range(3):
+        native.gpu_inject_alloc_failures(1)
+        try:
+            got = run()
+        finally:
+            native.gpu_inject_alloc_failures(0)
+        assert (native.gpu_workspace_size(), native.gpu_buffer_generation()) == before
+        assert max_abs(got, want) <= 1e-5
+    assert native.gpu_workspace_get(own) == base
+    run()                                                      # memory again: it grows
+    assert native.gpu_workspace_size() > before[0]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("f16,nk,M,N,K", [(True, False, 16, 768, 3072), (True, True, 16, 768, 3072),
                                           (False, False, 16, 768, 4096), (False, False, 512, 2304, 768),
                                           (False, True, 512, 2304, 768)])
