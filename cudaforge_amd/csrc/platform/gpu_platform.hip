@@ -47,6 +47,17 @@ int current_device() {
 size_t ws_need(size_t bytes) { return (bytes + 255) / 256 * 256; }
 size_t ws_grown(size_t need) { return need < (size_t)64 << 20 ? (size_t)64 << 20 : ws_need(need + need / 4); }
 
+// Whether the stream is not being captured: a recording can neither wait for the device nor
+// allocate, and an attempt would leave the stream, and this thread's allocations, unusable.
+bool can_reallocate(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cap == hipStreamCaptureStatusNone;
+}
+
 int rc(hipError_t e) { return e == hipSuccess ? 0 : (int)e; }
 
 }  // namespace
@@ -251,11 +262,13 @@ void* gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes) {
     const int dev = current_device();
     if (dev < 0 || dev >= kMaxDevices) return nullptr;
     hipStream_t st = (hipStream_t)stream;
+    const size_t need = ws_need(bytes);
     Workspace* slot = nullptr;
     for (int i = 0; i < kWsSlots && !slot; i++)
         if (g_ws[dev][i].used && g_ws[dev][i].stream == st) slot = &g_ws[dev][i];
     for (int i = 0; i < kWsSlots && !slot; i++)
         if (!g_ws[dev][i].used) slot = &g_ws[dev][i];
+    if ((!slot || !slot->base || slot->bytes < need) && st && !can_reallocate(st)) return nullptr;
     if (!slot) {
         slot = &g_ws[dev][0];
         for (int i = 1; i < kWsSlots; i++)
@@ -266,7 +279,6 @@ void* gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes) {
     slot->used = true;
     slot->stream = st;
     slot->last = ++g_ws_clock;
-    const size_t need = ws_need(bytes);
     if (slot->base && slot->bytes >= need) return slot->base;
     // Grow: in-flight kernels may still use the old buffer.
     if (slot->base) {
@@ -298,14 +310,7 @@ void* gpu_workspace_try_stream(gpu_stream_t stream, size_t bytes) {
         }
         if (!w.used && !slot) slot = &w;
     }
-    if (!slot) return nullptr;
-    // A recording can neither wait for the device nor allocate.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    if (!slot || !can_reallocate((hipStream_t)stream)) return nullptr;
     // The larger buffer first: with no memory for it the old one stays, and with it the
     // recordings that point at it and what the next operator finds.
     const size_t grown = ws_grown(need);

@@ -115,7 +115,9 @@ int   gpu_event_elapsed_ms(float* ms, gpu_event_t start, gpu_event_t stop);
  * reused; work on one stream is ordered, so successive operators there may share it.
  * Up to 16 streams per device keep their own buffer; a further stream takes over the
  * least recently used one after a device synchronisation.  Not thread-safe (like the
- * operator registry): one host thread drives a device.  NULL on allocation failure.
+ * operator registry): one host thread drives a device.  NULL on allocation failure, and
+ * where a stream that is being captured would need a larger buffer or another stream's
+ * (call the operator once before recording it).
  * gpu_workspace_get(bytes) is the default stream's buffer. */
 void*  gpu_workspace_get_stream(gpu_stream_t stream, size_t bytes);
 void*  gpu_workspace_get(size_t bytes);
