@@ -276,8 +276,9 @@ F32_TILES = [(16, 64), (32, 64), (64, 64), (32, 32), (128, 64), (16, 128)]
 @pytest.mark.parametrize("kernel,bm,bn", [("x3", *t) for t in X3_TILES] + [("f32", *t) for t in F32_TILES])
 def test_matmul_f32_tiles(gpu, native, nk, kernel, bm, bn):
     """Each FP32 tile with its last rows and columns cut, one and several ranges of k (the
-    last one shorter), W in both layouts, against float64.  Bound per element: the sum of K
-    products rounded once per step at most, K * 2^-24 * sum |a b|, ten times what is seen."""
+    last one shorter), W in both layouts, against float64.  Bound per element: K products rounded
+    once per step at most, by 2^-24 of |a b| and of the sum so far, independently of one another:
+    sqrt(K) * 2^-24 * sum |a b|, ten times what is seen."""
     for M, N, K, ks in ((1, 16, 32, 1), (130, 208, 352, 1), (277, 176, 3104, 3), (64, 64, 4096, 4)):
         A, B = O.normal((M, K), M + N), O.normal((K, N), K + 1, 0.0, 1.0 / np.sqrt(K))
         bias = O.normal((N,), 5, 0.0, 0.1)
