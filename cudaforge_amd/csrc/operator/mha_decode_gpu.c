@@ -57,6 +57,28 @@ static int decode_shape(const mha_decode_params_t* p, decode_shape_t* s) {
     return 0;
 }
 
+/* Short contexts, in positions, that run in one split, which writes O itself: the merge launch
+ * costs about as much as these lengths.  The lines are where the whole decode op with one split
+ * takes as long as with many and a merge (us, one split and many; 1 to 16 sequences measured):
+ *   fp16, d = 64, one wave per (sequence, KV head): 16 heads, 1 sequence, 128 positions 11.3 and
+ *     12.7, 256 12.7 and 12.8, 320 13.4 and 12.7; with 128 waves and more 320 positions gain too, as
+ *     many splits no longer fit the chip at once: 16 sequences 15.8 and 18.2;
+ *   fp16, d = 64, one workgroup per sequence (up to 8 KV heads): 8 / 2 heads 128 11.0 and 11.4,
+ *     160 11.5 and 11.5, 320 14.5 and 11.6; 64 / 8 heads 128 27.2 and 27.5, 160 28.1 and 27.6;
+ *   fp32, d = 64, which walks 64 positions at a time without reading ahead, a group's heads one
+ *     after another: 16 heads 192 15.4 and 15.6, 224 16.4 and 15.6; 16 / 8 heads 192 15.2 and 15.3,
+ *     224 16.1 and 15.4; 8 / 2 heads 128 13.8 and 14.2, 160 15.4 and 14.4; 32 / 4 heads 96 27.4 and
+ *     26.7;
+ *   d = 128, twice the bytes per position: 32 / 8 heads, fp16, 64 31.8 and 31.5 (16 sequences 33.0
+ *     and 33.5), 96 33.9 and 32.7; fp32 16 / 4 heads 64 25.7 and 25.7, 96 27.8 and 25.8; 8 / 1 heads
+ *     64 19.4 and 18.9. */
+static int64_t one_split_positions(int elem, const decode_shape_t* s, int wide) {
+    const int64_t G = s->H / s->H_kv;
+    if (s->d > 64) return elem == CF_ELEM_F32 && G > 4 ? 0 : 64;
+    if (elem == CF_ELEM_F16) return wide ? 160 : s->B * s->H_kv >= cf_cu_count() / 2 ? 320 : 256;
+    return G <= 2 ? 192 : G <= 4 ? 128 : 64;
+}
+
 static void plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t* chunk, int64_t* n_split) {
     const int G = (int)(s->H / s->H_kv);
     int64_t q = cf_decode_attn_chunk_quantum(elem, (int)s->d, G);
@@ -84,14 +106,7 @@ static void plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t
          * 1-17 % faster than one split per CU slot. */
         if (spread) target *= 4;
         int64_t n = cf_ceil_div(target, units);
-        /* Short contexts in one split, which writes O itself: the merge launch costs about
-         * 3.2 us, more than splitting saves.  One split against the plan above (core op,
-         * B = 6, 16 heads of 64, fp16): 128 positions 3.7 and 6.4 us, 256 5.1 and 6.1, 384 6.4
-         * and 6.4; fp32, whose split walks 64 positions at a time without reading ahead, 192
-         * 5.5 and 7.0 (and 257 7.8 against 7.3 inside the decode op, 12 heads); heads of 128
-         * move twice the bytes per position in groups of four: 64 positions 5.5 and 7.2 us,
-         * 128 7.8 and 7.3. */
-        if (fast && t_max <= (s->d > 64 ? 64 : elem == CF_ELEM_F16 ? 320 : 192)) n = 1;
+        if (fast && t_max <= one_split_positions(elem, s, wide_cu > 0)) n = 1;
         const int64_t nmax = cf_ceil_div(t_max, q);
         if (n > nmax) n = nmax;
         if (n < 1) n = 1;

@@ -355,6 +355,25 @@ def test_device_uniform_length_plans_as_uniform_over_capacity(native, B, H, H_kv
     assert plan(-1)[1] >= plan(-2)[1]
 
 
+@pytest.mark.parametrize("f16,B,H,H_kv,d,line", [
+    (1, 1, 8, 2, 64, 160), (1, 16, 4, 4, 64, 160), (1, 4, 64, 8, 64, 160), (1, 1, 16, 16, 64, 256),
+    (1, 7, 32, 16, 64, 256), (1, 8, 32, 16, 64, 320), (1, 2, 32, 8, 128, 64), (0, 1, 12, 12, 64, 192),
+    (0, 4, 16, 8, 64, 192), (0, 2, 8, 2, 64, 128), (0, 1, 32, 4, 64, 64), (0, 1, 8, 2, 128, 64), (0, 1, 8, 1, 128, 32)])
+def test_short_contexts_in_one_split_up_to_where_it_pays(native, f16, B, H, H_kv, d, line):
+    """One split, without the merge launch, up to the positions at which splitting is as fast
+    for the kernel that takes these heads (grouped heads cost one split more per position), and
+    more than one from the next on."""
+    import cudaforge_amd as cf
+
+    def splits(T):
+        p = cf.MhaDecodeParams(B, H * d, H, H_kv, d, 0.1, T - 1, 4096)
+        chunk, n = ctypes.c_int64(0), ctypes.c_int64(0)
+        assert native.mha_decode_plan(ctypes.addressof(p), f16, ctypes.byref(chunk), ctypes.byref(n)) == 0
+        return n.value
+
+    assert splits(1) == splits(line) == 1 and splits(line + 1) > 1
+
+
 def test_buffer_generation_counter(native):
     """gpu_buffer_generation_bump moves the counter that invalidates recordings."""
     g0 = native.gpu_buffer_generation()
