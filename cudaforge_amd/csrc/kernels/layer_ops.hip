@@ -124,22 +124,33 @@ hipError_t launch_layernorm(const cf_layernorm_args_t& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Cast: grid-stride elementwise.  Between f32 and f16, eight elements per thread with
-// 16-byte accesses where both ends are aligned (`vec`; the last n % 8 one by one).
+// Cast: grid-stride elementwise.  Between f32 and f16, 2048 elements per workgroup: where both
+// ends are 16-byte aligned (`vec`) eight per thread with 16-byte accesses (the last n % 8 one by
+// one), else eight passes over consecutive ones.  67 million to fp16 and back: aligned 68 and
+// 71 us, misaligned 97 and 120 (one per thread, grid-stride, 108 and 143); eight consecutive ones per thread one by one, which touch a
+// line per lane and access, took 214 and 212.
 template <typename I, typename O>
-__device__ __forceinline__ void cast8(const I* __restrict__ in, O* __restrict__ out, int64_t i, int64_t n, bool vec) {
+__device__ __forceinline__ void cast2048(const I* __restrict__ in, O* __restrict__ out, int64_t i0, int64_t n, bool vec) {
     typedef I i8_t __attribute__((ext_vector_type(8)));
     typedef O o8_t __attribute__((ext_vector_type(8)));
-    if (vec && i + 8 <= n) {
-        *(o8_t*)(out + i) = __builtin_convertvector(*(const i8_t*)(in + i), o8_t);
+    if (vec) {
+        const int64_t i = i0 + 8 * threadIdx.x;
+        if (i + 8 <= n) {
+            *(o8_t*)(out + i) = __builtin_convertvector(*(const i8_t*)(in + i), o8_t);
+        } else {
+            for (int64_t j = i; j < n; j++) out[j] = (O)in[j];
+        }
     } else {
-        for (int64_t j = i; j < i + 8 && j < n; j++) out[j] = (O)in[j];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int64_t i = i0 + 256 * k + threadIdx.x;
+            if (i < n) out[i] = (O)in[i];
+        }
     }
 }
 template <typename I, typename O>
 __global__ __launch_bounds__(256) void cast8_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n, bool vec) {
-    for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (int64_t)gridDim.x * 2048)
-        cast8(in, out, i, n, vec);
+    for (int64_t i = (int64_t)blockIdx.x * 2048; i < n; i += (int64_t)gridDim.x * 2048) cast2048(in, out, i, n, vec);
 }
 
 // Several f32 -> f16 arrays in one launch (the mixed-precision prefill's ten operands, whose
@@ -154,8 +165,8 @@ __global__ __launch_bounds__(256) void cast_many_kernel(CastMany c) {
     int e = 0;
 #pragma unroll
     for (int k = 1; k < CF_CAST_MANY; k++) e += blockIdx.x >= c.first[k] ? 1 : 0;
-    const int64_t i = ((int64_t)(blockIdx.x - c.first[e]) * 256 + threadIdx.x) * 8;
-    if (i < c.a.n[e]) cast8((const float*)c.a.in[e], (_Float16*)c.a.out[e], i, c.a.n[e], (c.vec >> e) & 1u);
+    cast2048((const float*)c.a.in[e], (_Float16*)c.a.out[e], (int64_t)(blockIdx.x - c.first[e]) * 2048, c.a.n[e],
+             (c.vec >> e) & 1u);
 }
 
 template <typename I, typename O>

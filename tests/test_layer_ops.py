@@ -135,6 +135,29 @@ def test_layernorm_row_widths(gpu, f16, N, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 7, 2047, 2048, 2049, 6151])
+@pytest.mark.parametrize("skew_in,skew_out", [(0, 0), (1, 0), (0, 1), (1, 1), (3, 5)])
+def test_cast_f16_misaligned(gpu, native, n, skew_in, skew_out):
+    """f32 <-> f16 with either end off its 16-byte alignment, around the 2048 elements of a
+    workgroup: nearest even and exact, and nothing written past the n elements."""
+    import cudaforge_amd as cf
+    x = O.normal((n + 8,), n, 0.0, 3.0)
+    x[::5] *= np.float32(1e-6)                                 # subnormal halves
+    for src, dst, a, b in ((O.ONNX_FLOAT, O.ONNX_FLOAT16, x, np.full(n + 16, 7.0, np.float16)),
+                           (O.ONNX_FLOAT16, O.ONNX_FLOAT, x.astype(np.float16), np.full(n + 16, 7.0, np.float32))):
+        A, B = cf.DeviceBuffer.from_numpy(a), cf.DeviceBuffer.from_numpy(b)
+        ins = (ctypes.c_void_p * 1)(A.ptr + skew_in * a.itemsize)
+        outs = (ctypes.c_void_p * 1)(B.ptr + skew_out * b.itemsize)
+        p = O.CastParams(src, dst, n)
+        assert cf.find_op("cast_f32_cuda").func(ctypes.cast(ins, ctypes.POINTER(ctypes.c_void_p)),
+                                                ctypes.cast(outs, ctypes.POINTER(ctypes.c_void_p)),
+                                                ctypes.cast(ctypes.pointer(p), ctypes.c_void_p), None) == 0
+        want = b.copy()
+        want[skew_out:skew_out + n] = a[skew_in:skew_in + n].astype(b.dtype)
+        assert np.array_equal(B.download(), want)
+
+
+@pytest.mark.gpu
 def test_cast_f32_cuda_all_pairs(gpu):
     import cudaforge_amd as cf
 
