@@ -31,7 +31,8 @@ __global__ __launch_bounds__(256) void layernorm_vec(cf_layernorm_args_t a) {
     constexpr int TPR = 64 * WPR;                  // threads per row
     __shared__ float red[2][4];
     const int r = threadIdx.x % TPR, wave = threadIdx.x >> 6;
-    const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+    const int64_t wg = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+    const int64_t row = wg * (256 / TPR) + threadIdx.x / TPR;
     if (row >= a.N) return;                        // WPR == 4: the whole workgroup
     const int D = a.D, ng = D >> 2;
     const V* x = (const V*)((const T*)a.x + row * D);
@@ -100,7 +101,10 @@ __global__ __launch_bounds__(256) void layernorm_any(cf_layernorm_args_t a) {
 
 template <typename T, int VPL>
 void launch_layernorm_vec(const cf_layernorm_args_t& a, bool wide, hipStream_t s) {
-    if (wide) hipLaunchKernelGGL((layernorm_vec<T, VPL, 4>), dim3((unsigned)a.N), dim3(256), 0, s, a);
+    // A workgroup per row: beyond 65536 rows along y, as a launch holds fewer than 2^32 threads
+    // along x (2^24 rows, which four rows per workgroup do not reach).
+    const unsigned gx = (unsigned)(a.N < 65536 ? a.N : 65536);
+    if (wide) hipLaunchKernelGGL((layernorm_vec<T, VPL, 4>), dim3(gx, (unsigned)((a.N + gx - 1) / gx)), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((layernorm_vec<T, VPL, 1>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
 }
 

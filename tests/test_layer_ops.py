@@ -135,6 +135,25 @@ def test_layernorm_row_widths(gpu, f16, N, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N", [65535, 65536, 65537, 131075])
+def test_layernorm_many_long_rows(gpu, native, N):
+    """Rows that a whole workgroup takes, more of them than the grid has along x: the first,
+    the last and those around its end against the oracle, in place, and nothing written behind."""
+    import cudaforge_amd as cf
+    D = 2052
+    x = cf.DeviceBuffer.normal((N + 1, D), np.float16, 17)
+    g, b = O.round_f16(O.normal((D,), 18, 1.0, 0.1)), O.round_f16(O.normal((D,), 19, 0.0, 0.1))
+    before = x.download()
+    assert cf.call_op("layernorm_f16_cuda", [x, dev(g, True), dev(b, True)], [x], cf.LayerNormParams(N, D, 1e-5)) == 0
+    after = x.download()
+    rows = sorted({0, 1, 65534, N - 2, N - 1} | ({65535, 65536} & set(range(N))))
+    want = O.layernorm(before[rows].astype(np.float32), g, b, 1e-5)
+    assert max_abs(want, after[rows].astype(np.float32)) <= TOL16
+    assert np.array_equal(after[N], before[N])
+    assert np.all(after[:N].std(axis=1, dtype=np.float32) > 0.5)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 7, 2047, 2048, 2049, 6151])
 @pytest.mark.parametrize("skew_in,skew_out", [(0, 0), (1, 0), (0, 1), (1, 1), (3, 5)])
 def test_cast_f16_misaligned(gpu, native, n, skew_in, skew_out):
