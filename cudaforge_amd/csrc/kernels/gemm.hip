@@ -1469,7 +1469,11 @@ hipError_t launch_ws(dim3 grid, hipStream_t st, const cf_gemm_args_t& a, const T
     if (a.w_nk)
         return a.residual ? launch_ws_epi<BM, BN, S, WS_EPI_RESIDUAL, true>(grid, st, a, t)
                           : launch_ws_epi<BM, BN, S, WS_EPI_ROWMAJOR, true>(grid, st, a, t);
-    if (a.out_kind == CF_GEMM_OUT_QKV) return launch_ws_epi<BM, BN, S, WS_EPI_QKV, false, false>(grid, st, a, t);
+    if (a.out_kind == CF_GEMM_OUT_QKV) {
+        // Reached with a forced tile only (ws_pick), of the taller ones.
+        if constexpr (BM >= 128) return launch_ws_epi<BM, BN, S, WS_EPI_QKV, false, false>(grid, st, a, t);
+        return hipErrorInvalidValue;
+    }
     if (a.M % BM == 0 && (a.n[0] + (a.nseg > 1 ? a.n[1] : 0) + (a.nseg > 2 ? a.n[2] : 0)) % BN == 0 && !a.out_f32)
         return a.residual ? launch_ws_epi<BM, BN, S, WS_EPI_RESIDUAL, false, false>(grid, st, a, t)
                           : launch_ws_epi<BM, BN, S, WS_EPI_ROWMAJOR, false, false>(grid, st, a, t);
@@ -1542,7 +1546,7 @@ WsChoice ws_pick(const cf_gemm_args_t* a, const Tiling& t) {
     for (int i = 0; i < kWsCount; i++) {
         const WsCandidate& c = kWsShapes[i];
         // The Q|K|V scatter takes whole tiles; row-major outputs any rows and columns.
-        if (a->out_kind == CF_GEMM_OUT_QKV && (a->M % c.bm != 0 || ntot % c.bn != 0)) continue;
+        if (a->out_kind == CF_GEMM_OUT_QKV && (c.bm < 128 || a->M % c.bm != 0 || ntot % c.bn != 0)) continue;
         // The staged tile (fp32 with a residual, else fp16) fits in the rings.
         const unsigned staged = res32 ? (unsigned)c.bm * (c.bn + 4) * 4u : (unsigned)c.bm * (c.bn + 8) * 2u;
         const unsigned staged_vt = (unsigned)c.bn * (c.bm + 8) * 2u;     // v^T tiles, column-major
