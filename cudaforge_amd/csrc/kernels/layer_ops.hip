@@ -25,14 +25,17 @@ template <> struct Vec4<_Float16> { typedef _Float16 type __attribute__((ext_vec
 // the row's last group), gain and bias included, so a row costs one round trip to memory:
 // under a branch each group's load was waited for before the next (16 rows x 4096, 16
 // groups per lane: 16.0 us in a kernel trace; 4.8 us with four waves per row).
+constexpr int kRowsX = 65536;                      // rows along x of a grid with a workgroup per row
 template <typename T, int VPL, int WPR>
 __global__ __launch_bounds__(256) void layernorm_vec(cf_layernorm_args_t a) {
     typedef typename Vec4<T>::type V;
     constexpr int TPR = 64 * WPR;                  // threads per row
     __shared__ float red[2][4];
     const int r = threadIdx.x % TPR, wave = threadIdx.x >> 6;
-    const int64_t wg = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
-    const int64_t row = wg * (256 / TPR) + threadIdx.x / TPR;
+    // kRowsX and not gridDim.x: a kernel that reads its grid's size gets it as hidden arguments,
+    // which cost the host 0.5 us more per launch (2.7 -> 3.2).
+    const int64_t row = WPR == 4 ? (int64_t)blockIdx.y * kRowsX + blockIdx.x
+                                 : (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
     if (row >= a.N) return;                        // WPR == 4: the whole workgroup
     const int D = a.D, ng = D >> 2;
     const V* x = (const V*)((const T*)a.x + row * D);
@@ -101,10 +104,12 @@ __global__ __launch_bounds__(256) void layernorm_any(cf_layernorm_args_t a) {
 
 template <typename T, int VPL>
 void launch_layernorm_vec(const cf_layernorm_args_t& a, bool wide, hipStream_t s) {
-    // A workgroup per row: beyond 65536 rows along y, as a launch holds fewer than 2^32 threads
+    // A workgroup per row: beyond kRowsX rows along y, as a launch holds fewer than 2^32 threads
     // along x (2^24 rows, which four rows per workgroup do not reach).
-    const unsigned gx = (unsigned)(a.N < 65536 ? a.N : 65536);
-    if (wide) hipLaunchKernelGGL((layernorm_vec<T, VPL, 4>), dim3(gx, (unsigned)((a.N + gx - 1) / gx)), dim3(256), 0, s, a);
+    if (wide)
+        hipLaunchKernelGGL((layernorm_vec<T, VPL, 4>),
+                           dim3((unsigned)(a.N < kRowsX ? a.N : kRowsX), (unsigned)((a.N + kRowsX - 1) / kRowsX)),
+                           dim3(256), 0, s, a);
     else hipLaunchKernelGGL((layernorm_vec<T, VPL, 1>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
 }
 
@@ -112,10 +117,12 @@ template <typename T>
 hipError_t launch_layernorm(const cf_layernorm_args_t& a, hipStream_t s) {
     const uintptr_t al = (uintptr_t)a.x | (uintptr_t)a.y | (uintptr_t)a.gamma | (uintptr_t)a.beta;
     const bool vec = a.D % 4 == 0 && al % (4 * sizeof(T)) == 0;
-    // Four waves per row for long rows (a wave would hold more than 8 groups per lane) and
-    // while one wave per row gives the CUs less than two waves each.
+    // Four waves per row for long rows (a wave would hold more than 8 groups per lane in fp16,
+    // 6 in fp32: with gain and bias 8 take 96 registers, and 4096 rows of 1792 took 11.6 us
+    // against 9.9, 8192 of 2048 21.6 and 20.0) and while one wave per row gives the CUs less
+    // than two waves each.
     const int g1 = (a.D / 4 + 63) / 64;
-    const bool wide = g1 > 8 || (g1 > 1 && a.N < 2LL * cdna4::cu_count());
+    const bool wide = g1 > (sizeof(T) == 4 ? 6 : 8) || (g1 > 1 && a.N < 2LL * cdna4::cu_count());
     const int groups = wide ? (a.D / 4 + 255) / 256 : g1;
     if (!vec || groups > 8 || (wide && a.N > 0x7fffffffLL))
         hipLaunchKernelGGL((layernorm_any<T>), dim3((unsigned)((a.N + 3) / 4)), dim3(256), 0, s, a);
