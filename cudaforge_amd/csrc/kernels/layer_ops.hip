@@ -160,8 +160,9 @@ __device__ __forceinline__ void cast2048(const I* __restrict__ in, O* __restrict
     }
 }
 template <typename I, typename O>
-__global__ __launch_bounds__(256) void cast8_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n, bool vec) {
-    for (int64_t i = (int64_t)blockIdx.x * 2048; i < n; i += (int64_t)gridDim.x * 2048) cast2048(in, out, i, n, vec);
+__global__ __launch_bounds__(256) void cast8_kernel(const I* __restrict__ in, O* __restrict__ out, int64_t n, bool vec,
+                                                    int64_t stride) {
+    for (int64_t i = (int64_t)blockIdx.x * 2048; i < n; i += stride) cast2048(in, out, i, n, vec);
 }
 
 // Several f32 -> f16 arrays in one launch (the mixed-precision prefill's ten operands, whose
@@ -225,11 +226,12 @@ extern "C" int cf_launch_cast(const void* in, void* out, int64_t n, int32_t kind
     hipStream_t s = (hipStream_t)stream;
     const dim3 g(grid_1d(n)), g8(grid_1d((n + 7) / 8)), b(256);
     const bool vec = ((uintptr_t)in | (uintptr_t)out) % 16 == 0;
+    const int64_t stride = 2048 * (int64_t)g8.x;           // passed: gridDim.x would be a hidden argument
     switch (kind) {
         case CF_CAST_I64_F32: hipLaunchKernelGGL((cast_kernel<int64_t, float>), g, b, 0, s, (const int64_t*)in, (float*)out, n); break;
         case CF_CAST_F32_I64: hipLaunchKernelGGL((cast_kernel<float, int64_t>), g, b, 0, s, (const float*)in, (int64_t*)out, n); break;
-        case CF_CAST_F32_F16: hipLaunchKernelGGL((cast8_kernel<float, _Float16>), g8, b, 0, s, (const float*)in, (_Float16*)out, n, vec); break;
-        case CF_CAST_F16_F32: hipLaunchKernelGGL((cast8_kernel<_Float16, float>), g8, b, 0, s, (const _Float16*)in, (float*)out, n, vec); break;
+        case CF_CAST_F32_F16: hipLaunchKernelGGL((cast8_kernel<float, _Float16>), g8, b, 0, s, (const float*)in, (_Float16*)out, n, vec, stride); break;
+        case CF_CAST_F16_F32: hipLaunchKernelGGL((cast8_kernel<_Float16, float>), g8, b, 0, s, (const _Float16*)in, (float*)out, n, vec, stride); break;
         default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
