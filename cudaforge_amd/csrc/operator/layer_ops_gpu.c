@@ -119,10 +119,13 @@ static int matmul_op(int elem, const void* inputs[], void* outputs[], const oper
     char* ws = NULL;
     if (part > 0) {
         /* Without room for the partial sums (a recording on a stream with no buffer of that
-         * size, or no memory) the product runs as a launch that needs none. */
+         * size, or no memory) the product runs as a launch that needs none.  So it does in a
+         * capture that is not this library's, where nothing is transposed: such a recording
+         * then holds the caller's pointers only and stays valid when the workspace grows. */
+        const int keep_out = !p->transpose_a && !p->transpose_b && gpu_capture_foreign(st);
         size_t all = cur;
         const size_t off_p = cf_ws_take(&all, part * sizeof(float));
-        if ((ws = (char*)gpu_workspace_try_stream(st, all)) != NULL) {
+        if (!keep_out && (ws = (char*)gpu_workspace_try_stream(st, all)) != NULL) {
             g.partials = (float*)(ws + off_p);
         } else {
             cur = 0;

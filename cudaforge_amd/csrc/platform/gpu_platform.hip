@@ -31,6 +31,7 @@ Workspace g_ws[kMaxDevices][kWsSlots];
 unsigned long g_ws_clock = 0;
 int g_inject_failures = 0;
 int g_initialized_device = -1;
+thread_local int g_own_captures = 0;     // begun by gpu_capture_begin on this thread and not ended
 // Bumped whenever a buffer that recorded work may point at is freed or handed to
 // another stream (workspace slots, operator tables): recordings made before the bump
 // must not be replayed.
@@ -161,12 +162,20 @@ int gpu_device_synchronize(void) { return rc(hipDeviceSynchronize()); }
 
 int gpu_capture_begin(gpu_stream_t stream) {
     if (!stream) return (int)hipErrorInvalidValue;   // the legacy stream cannot be captured
-    return rc(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal));
+    const hipError_t e = hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) g_own_captures++;
+    return rc(e);
+}
+
+int gpu_capture_foreign(gpu_stream_t stream) {
+    if (!stream || g_own_captures > 0) return 0;
+    return can_reallocate((hipStream_t)stream) ? 0 : 1;
 }
 
 int gpu_capture_end(gpu_stream_t stream, void** exec) {
     if (!exec) return (int)hipErrorInvalidValue;
     *exec = nullptr;
+    if (g_own_captures > 0) g_own_captures--;
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture((hipStream_t)stream, &graph);
     if (e != hipSuccess || !graph) {

@@ -92,6 +92,10 @@ int   gpu_stream_destroy(gpu_stream_t stream);
  * (graph_set_replay in graph.h). */
 int   gpu_capture_begin(gpu_stream_t stream);
 int   gpu_capture_end(gpu_stream_t stream, void** exec);
+/* 1 when `stream` is being captured and this thread has not begun a capture with
+ * gpu_capture_begin: a recording of somebody who need not know the buffer generation
+ * (below).  Operators that can do without the workspace keep out of it there. */
+int   gpu_capture_foreign(gpu_stream_t stream);
 int   gpu_graph_launch(void* exec, gpu_stream_t stream);
 void  gpu_graph_exec_destroy(void* exec);
 int   gpu_device_synchronize(void);

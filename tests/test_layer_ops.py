@@ -537,6 +537,44 @@ def test_fp16_layer_chain_through_the_graph(gpu, native):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("f16,M,N,K", [(True, 16, 768, 3072), (False, 16, 768, 4096), (False, 512, 2304, 768)])
+def test_matmul_in_a_callers_own_recording_holds_the_callers_pointers(gpu, native, f16, M, N, K):
+    """A MatMul without transposes captured by the caller through HIP itself, with a workspace
+    there that its plan would use: one launch, of the caller's buffers only (with partial sums
+    or split operands in the workspace there are two and more), so growing the workspace cannot
+    take anything from under the recording.  A capture through gpu_capture_begin, whose caller
+    watches the buffer generation, uses the workspace as an eager call does."""
+    import cudaforge_amd as cf
+    hip = ctypes.CDLL("libamdhip64.so")
+    r = O.round_f16 if f16 else (lambda a: a)
+    A, B = r(O.normal((M, K), M + N)), r(O.normal((K, N), K + 1, 0.0, 1.0 / np.sqrt(K)))
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    ins, C = [dev(A, f16), dev(B, f16), None], cf.DeviceBuffer.empty((M, N), np.float16 if f16 else np.float32)
+    p, st = cf.MatmulParams(M, N, K, False, False, 1, 0, 0, 0, 0), cf.Stream()
+    name, tol = ("matmul_f16_cuda", TOL16) if f16 else ("matmul_f32_cuda", 1e-4)
+    assert cf.call_op(name, ins, [C], p, st) == 0              # the workspace
+    st.synchronize()
+    assert native.gpu_workspace_size() > 0
+    handle, graph, ex, n = st.handle, ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t()
+    assert hip.hipStreamBeginCapture(handle, 1) == 0           # thread-local mode
+    rc = cf.call_op(name, ins, [C], p, st)
+    assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0 and rc == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0 and n.value == 1
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        C.fill_zero()
+        native.gpu_device_synchronize()
+        assert hip.hipGraphLaunch(ex, handle) == 0
+        assert max_abs(want, C.download(st).astype(np.float64)) <= tol
+    hip.hipGraphExecDestroy(ex)
+    hip.hipGraphDestroy(graph)
+    assert native.gpu_capture_begin(st.handle) == 0
+    assert native.gpu_capture_foreign(handle) == 0
+    assert native.gpu_capture_end(st.handle, ctypes.byref(ex)) == 0
+    native.gpu_graph_exec_destroy(ex)
+
+
+@pytest.mark.gpu
 def test_workspace_request_of_all_it_holds_inside_a_recording(gpu, native):
     """A buffer grown by a quarter, asked for down to its last byte and for one byte more while
     its stream is captured: the first is given as it is, the second refused, and neither frees
