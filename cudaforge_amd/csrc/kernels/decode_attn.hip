@@ -159,7 +159,11 @@ __device__ __forceinline__ int vswz(int row) { return 2 * ((row / (128 / D)) % (
 // whose B operand is exactly the four probabilities a score lane holds.
 // Positions [t0, t1) of (b, kv head kvh) through one wave's ring: the partial goes to
 // `part`, or, when part is null (the range is the whole sequence), O itself.
-template <int D, int G, int NS, bool WIDE>
+// FINE: p as the sum of two fp16 numbers, so that its rounding leaves the result.  A short
+// context in one split takes this: several splits round their p under a maximum of their
+// own, where the largest p is 1 and exact, and one split's are not (12 heads of 64, 200
+// positions, against 64 bits: four splits 2.5e-4, one 2.9e-4, one FINE 2.1e-4).
+template <int D, int G, int NS, bool WIDE, bool FINE>
 __device__ __forceinline__ void split_range(const cf_decode_attn_args_t& a, _Float16* ring, int b, int kvh,
                                             int t0, int t1, float* part) {
     constexpr int KT = D / 32;          // 32-dim MFMA steps per 16 positions
@@ -325,12 +329,13 @@ __device__ __forceinline__ void split_range(const cf_decode_attn_args_t& a, _Flo
             for (int n = 0; n < NT; n++) acc[n] *= alpha;
         }
         float ps = 0.0f;
-        _Float16 pv[4 * NH];
+        _Float16 pv[4 * NH], pl[FINE ? 4 * NH : 1];
 #pragma unroll
         for (int i = 0; i < 4 * NH; i++) {
             const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(x[i], qk_scale, -m_run));
             ps += p;
             pv[i] = (_Float16)p;
+            if constexpr (FINE) pl[i] = (_Float16)(p - (float)pv[i]);
         }
         l_run += ps;
         if constexpr (NH == 2) {
@@ -338,7 +343,19 @@ __device__ __forceinline__ void split_range(const cf_decode_attn_args_t& a, _Flo
 #pragma unroll
             for (int n = 0; n < NT; n++) {
                 const h8_t vf = cat8(ds_read_tr4(st + v_rd[n][0]), ds_read_tr4(st + v_rd[n][1]));
+                if constexpr (FINE) {
+                    const h8_t lf = {pl[0], pl[1], pl[2], pl[3], pl[4], pl[5], pl[6], pl[7]};
+                    acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, lf, acc[n], 0, 0, 0);
+                }
                 acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf, acc[n], 0, 0, 0);
+            }
+        } else if constexpr (FINE) {
+            // Both parts of 16 positions in one 32-k MFMA, V twice.
+            const h8_t pf = {pv[0], pv[1], pv[2], pv[3], pl[0], pl[1], pl[2], pl[3]};
+#pragma unroll
+            for (int n = 0; n < NT; n++) {
+                const h4_t v = ds_read_tr4(st + v_rd[n][0]);
+                acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cat8(v, v), pf, acc[n], 0, 0, 0);
             }
         } else {
             const h4_t pf = {pv[0], pv[1], pv[2], pv[3]};
@@ -573,7 +590,7 @@ __device__ __forceinline__ void split_range_kv(const cf_decode_attn_args_t& a, _
     }
 }
 
-template <int D, int G, int NS, bool WIDE = false>
+template <int D, int G, int NS, bool WIDE, bool FINE>
 __global__ __launch_bounds__(WIDE ? 512 : 64)
 void split_f16(cf_decode_attn_args_t a) {
     constexpr int BP = WIDE ? 16 : 32;
@@ -583,7 +600,7 @@ void split_f16(cf_decode_attn_args_t a) {
     __shared__ __attribute__((aligned(16))) _Float16 ring_all[(WIDE ? 8 : 1) * WAVE_LDS];
     const int kvh = WIDE ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : (int)blockIdx.y;   // wave-uniform
     _Float16* ring = ring_all + (WIDE ? kvh * WAVE_LDS : 0);
-    if constexpr (WIDE) {
+    if constexpr (WIDE && !FINE) {
         if (a.balanced) {
             // Ragged lengths: one range of one sequence per workgroup (balanced_geom).
             const BalancedGeom geo = balanced_geom(a);
@@ -591,7 +608,7 @@ void split_f16(cf_decode_attn_args_t a) {
             const BalancedRange r = balanced_range(a, geo, (int)blockIdx.x);
             float* part = r.ns == 1 ? nullptr
                                     : a.partials + ((size_t)blockIdx.x * a.H_kv + kvh) * part_stride(G, D);
-            split_range<D, G, NS, WIDE>(a, ring, r.b, kvh, r.t0, r.t1, part);
+            split_range<D, G, NS, WIDE, false>(a, ring, r.b, kvh, r.t0, r.t1, part);
             return;
         }
     }
@@ -601,8 +618,8 @@ void split_f16(cf_decode_attn_args_t a) {
     const int t0 = split * a.chunk;
     if (t0 >= T_b) return;
     const int nsplit_b = (T_b + a.chunk - 1) / a.chunk;
-    split_range<D, G, NS, WIDE>(a, ring, b, kvh, t0, min(t0 + a.chunk, T_b),
-                                nsplit_b == 1 ? nullptr : partial_at(a, b * a.H_kv + kvh, split, G, D));
+    split_range<D, G, NS, WIDE, FINE>(a, ring, b, kvh, t0, min(t0 + a.chunk, T_b),
+                                      nsplit_b == 1 ? nullptr : partial_at(a, b * a.H_kv + kvh, split, G, D));
 }
 
 // The grouped kernel with K in registers (split_range_kv): a wave per KV head, each with
@@ -1153,6 +1170,10 @@ hipError_t launch_split_fast(const cf_decode_attn_args_t& a, hipStream_t s) {
     dim3 grid((unsigned)a.n_split, (unsigned)a.H_kv, (unsigned)a.B);
     if (use_wide(&a)) {
         const dim3 wgrid = a.balanced ? dim3((unsigned)a.n_split) : dim3((unsigned)a.n_split, (unsigned)a.B);
+        if (a.fine && !a.balanced) {
+            hipLaunchKernelGGL((split_f16<D, G, kWideStages, true, true>), wgrid, dim3(64 * (unsigned)a.H_kv), 0, s, a);
+            return hipGetLastError();
+        }
         bool kreg = false;
         if constexpr (D == 128) {
             if (g_kreg && kv_kernel_ok<D, G>()) {
@@ -1160,12 +1181,16 @@ hipError_t launch_split_fast(const cf_decode_attn_args_t& a, hipStream_t s) {
                 hipLaunchKernelGGL((split_f16_kv<D, G>), wgrid, dim3(64 * (unsigned)a.H_kv), 0, s, a);
             }
         }
-        if (!kreg) hipLaunchKernelGGL((split_f16<D, G, kWideStages, true>), wgrid, dim3(64 * (unsigned)a.H_kv), 0, s, a);
+        if (!kreg) hipLaunchKernelGGL((split_f16<D, G, kWideStages, true, false>), wgrid, dim3(64 * (unsigned)a.H_kv), 0, s, a);
     } else if (a.elem == CF_ELEM_F16) {
+        if (a.fine) {
+            hipLaunchKernelGGL((split_f16<D, G, kDecodeStages, false, true>), grid, dim3(64), 0, s, a);
+            return hipGetLastError();
+        }
         switch (f16_stages()) {
-            case 2: hipLaunchKernelGGL((split_f16<D, G, 2>), grid, dim3(64), 0, s, a); break;
-            case 3: hipLaunchKernelGGL((split_f16<D, G, 3>), grid, dim3(64), 0, s, a); break;
-            default: hipLaunchKernelGGL((split_f16<D, G, 4>), grid, dim3(64), 0, s, a); break;
+            case 2: hipLaunchKernelGGL((split_f16<D, G, 2, false, false>), grid, dim3(64), 0, s, a); break;
+            case 3: hipLaunchKernelGGL((split_f16<D, G, 3, false, false>), grid, dim3(64), 0, s, a); break;
+            default: hipLaunchKernelGGL((split_f16<D, G, 4, false, false>), grid, dim3(64), 0, s, a); break;
         }
     } else {
         const int NW = kF32Threads / 64;

@@ -44,6 +44,7 @@ typedef struct {
     int32_t        chunk, n_split;
     float          scale;
     int32_t        elem;
+    int32_t        fine;       /* fp16, one split: the probabilities as two fp16 numbers each */
 } cf_decode_attn_args_t;
 
 /* Positions one workgroup pass covers (chunk must be a multiple); 0 = generic kernel. */

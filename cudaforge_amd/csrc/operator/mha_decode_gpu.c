@@ -79,7 +79,9 @@ static int64_t one_split_positions(int elem, const decode_shape_t* s, int wide) 
     return G <= 2 ? 192 : G <= 4 ? 128 : 64;
 }
 
-static void plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t* chunk, int64_t* n_split) {
+/* Returns 1 where a short context runs in one split in place of several. */
+static int plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t* chunk, int64_t* n_split) {
+    int merged = 0;
     const int G = (int)(s->H / s->H_kv);
     int64_t q = cf_decode_attn_chunk_quantum(elem, (int)s->d, G);
     const int fast = q > 0;
@@ -106,7 +108,10 @@ static void plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t
          * 1-17 % faster than one split per CU slot. */
         if (spread) target *= 4;
         int64_t n = cf_ceil_div(target, units);
-        if (fast && t_max <= one_split_positions(elem, s, wide_cu > 0)) n = 1;
+        if (fast && n > 1 && t_max > q && t_max <= one_split_positions(elem, s, wide_cu > 0)) {
+            n = 1;
+            merged = 1;
+        }
         const int64_t nmax = cf_ceil_div(t_max, q);
         if (n > nmax) n = nmax;
         if (n < 1) n = 1;
@@ -118,6 +123,7 @@ static void plan_split(int elem, const decode_shape_t* s, int64_t t_max, int64_t
     if (cf_ceil_div(t_max, c) > 1024) c = cf_ceil_div(cf_ceil_div(t_max, 1024), q) * q;
     *chunk = c;
     *n_split = cf_ceil_div(t_max, c);
+    return merged;
 }
 
 int mha_decode_plan(const mha_decode_params_t* p, int elem_f16, int64_t* chunk, int64_t* n_split) {
@@ -138,7 +144,8 @@ static size_t attn_args(int elem, const decode_shape_t* s, const int32_t* lens, 
     memset(a, 0, sizeof(*a));
     const int64_t t_max = s->ragged ? s->max_seq : s->cache_len + 1;
     int64_t chunk, n_split;
-    plan_split(elem, s, t_max, &chunk, &n_split);
+    /* In one split fp16 keeps the error it had in several (split_range in decode_attn.hip). */
+    a->fine = plan_split(elem, s, t_max, &chunk, &n_split) && elem == CF_ELEM_F16;
     const int G = (int)(s->H / s->H_kv);
     if (s->ragged && !s->lens_uniform && fast_ok &&
         cf_decode_attn_balanced_ok(elem, (int)s->d, G, (int)s->H_kv, (int)s->B)) {

@@ -323,6 +323,29 @@ def test_short_context_in_one_split(gpu, native, f16, H, H_kv, d, T):
     assert max_abs(ref, got) <= tol and max_abs(split, got) <= tol
 
 
+@pytest.mark.parametrize("H,H_kv,d,T,ragged", [(12, 12, 64, 200, False), (12, 12, 64, 33, False), (32, 16, 64, 256, False),
+                                               (8, 2, 64, 150, False), (64, 8, 64, 160, False), (8, 8, 64, 47, False),
+                                               (16, 4, 128, 64, False), (32, 16, 128, 64, False), (12, 12, 64, 192, True)])
+def test_short_context_in_one_split_is_no_less_exact(gpu, native, H, H_kv, d, T, ragged):
+    """fp16, one split where there were several (one wave or one workgroup per sequence, both
+    head sizes, lengths inside a block and on the device): no further from float64 than splits of
+    the smallest size, which round their probabilities under a maximum of their own."""
+    from helpers import attn_ref64_all
+    err = {0: 0.0, 1: 0.0}
+    for seed in range(6):
+        Q, K, V = (O.round_f16(O.normal(s, 900 + 10 * seed + i)) for i, s in enumerate([(5, H, d), (5, T, H_kv, d), (5, T, H_kv, d)]))
+        lens = np.array([T - 1, T // 2, T - 5, T // 3, T - 1] if ragged else [T - 1] * 5, np.int32)
+        ref = attn_ref64_all(Q, K, V, lens + 1, H_kv, float(1 / np.sqrt(d)))
+        try:
+            for chunk in err:
+                native.mha_decode_set_split_chunk(chunk)
+                got = run_decode_attn_gpu(Q, K, V, -1 if ragged else T - 1, H_kv, True, seq_lens=lens if ragged else None)
+                err[chunk] += float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+        finally:
+            native.mha_decode_set_split_chunk(0)
+    assert err[0] <= err[1]
+
+
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1], [4096, 1, 17, 2999], [33] * 64, [1] * 63 + [5000],
                                   [16, 4080, 16, 4080], [257, 4095, 1000, 3]])
 def test_balanced_ragged_partition(gpu, native, lens):
