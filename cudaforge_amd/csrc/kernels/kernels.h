@@ -33,7 +33,8 @@ typedef struct {
     const void*    v;
     void*          o;
     const int32_t* seq_lens;   /* device, NULL = uniform cache_len */
-    int32_t        lens_uniform; /* seq_lens all hold one value (a device-held uniform length) */
+    int16_t        lens_uniform; /* seq_lens all hold one value (a device-held uniform length) */
+    int16_t        fine;       /* fp16, one split: the probabilities as two fp16 numbers each */
     int32_t        balanced;   /* ragged seq_lens on the grouped fp16 kernel: n_split workgroups
                                   (>= 2B) share the batch's attended positions about equally,
                                   each one range of one sequence (chunk unused); partial
@@ -44,7 +45,6 @@ typedef struct {
     int32_t        chunk, n_split;
     float          scale;
     int32_t        elem;
-    int32_t        fine;       /* fp16, one split: the probabilities as two fp16 numbers each */
 } cf_decode_attn_args_t;
 
 /* Positions one workgroup pass covers (chunk must be a multiple); 0 = generic kernel. */

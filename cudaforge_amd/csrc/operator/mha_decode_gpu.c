@@ -154,7 +154,7 @@ static size_t attn_args(int elem, const decode_shape_t* s, const int32_t* lens, 
         chunk = cf_decode_attn_chunk_quantum(elem, (int)s->d, G);   /* unused by the balanced kernel */
     }
     a->seq_lens = lens;
-    a->lens_uniform = s->lens_uniform;
+    a->lens_uniform = (int16_t)s->lens_uniform;
     a->B = (int32_t)s->B;
     a->H_q = (int32_t)s->H;
     a->H_kv = (int32_t)s->H_kv;
