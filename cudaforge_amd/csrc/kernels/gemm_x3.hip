@@ -23,9 +23,11 @@
 // 4.3e-7 -> 0.8e-7, 9.3e-7 -> 0.9e-7, 1.8e-6 -> 0.9e-7.
 // Times, the 128 x 128 fp32 MFMA kernel (gemm.hip) -> this one with the splitting launch:
 // 4096 x 2304 x 768 170 -> 81 us, 4096 x 768 x 768 68 -> 37, 2048 x 1024 x 4096 383 -> 111.
-// What bounds it: six MFMAs per product at the rate the chip holds with every CU busy (1.4
-// PFLOP/s of bf16 on 256 x 144 tiles, against 2.5 nominal; one tile on an idle chip runs its
-// stages within 20 % of the MFMA time), plus about 11 us of splitting at that shape.
+// What bounds it: the stage of one compute wave per SIMD.  On 256 x 144 tiles that is 216 MFMAs
+// (3456 clk), 144 fp32 adds and 39 LDS reads of 1 KB that one wave does not overlap whole: by
+// the counters the matrix cores are busy 44 % of the 4096 x 2304 x 768 product (1.14 PFLOP/s of
+// bf16) and 35 % of 4096 x 768 x 768 on 128 x 96; the chip itself holds 2.4 PFLOP/s of 16-bit
+// MFMAs.  Beside it, about 11 and 8 us of splitting at those shapes.
 //
 // 1. split_kernel writes both operands' parts in MFMA fragment order: units of 16 rows (of
 //    A, or columns of W) x 32 k, 1 KB each, lane (lr, lq)'s 16 bytes at lane * 16 = row lr,
