@@ -236,9 +236,9 @@ void flash_f16(cf_flash_args_t a) {
 // whole block's arithmetic (about 0.8 us with two workgroups per CU) to land.  What bounds
 // it is LDS reads and MFMAs about equally (a 16-query wave reads 32 KB per key block, ~240
 // clk of the CU's LDS against 128 clk of its MFMAs; 32-query waves halve the former).  One
-// sequence of 2048, 32 / 8 heads, causal: 101 us register-staged, 52 us here (660 TFLOP/s
-// of the causal work; not causal 77 us, 890).  3 sequences of 197, 12 heads of 64, causal:
-// 16.5 us register-staged (its V^T rows are misaligned at odd S), 5.5 us here.
+// sequence of 2048, 32 / 8 heads, causal: 101 us register-staged, 52 to 56 us here (610 to 660
+// TFLOP/s of the causal work).  3 sequences of 197, 12 heads of 64, causal: 16.5 us
+// register-staged (its V^T rows are misaligned at odd S), 5 us here.
 // At d = 64: K rows (128 B) and V^T rows (64
 // keys, 128 B) are XOR-swizzled in 16-byte chunks so the K fragment reads (16 rows, one
 // chunk: chunk ^ (row / 2) % 8) and the V^T fragment reads (16 rows, 8 bytes: chunk ^
