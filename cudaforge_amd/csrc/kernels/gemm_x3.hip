@@ -41,8 +41,8 @@
 // kept for another tile, launch or replay of a recording.
 // Very small numbers cannot be split either: the bf16 MFMA takes subnormal operands as zero, so
 // below 2^-103 the last part is lost, below 2^-118 the second (1e-37 x 1e5 was off by 1e-3).  Where a
-// row's 32 k hold such a number and nothing from 2^-80 on, its parts are stored as NaN, with the
-// same consequence; beside a larger number what is lost is below 2^-46 of that.
+// row's 32 k hold such a number and nothing from 2^-95 on, its parts are stored as NaN, with the
+// same consequence; beside a larger number what is lost is below 2^-31 of that.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -87,7 +87,7 @@ __device__ __forceinline__ void split3(float x, uint32_t& h, uint32_t& m, uint32
 }
 __device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
 
-constexpr uint32_t kTiny = (127u - 103u) << 23, kSmall = (127u - 80u) << 23;     // 2^-103, 2^-80
+constexpr uint32_t kTiny = (127u - 103u) << 23, kSmall = (127u - 95u) << 23;     // 2^-103, 2^-95
 
 // One unit per wave: lane (lr, lq) takes row lr's k 8 lq .. +7.  Workgroups 0 .. (A's row
 // tiles x k tile groups) - 1 split A, the rest W.  Bound by memory (4 bytes in, 6 out).

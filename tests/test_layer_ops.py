@@ -413,7 +413,7 @@ def test_matmul_f32_split_operands_very_small_numbers(gpu, native, nk):
     """FP32 products on split operands whose parts would be subnormal (the bf16 MFMA takes those
     as zero): operands down to the smallest normal numbers, on either side, in some rows only
     and beside zeros and ordinary numbers.  Bound per element: each of the K products rounded
-    once per step (test_matmul_f32_tiles), and beside a number of 2^-80 or more what is lost is
+    once per step (test_matmul_f32_tiles), and beside a number of 2^-95 or more what is lost is
     below 2^-126 per element; subnormal operands give what the general kernel gives."""
     rng = np.random.default_rng(10)
     M, N, K = 80, 64, 96
@@ -423,7 +423,7 @@ def test_matmul_f32_split_operands_very_small_numbers(gpu, native, nk):
     some[:, 1:] *= 1e-37
     sparse = np.where(rng.random((M, K)) < 0.1, a * 1e-36, 0.0)
     for A, B in ((a * 1e-37, b * 1e5), (a * 1e5, b * 1e-37), (a * tiny, b * 1e5), (a * 1e-32, b * 1e-3),
-                 (sparse, b * 1e5), (some, b), (a * 2.0 ** -90, b)):
+                 (sparse, b * 1e5), (some, b), (a * 2.0 ** -90, b), (a * 2.0 ** -94, b), (a * 2.0 ** -100, b)):
         A, B = A.astype(np.float32), B.astype(np.float32)
         want = A.astype(np.float64) @ B.astype(np.float64)
         bound = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64) * (K ** 0.5 * 2.0 ** -24) + 2.0 ** -126 * K
