@@ -304,10 +304,12 @@ def test_config4_ragged_full_size(gpu):
 
 @pytest.mark.parametrize("f16", [True, False])
 @pytest.mark.parametrize("H,H_kv,d,T", [(4, 4, 64, 64), (4, 2, 64, 320), (4, 4, 64, 321), (8, 2, 128, 64), (8, 2, 128, 65), (4, 4, 64, 192),
-                                        (8, 1, 64, 319)])
+                                        (8, 1, 64, 319), (4, 2, 64, 160), (8, 8, 64, 161), (12, 12, 64, 256), (12, 12, 64, 257),
+                                        (8, 2, 64, 128), (8, 2, 64, 129), (4, 4, 64, 193), (8, 1, 128, 33)])
 def test_short_context_in_one_split(gpu, native, f16, H, H_kv, d, T):
-    """Contexts up to the length that runs as one split (no merge) and one position past
-    it, against float64 and against splits of 64 positions."""
+    """Contexts around the lengths that run as one split (no merge; by type, head size and
+    group: 64 to 256 positions at three sequences) and one position past them, against float64
+    and against splits of 64 positions."""
     from helpers import attn_ref64_all
     Q, K, V = (O.normal(s, 610 + i) for i, s in enumerate([(3, H, d), (3, T, H_kv, d), (3, T, H_kv, d)]))
     if f16:
